@@ -24,57 +24,59 @@
 // range, N fastest, so a cell block and one batch's weights are re-read from that
 // XCD's L2.
 // The tile kernel and its helpers are in gemm_tile.hpp (also built, with an adding
-// fp32 epilogue, by gemm_add.hip); this file holds the fallback, the launchers and
-// the weight folding.
+// fp32 epilogue, by gemm_add.hip); this file holds the choice between it and the smaller
+// tiles of gemm_small.hip, the launchers and the weight folding.
 #include "gemm_tile.hpp"
 
 namespace slime {
 namespace {
 
-// Any-shape fallback: one thread per output, fp32 accumulation.
-template <typename T>
-__global__ __launch_bounds__(256) void gemm_simple_kernel(GemmArgs g) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long long)g.M * g.N) return;
-    const int m = (int)(idx / g.N), n = (int)(idx % g.N);
-    const T* a = static_cast<const T*>(g.A) + (long long)m * g.K;
-    const T* b = static_cast<const T*>(g.Bt) + (long long)(m / g.rows_per_batch) * g.bt_batch_stride +
-                 (long long)n * g.K;
-    float acc = 0.f;
-    for (int k = 0; k < g.K; ++k) acc = __builtin_fmaf(Store<T>::to_f32(a[k]), Store<T>::to_f32(b[k]), acc);
-    const int plane = n / g.ncol, col = n % g.ncol;
-    static_cast<T*>(g.out[plane])[(long long)m * g.ncol + col] =
-        Store<T>::from_f32(apply_act(acc, g.act[plane]));
-}
-
-template <typename T>
-hipError_t launch_t(const GemmArgs& a, hipStream_t s, bool mfma) {
-    if (mfma) {
-        int n_cu = 0;
-        if (hipError_t e = device_cu_count(&n_cu); e != hipSuccess) return e;
-        const int ntiles = (a.M / kBM) * (a.N / kBN);
-        const int grid = ntiles < n_cu ? ntiles : n_cu;  // one persistent WG per CU
-        hipLaunchKernelGGL(gemm_mfma_kernel<T>, dim3(grid), dim3(kThreads), 0, s, a);
-    } else {
-        const long long total = (long long)a.M * a.N;
-        hipLaunchKernelGGL(gemm_simple_kernel<T>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
-                           s, a);
-    }
-    return hipGetLastError();
-}
-
-}  // namespace
-
-bool gemm_uses_mfma(int dtype, const GemmArgs& a) {
-    // K must fill whole groups of 4 slabs (4 x 64 bytes: 128 bf16 or 64 fp32).
+// The 256 x 256 kernel's shapes: whole tiles in M, N, the planes and the batches, and K in
+// whole groups of 4 slabs (4 x 64 bytes: 128 bf16 or 64 fp32).
+bool fits256(int dtype, const GemmArgs& a) {
     const int k_group = dtype == 1 ? 128 : 64;
     return a.M % kBM == 0 && a.N % kBN == 0 && a.ncol % kBN == 0 && a.K % k_group == 0 &&
            a.rows_per_batch % kBM == 0;
 }
 
+}  // namespace
+
+// The tile whose rounds over the card take least time: ceil(tiles / CUs) rounds of
+// tile^2 products each, at the rate the kernel reaches once it fills the card. Measured on
+// K = 512 forward products (TFLOP/s, 256 / 128 / 64 wide): bf16 915 / 690 / 560 at 65,536
+// rows or more, fp32 139 / 132 / 127; so the 256-wide kernel keeps what it tiles and
+// fills, and a batch that leaves its last round mostly empty goes to the smaller tiles:
+// 16,384 x 1536 x 512 in fp32 (384 tiles of 256 on 256 CUs) 272 -> 198 us in 1536 tiles of
+// 128; 8192 x 768 x 256 80 -> 31 us in tiles of 64. Shapes that 256 does not divide ran one
+// thread per output before (0.55 TFLOP/s): 73,984 x 1536 x 512 bf16 211 ms -> 0.18 ms.
+int gemm_tile(int dtype, const GemmArgs& a, int n_cu) {
+    int best = 0;
+    double best_t = 0.0;
+    for (int tile : {256, 128, 64}) {
+        if (tile == 256 ? !fits256(dtype, a) : !gemm_small_fits(dtype, tile, a)) continue;
+        const long long rows = (a.rows_per_batch + tile - 1) / tile;  // per batch
+        const long long ntiles = a.M / a.rows_per_batch * rows * (a.N / tile);
+        const long long rounds = (ntiles + n_cu - 1) / n_cu;
+        const double rate = tile == 256 ? 1.0 : dtype == 1 ? (tile == 128 ? 0.75 : 0.6) : (tile == 128 ? 0.95 : 0.9);
+        const double t = (double)rounds * tile * tile / rate;
+        if (!best || t < best_t) best = tile, best_t = t;
+    }
+    return best;
+}
+
 hipError_t launch_gemm(int dtype, const GemmArgs& a, hipStream_t s) {
-    const bool mfma = gemm_uses_mfma(dtype, a);
-    return dtype == 1 ? launch_t<bf16_t>(a, s, mfma) : launch_t<float>(a, s, mfma);
+    int n_cu = 0;
+    if (hipError_t e = device_cu_count(&n_cu); e != hipSuccess) return e;
+    const int tile = gemm_tile(dtype, a, n_cu);
+    if (tile == 0) return hipErrorInvalidValue;
+    if (tile != 256) return launch_gemm_small(dtype, tile, a, s);
+    const int ntiles = (a.M / kBM) * (a.N / kBN);
+    const int grid = ntiles < n_cu ? ntiles : n_cu;  // one persistent WG per CU
+    if (dtype == 1)
+        hipLaunchKernelGGL(gemm_mfma_kernel<bf16_t>, dim3(grid), dim3(kThreads), 0, s, a);
+    else
+        hipLaunchKernelGGL(gemm_mfma_kernel<float>, dim3(grid), dim3(kThreads), 0, s, a);
+    return hipGetLastError();
 }
 
 // ---- weight preparation --------------------------------------------------------------

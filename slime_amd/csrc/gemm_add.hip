@@ -8,9 +8,12 @@
 namespace slime {
 
 hipError_t launch_gemm_add_f32(int dtype, const GemmArgs& a, const float* add, hipStream_t s) {
-    if (!gemm_uses_mfma(dtype, a) || a.N != a.ncol || a.act[0] != 0 || !add) return hipErrorInvalidValue;
+    if (a.N != a.ncol || a.act[0] != 0 || !add) return hipErrorInvalidValue;
     int n_cu = 0;
     if (hipError_t e = device_cu_count(&n_cu); e != hipSuccess) return e;
+    const int tile = gemm_tile(dtype, a, n_cu);
+    if (tile == 0) return hipErrorInvalidValue;
+    if (tile != 256) return launch_gemm_small_add(dtype, tile, a, add, s);
     const int ntiles = (a.M / kBM) * (a.N / kBN);
     const int grid = ntiles < n_cu ? ntiles : n_cu;  // one persistent WG per CU
     if (dtype == 1)

@@ -9,9 +9,12 @@
 namespace slime {
 
 hipError_t launch_gemm_tape(int dtype, const GemmArgs& a, void* pre, hipStream_t s) {
-    if (!gemm_uses_mfma(dtype, a) || !pre) return hipErrorInvalidValue;
+    if (!pre) return hipErrorInvalidValue;
     int n_cu = 0;
     if (hipError_t e = device_cu_count(&n_cu); e != hipSuccess) return e;
+    const int tile = gemm_tile(dtype, a, n_cu);
+    if (tile == 0) return hipErrorInvalidValue;
+    if (tile != 256) return launch_gemm_small_tape(dtype, tile, a, pre, s);
     const int ntiles = (a.M / kBM) * (a.N / kBN);
     const int grid = ntiles < n_cu ? ntiles : n_cu;  // one persistent WG per CU
     if (dtype == 1)

@@ -24,16 +24,22 @@ struct GemmArgs {
     int ncol;                  // columns per plane
     int act[3];                // 0 identity, 1 ReLU, 2 tanh-GELU
 };
-// Returns true when the MFMA tile kernel handles this shape (else the generic
-// kernel runs). dtype: 0 fp32, 1 bf16.
-bool gemm_uses_mfma(int dtype, const GemmArgs& a);
+// The tile that a launch on n_cu compute units uses: 256 (gemm_tile.hpp), 128 or 64
+// (gemm_small.hip); 0 when none fits the shape. dtype: 0 fp32, 1 bf16.
+int gemm_tile(int dtype, const GemmArgs& a, int n_cu);
 hipError_t launch_gemm(int dtype, const GemmArgs& a, hipStream_t s);
 // One output plane (N = ncol, identity) written as fp32 out[0] = A Bt^T + add, add of
-// out[0]'s layout (in place allowed); MFMA shapes only (else hipErrorInvalidValue).
+// out[0]'s layout and another buffer.
 hipError_t launch_gemm_add_f32(int dtype, const GemmArgs& a, const float* add, hipStream_t s);
 // As launch_gemm, and every output plane with the GELU activation is also written
-// before it to `pre` (that plane's layout); MFMA shapes only (else hipErrorInvalidValue).
+// before it to `pre` (that plane's layout).
 hipError_t launch_gemm_tape(int dtype, const GemmArgs& a, void* pre, hipStream_t s);
+// The same three in tiles of 128 or 64, for shapes that gemm_small_fits (else
+// hipErrorInvalidValue).
+bool gemm_small_fits(int dtype, int tile, const GemmArgs& a);
+hipError_t launch_gemm_small(int dtype, int tile, const GemmArgs& a, hipStream_t s);
+hipError_t launch_gemm_small_add(int dtype, int tile, const GemmArgs& a, const float* add, hipStream_t s);
+hipError_t launch_gemm_small_tape(int dtype, int tile, const GemmArgs& a, void* pre, hipStream_t s);
 
 // The perception input of the reference's S1 (pvi_chain = 2): S = the toroidal 3x3
 // neighbourhood sum of every channel of X, [B][G][G][C] in the storage type
@@ -215,8 +221,6 @@ long long backward_dw_rows_per_chunk(int dtype, int C, long long rows_per_pod);
 int backward_dw_chunks_per_pod(int dtype, int C, long long rows_per_pod);
 hipError_t launch_backward_stencil(int dtype, const BackwardArgs& a, hipStream_t s);
 hipError_t launch_backward_dw(int dtype, const BackwardArgs& a, const DwArgs& d, hipStream_t s);
-hipError_t launch_backward_final(int dtype, const float* gXd, const void* gXp, float* gX, long long n,
-                                 hipStream_t s);
 
 // ---- organism adapters (slime/core/organism.cu:691-743) -----------------------------
 hipError_t launch_init_from_field(int dtype, const float* conc, void* X, int G, int C,
