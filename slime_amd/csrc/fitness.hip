@@ -16,7 +16,7 @@
 // The reference launches SVD, rank and coherence as dynamic-parallelism children
 // of one parent (slime/kernels/warp_ca.cu:178-226). Here two stream-ordered
 // kernels do the work: a wide pass over the history that writes per-chunk fp64
-// Gram and moment partials, then one wave per (batch, head) that reduces them in
+// Gram and moment partials, then one workgroup per (batch, head) that reduces them in
 // fixed order, runs the cyclic Jacobi on the fp64 matrix in LDS, and finishes
 // rank, coherence and fitness.
 #include <cstring>
@@ -24,6 +24,7 @@
 
 #include "common.hpp"
 #include "fp64.hpp"
+#include "jacobi_wave.hpp"
 #include "kernels.hpp"
 
 // Scratch of the allocation-free entry point slime_ca_fitness_static: the Gram and
@@ -226,51 +227,62 @@ __global__ __launch_bounds__(256) void fitness_partial_kernel(FitnessArgs f) {
     }
 }
 
-// Value of v in lane l (l uniform), through two 32-bit lane reads.
-__device__ __forceinline__ double lane_f64(double v, int l) {
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
 // Keeps the compiler from moving LDS accesses across this point. The block is one
 // wave and LDS executes a wave's accesses in issue order, so program order is all
 // the ordering that one lane's write and another lane's later read need.
 __device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
 
-// One wave per (batch, head): fixed-order reduction of the partials, the cyclic
+// Workgroup barrier for LDS data.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // s_waitcnt lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// One workgroup per (batch, head): fixed-order reduction of the partials, the cyclic
 // two-sided Jacobi solve in fp64, then rank, coherence and fitness.
 //
-// The solve visits the pairs (p, q) in the reference's cyclic row order
+// The solve rotates the pairs (p, q) in the reference's cyclic row order
 // (failed_attempts/pseudopod.cu:391-436) and skips |a_pq| <= 1e-6. That absolute
-// threshold makes the converged diagonal depend on the visiting order when the
-// Gram is nearly singular, so the order is kept rather than a parallel one, and the
-// rotation chain is serial. Its latency is kept to the scalar arithmetic: lane i
-// holds column p (A[i][p]) and the diagonal (A[i][i]) in registers, so a_pq and
-// a_qq of the next pair are lane reads of registers rather than LDS round trips.
-// The matrix stays in LDS (exactly symmetric: each new value is written to both
-// (i, p) and (p, i)); column q is read from it once per rotation, in parallel with
-// the rotation's scalar chain, and column p once per row p. The chain's divisions
-// and square roots use the short correctly rounded forms of fp64.hpp, whose
-// preconditions every Gram of fp32 data meets.
+// threshold makes the converged diagonal depend on the order when the Gram is nearly
+// singular, so the order is kept. What bounds it is the chain of a rotation's fp64
+// operations (four hardware estimates in a row with their refinements, ~600 cycles), so
+// the solve runs the cyclic order as a wave front (jacobi_wave.hpp): the up to D / 2
+// rotations of a step share no index, commute, and run in the lanes of one wave, D steps
+// to a sweep instead of D (D - 1) / 2 rotations; every rotation sees the values that the
+// serial order would give it, up to the fp64 rounding of commuted updates.
 //
-// Skipped pairs cost no serial step: one ballot over column p finds the next pair
-// that rotates, and each lane keeps its own share of the off-diagonal sum, added
-// across lanes at the end of the sweep (the reference adds the same |a_pq| values
-// one by one in visiting order; the two sums can differ in their last bits, and
-// only their comparison with 1e-6 n is used). Since a pair at or below 1e-6 is
-// never rotated, that sum usually stays above 1e-6 n and the solve runs to its
-// 30-sweep limit, the last sweeps rotating nothing; a sweep that rotates nothing
-// ends the solve at once with the same matrix and sweep count.
-template <int D>
-__global__ __launch_bounds__(64) void fitness_finalize_kernel(FitnessArgs f) {
-    constexpr int kLd = D + 1;  // padded row
-    __shared__ double A[D * kLd];
-    __shared__ double rho[64];
+// Wave 0 computes the rotations, one step ahead: for step T + 1 it reads four elements
+// of the matrix as it was before step T and applies step T's rotations to them itself,
+// while the other waves apply step T to the whole upper triangle, from one LDS copy to
+// the other; one barrier per step. The diagonal is wave 0's alone. A step without a
+// rotation leaves the matrix alone.
+//
+// A sweep's last rotations run beside the first ones of the next sweep, so each index's
+// diagonal is noted when its row of the sweep is done, and the result is the noted
+// diagonal of the sweep that ends the solve: the one whose sum |a_pq| is below 1e-6 D,
+// the one that rotated nothing (every later sweep would repeat it up to the limit, and
+// 30 sweeps are reported, as the reference runs them), or the 30th.
+//
+// Measured on 128 Grams of 64 x 64 (16 pods x 8 heads, ~11.7k rotations each): 377 us,
+// 2920 us as one rotation at a time. A step takes the chain's latency plus one LDS round
+// trip and the barrier; the update waves (one item each) stay below that.
+constexpr int kFinUpdate = 512;                // threads that apply the rotations
+constexpr int kFinThreads = 64 + kFinUpdate;   // wave 0 computes them
 
-    const int bh = blockIdx.x, lane = threadIdx.x;
-    const bool own = D == kWave || lane < D;  // lane owns row/column `lane` of the matrix
+template <int D>
+__global__ __launch_bounds__(kFinThreads) void fitness_finalize_kernel(FitnessArgs f) {
+    using namespace jacobi_wave;
+    constexpr int S = D / 2;  // pairs per step
+    __shared__ double A[2][D * D];  // upper triangle
+    __shared__ __attribute__((aligned(16))) double2 cs[2][D];  // new a_i = c a_i + s a_partner
+    __shared__ int flag[2];  // a step's: 0 no rotation, 1 rotations, 2 the solve has ended
+    __shared__ double dg[D];  // the diagonal (wave 0 only)
+    __shared__ double rho[64];
+    __shared__ double sv[D], term[D];
+
+    const int bh = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const double ncell = (double)f.G * f.G;
     const double tol = 1e-6;
     const int BH = gridDim.x;
@@ -279,142 +291,194 @@ __global__ __launch_bounds__(64) void fitness_finalize_kernel(FitnessArgs f) {
     const double s_last = scale_of(f.T - 1);
     const double gram_scale = s_last * s_last / ncell;
 
-    // Fixed-order reduction of the Gram partials: element e sums chunks 0, 1, ... in
-    // turn; kE elements per lane at once keep the loads independent.
+    // Fixed-order reduction of the Gram partials: an element sums chunks 0, 1, ... in turn.
     {
-        constexpr int kE = D * D >= 4 * 64 ? 4 : D * D / 64;  // D * D is a multiple of 64
-        static_assert(D * D % (kE * 64) == 0, "whole groups of elements");
         const double* gp = f.gram_part + (long long)bh * f.chunks * D * D;
-        for (int e0 = 0; e0 < D * D; e0 += kE * 64) {
-            double s[kE];
-#pragma unroll
-            for (int k = 0; k < kE; ++k) s[k] = 0.0;
-#pragma unroll 4
-            for (int c = 0; c < f.chunks; ++c)
-#pragma unroll
-                for (int k = 0; k < kE; ++k) s[k] += gp[(long long)c * D * D + e0 + k * 64 + lane];
-#pragma unroll
-            for (int k = 0; k < kE; ++k) {
-                const int e = e0 + k * 64 + lane;
-                A[(e / D) * kLd + e % D] = f.scales ? s[k] * gram_scale : s[k] / ncell;
-            }
+        for (int e = tid; e < D * D; e += kFinThreads) {
+            if (e % D < e / D) continue;
+            double s = 0.0;
+#pragma unroll 8
+            for (int c = 0; c < f.chunks; ++c) s += gp[(long long)c * D * D + e];
+            A[0][e] = f.scales ? s * gram_scale : s / ncell;
         }
+        if (tid < 2) flag[tid] = 0;
     }
     __syncthreads();
 
-    double diag = own ? A[lane * kLd + lane] : 0.0;
-    int sweeps = 0;
-    for (int sweep = 0; sweep < 30; ++sweep) {
-        ++sweeps;
-        double offl = 0.0;  // lane q: sum over the rows p < q of |a_pq| when (p, q) is visited
-        bool rotated = false;
-        for (int p = 0; p < D - 1; ++p) {
-            lds_order();
-            double colp = own ? A[lane * kLd + p] : 0.0;  // A[lane][p] = a_p,lane
-            // The read has landed before the rotations start; without this the loop
-            // head waits for every LDS access in flight, the previous rotation's
-            // writes included, on each rotation.
-            asm volatile("" : "+v"(colp));
-            double app = lane_f64(diag, p);
-            for (int q = p + 1;;) {
-                // Pairs (p, q..) with |a_pq| <= tol are skipped without changing anything,
-                // so the next rotation is at the lowest lane >= q whose column-p entry
-                // exceeds tol; the skipped pairs only add their |a_pq| to the sum.
-                const bool ahead = own && lane >= q;
-                const unsigned long long m = __ballot(ahead && fabs(colp) > tol);
-                const int qn = m ? (int)__builtin_ctzll(m) : D;
-                if (ahead && lane <= qn) offl += fabs(colp);  // lane qn: the rotated pair's a_pq
-                if (qn >= D) break;
-                lds_order();
-                const double colq = own ? A[lane * kLd + qn] : 0.0;
-                const double apq = lane_f64(colp, qn);
-                const double aqq = lane_f64(diag, qn);
-                double c, s;
-                jacobi_rotation<true>(app, aqq, apq, c, s);
-                const double app_new = c * c * app + s * s * aqq - 2.0 * c * s * apq;
-                const double aqq_new = s * s * app + c * c * aqq + 2.0 * c * s * apq;
-                double np = c * colp - s * colq;
-                double nq = s * colp + c * colq;
-                if (lane == p) {
-                    np = app_new;
-                    nq = 0.0;
-                } else if (lane == qn) {
-                    np = 0.0;
-                    nq = aqq_new;
+    int cur = 0;
+    if (tid >= 64) {
+        // ---- apply step T to the matrix ----------------------------------------------------
+        // One item per thread (D = 64), and threads 0 .. S - 1 a rotated pair's own element.
+        static_assert(S * S / 2 <= kFinUpdate, "one work item per thread");
+        const int u = tid - 64;
+        int d1, d2;
+        const bool act = u < S * S / 2 && item(u, S, &d1, &d2), pairs = u < S;
+        for (int T = 0;; ++T) {
+            const int sig = T & (D - 1);
+            const double* M = A[cur];
+            double* W = A[cur ^ 1];
+            const double2* r = cs[T & 1];
+            int i1 = 0, j1 = 1, i2 = 0, j2 = 1, pi = 0, pj = 1;
+            if (act) slot(sig, d1, D, &i1, &j1), slot(sig, d2, D, &i2, &j2);
+            if (pairs) slot(sig, u, D, &pi, &pj);
+            const int ea = upper(i1, i2, D), eb = upper(i1, j2, D), ec = upper(j1, i2, D), ed = upper(j1, j2, D);
+            const int ep = upper(pi, pj, D);
+            // all reads at once, before the step is known to rotate anything
+            const int fl = flag[T & 1];
+            const double2 r1 = r[i1], r2 = r[i2];
+            const double a = M[ea], b = M[eb], c = M[ec], d = M[ed];
+            const double ps = r[pi].y, pv = M[ep];
+            if (fl == 2) return;
+            if (fl) {
+                if (act) {
+                    const double ar = r1.x * a + r1.y * c, br = r1.x * b + r1.y * d;
+                    const double cr = r1.x * c - r1.y * a, dr = r1.x * d - r1.y * b;
+                    W[ea] = r2.x * ar + r2.y * br;
+                    W[eb] = r2.x * br - r2.y * ar;
+                    W[ec] = r2.x * cr + r2.y * dr;
+                    W[ed] = r2.x * dr - r2.y * cr;
                 }
-                if (own) {
-                    A[lane * kLd + p] = np;
-                    A[p * kLd + lane] = np;
-                    A[lane * kLd + qn] = nq;
-                    A[qn * kLd + lane] = nq;
-                }
-                diag = lane == p ? app_new : (lane == qn ? aqq_new : diag);
-                colp = np;
-                app = app_new;
-                rotated = true;
-                q = qn + 1;
+                if (pairs) W[ep] = ps != 0.0 ? 0.0 : pv;
+                cur ^= 1;
             }
-        }
-        const double off = wave_sum_f64(offl);
-        if (off < tol * D) break;
-        // A sweep without a rotation leaves the matrix as it found it, so every later
-        // sweep repeats it exactly: the solve ends at the sweep limit.
-        if (!rotated) {
-            sweeps = 30;
-            break;
+            lds_barrier();
         }
     }
-    lds_order();
+
+    // ---- wave 0: the rotations of step T + 1 --------------------------------------------------
+    const bool own = D == kWave || lane < D;
+    double c = 1.0, s = 0.0;           // this lane's rotation of step T
+    double off = 0.0, off_done = 0.0;  // this row's share of sum |a_pq|: running, and of its last whole sweep
+    bool rot = false, rot_done = false;
+    double diag = 0.0;                 // index `lane`'s diagonal at the end of that sweep
+    int sweeps = 0;
+    bool any = false;                  // step T rotates
+    if (own) dg[lane] = A[0][lane * D + lane];
+    // The four elements of a step, with m = q_partner_before(p): (p, m), (p, q), (q - 1, m)
+    // and (q - 1, q), are at offsets linear in q (lanes without a pair read in range and
+    // use nothing).
+    const int lp = own ? lane : 0, m = q_partner_before(lp, D);
+    const int at1 = upper(lp, m, D);
+    const int at3_0 = lp > 0 ? m * D - 1 : m - D, at3_q = lp > 0 ? 1 : D;
+    for (int T = 0;; ++T) {
+        const int sig = (T + 1) & (D - 1);
+        const Role ro = role(sig, lane, D);
+        const bool pair = own && ro.pair, self = own && ro.self;
+        const int q = ro.q > 0 ? ro.q : 1;
+        const double* M = A[cur];
+        lds_order();
+        const double e1 = M[at1], e2 = M[lp * D + q], e3 = M[at3_0 + q * at3_q], e4 = M[q * (D + 1) - D];
+        const double app = dg[lp];
+        double aqq = dg[q];
+        double2 rq = cs[T & 1][q];  // index q's rotation of step T, with index m
+        asm volatile("" : "+v"(aqq));  // read here, not where it is first used
+        if (!any) rq = make_double2(1.0, 0.0);
+        const double x = c * e1 - s * e3, y = c * e2 - s * e4;
+        const double apq = rq.y * x + rq.x * y;
+        const bool real = pair && (T + 1 >= D || !ro.prev);  // sweep 0 has no sweep before it
+        const double mag = real ? fabs(apq) : 0.0;
+        const bool rotate = mag > tol;
+        const bool any1 = __ballot(rotate) != 0;
+        c = 1.0;
+        s = 0.0;
+        double app_now = app;
+        if (any1) {
+            double cr, sr;
+            jacobi_rotation<true>(app, aqq, rotate ? apq : 1.0, cr, sr);
+            const double app_new = cr * cr * app + sr * sr * aqq - 2.0 * cr * sr * apq;
+            const double aqq_new = sr * sr * app + cr * cr * aqq + 2.0 * cr * sr * apq;
+            c = rotate ? cr : 1.0;
+            s = rotate ? sr : 0.0;
+            app_now = rotate ? app_new : app;
+            double2* w = cs[(T + 1) & 1];
+            if (own && !(ro.q < lane)) {  // a pair, or an index that rests: both writes are its own
+                w[ro.q] = make_double2(c, s);
+                w[lane] = make_double2(c, -s);
+                dg[ro.q] = rotate ? aqq_new : aqq;
+                dg[lane] = app_now;
+            }
+        }
+        if (self) {
+            off = 0.0;
+            rot = false;
+        }
+        off += mag;
+        rot = rot || rotate;
+        if (own && ro.q == D - 1) {  // this row's sweep is done (index D - 1: with all others)
+            diag = app_now;
+            off_done = off;
+            rot_done = rot;
+        }
+        bool end = false;
+        if (sig == D - 2 && T + 1 >= 2 * D - 2) {
+            sweeps = (T + 1) / D;
+            const bool converged = wave_sum_f64(own ? off_done : 0.0) < tol * D;
+            const bool idle = __ballot(own && rot_done) == 0;
+            if (idle && !converged) sweeps = 30;
+            end = converged || idle || sweeps == 30;
+        }
+        if (lane == 0) flag[(T + 1) & 1] = end ? 2 : (any1 ? 1 : 0);
+        cur ^= any ? 1 : 0;
+        any = any1;
+        lds_barrier();
+        if (end) break;
+    }
 
     // Coherence from the per-state sums: pair t = (t - 1, t) has sum a = S1(t-1),
     // sum b = S1(t), sum ab = P(t), sum aa = S2(t-1), sum bb = S2(t); chunks in order.
     const int npair = f.T - 1;
     const double n = ncell * D;
     for (int t = lane + 1; t < f.T; t += 64) {
-        double m[5] = {0, 0, 0, 0, 0};
-        for (int c = 0; c < f.chunks; ++c) {
-            const double* q = f.mom_part + ((long long)bh * f.chunks + c) * f.T * 3;
-            m[0] += q[(t - 1) * 3];
-            m[1] += q[t * 3];
-            m[2] += q[t * 3 + 2];
-            m[3] += q[(t - 1) * 3 + 1];
-            m[4] += q[t * 3 + 1];
+        double mo[5] = {0, 0, 0, 0, 0};
+        for (int ch = 0; ch < f.chunks; ++ch) {
+            const double* qm = f.mom_part + ((long long)bh * f.chunks + ch) * f.T * 3;
+            mo[0] += qm[(t - 1) * 3];
+            mo[1] += qm[t * 3];
+            mo[2] += qm[t * 3 + 2];
+            mo[3] += qm[(t - 1) * 3 + 1];
+            mo[4] += qm[t * 3 + 1];
         }
         if (f.scales) {
             const double sa = scale_of(t - 1), sb = scale_of(t);
-            m[0] *= sa;
-            m[1] *= sb;
-            m[2] *= sa * sb;
-            m[3] *= sa * sa;
-            m[4] *= sb * sb;
+            mo[0] *= sa;
+            mo[1] *= sb;
+            mo[2] *= sa * sb;
+            mo[3] *= sa * sa;
+            mo[4] *= sb * sb;
         }
-        const double cov = m[2] - m[0] * m[1] / n;
-        const double va = m[3] - m[0] * m[0] / n;
-        const double vb = m[4] - m[1] * m[1] / n;
+        const double cov = mo[2] - mo[0] * mo[1] / n;
+        const double va = mo[3] - mo[0] * mo[0] / n;
+        const double vb = mo[4] - mo[1] * mo[1] / n;
         const double den = sqrt(fmax(va, 0.0) * fmax(vb, 0.0));
         rho[t - 1] = den > 0.0 ? cov / den : 0.0;
     }
-    double* sv = A;  // the matrix is no longer needed: its first row holds the singular values
-    __syncthreads();
-    if (own) sv[lane] = sqrt(fabs(diag));
-    __syncthreads();
-    if (lane == 0) {
-        for (int i = 1; i < D; ++i) {  // descending insertion sort
-            const double v = sv[i];
-            int j = i - 1;
-            while (j >= 0 && sv[j] < v) {
-                sv[j + 1] = sv[j];
-                --j;
-            }
-            sv[j + 1] = v;
-        }
-        double sum = 0.0;
-        for (int i = 0; i < D; ++i) sum += sv[i];
-        double ent = 0.0;
+    // Singular values in descending order (each lane counts the ones before its own), then
+    // the sums in that order.
+    const double v = own ? sqrt(fabs(diag)) : 0.0;
+    if (own) term[lane] = v;
+    lds_order();
+    if (own) {
+        int rank = 0;
+#pragma unroll 8
         for (int i = 0; i < D; ++i) {
-            const double p = sv[i] / (sum + 1e-7);
-            ent += -p * log(p + 1e-7);
+            const double o = term[i];
+            rank += o > v || (o == v && i < lane) ? 1 : 0;
         }
+        sv[__ballot(v != v) ? lane : rank] = v;  // NaN has no rank, and every order gives NaN
+    }
+    lds_order();
+    double sum = 0.0;
+#pragma unroll 8
+    for (int i = 0; i < D; ++i) sum += sv[i];
+    if (own) {
+        const double pr = sv[lane] / (sum + 1e-7);
+        term[lane] = -pr * log(pr + 1e-7);
+    }
+    lds_order();
+    if (lane == 0) {
+        double ent = 0.0;
+#pragma unroll 8
+        for (int i = 0; i < D; ++i) ent += term[i];
         const double er = exp(ent);
         double rs_ = 0.0;
         for (int t = 0; t < npair; ++t) rs_ += rho[t];
@@ -431,7 +495,7 @@ hipError_t launch_td(const FitnessArgs& f, hipStream_t s) {
     hipLaunchKernelGGL((fitness_partial_kernel<T, D>), dim3(f.B * kHeads, f.chunks), dim3(256), 0, s, f);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(fitness_finalize_kernel<D>, dim3(f.B * kHeads), dim3(64), 0, s, f);
+    hipLaunchKernelGGL(fitness_finalize_kernel<D>, dim3(f.B * kHeads), dim3(kFinThreads), 0, s, f);
     return hipGetLastError();
 }
 
