@@ -201,9 +201,9 @@ int slime_ca_fitness_scaled(slime_ca* ca, const void* x_hist, const double* scal
  * reference. For callers that cannot call hipMalloc (code under HIP graph capture,
  * tight serving loops, harnesses that forbid allocation). The partial sums go to a
  * static device buffer of 32 MiB per GPU that the library holds until the process
- * ends; B*H*chunks*(D*D + 3T) fp64 partials must fit, with the chunk count lowered
- * from slime_ca_fitness's when needed (which can change the last bits of the Gram
- * sums), else SLIME_EINVAL. Every call on a GPU shares that buffer: a call on
+ * ends; B*H*(D*D + 3T) fp64 partials must fit (more where they do, with the cells
+ * split into fewer parts than slime_ca_fitness's when needed, which can change the
+ * last bits of the sums), else SLIME_EINVAL. Every call on a GPU shares that buffer: a call on
  * another stream than the previous call's waits for it (an event recorded after
  * each call), but under graph capture no event is used, and replays that overlap
  * on one GPU race. Loading the library reserves the buffer on every GPU it runs

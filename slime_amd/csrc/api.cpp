@@ -50,7 +50,6 @@ struct slime_ca {
     double* mass_in = nullptr;             // [B*H]
     double* mass_out = nullptr;
 
-    int fit_chunks = 0;
     int fit_T = 0;             // history length the fitness partials are sized for
     double* gram_part = nullptr;
     double* mom_part = nullptr;
@@ -330,20 +329,16 @@ int run_fitness(slime_ca* h, const void* x_hist, long long t_stride, int T, floa
                 float* coherence, float* fitness, hipStream_t s, const double* scales = nullptr) {
     const slime_ca_config& c = h->cfg;
     const size_t BH = (size_t)c.B * c.H;
-    const int chunks = fitness_chunks(c.G);
-    if (chunks < 1) return fail(SLIME_EINVAL, "grid too small for the fitness pass");
+    const FitnessChunks chunks = fitness_chunks(c.B, c.G);
     int rc = SLIME_OK;
-    if (!h->gram_part || h->fit_chunks != chunks) {
-        if (h->gram_part) (void)hipFree(h->gram_part);
-        h->gram_part = nullptr;
-        rc = dalloc_t(&h->gram_part, BH * chunks * c.D * c.D * 8);
+    if (!h->gram_part) {
+        rc = dalloc_t(&h->gram_part, BH * chunks.gram * c.D * c.D * 8);
         if (rc) return rc;
-        h->fit_chunks = chunks;
     }
     if (!h->mom_part || h->fit_T < T) {
         if (h->mom_part) (void)hipFree(h->mom_part);
         h->mom_part = nullptr;
-        rc = dalloc_t(&h->mom_part, BH * chunks * (size_t)T * 3 * 8);
+        rc = dalloc_t(&h->mom_part, BH * chunks.mom * (size_t)T * 3 * 8);
         if (rc) return rc;
         h->fit_T = T;
     }
@@ -357,7 +352,8 @@ int run_fitness(slime_ca* h, const void* x_hist, long long t_stride, int T, floa
     f.D = c.D;
     f.gram_part = h->gram_part;
     f.mom_part = h->mom_part;
-    f.chunks = chunks;
+    f.chunks = chunks.gram;
+    f.mom_chunks = chunks.mom;
     f.erank = erank;
     f.coh = coherence;
     f.fitness = fitness;
@@ -698,13 +694,12 @@ int slime_ca_fitness_static(const slime_ca_config* config, const void* x_hist, i
         return fail(SLIME_EINVAL, "a tensor pointer is NULL");
     if (T < 2 || T > 65) return fail(SLIME_EINVAL, "T=%d must be in [2, 65]", T);
     const slime_ca_config& c = *config;
-    if (fitness_chunks(c.G) < 1) return fail(SLIME_EINVAL, "grid too small for the fitness pass");
-    const int chunks = fitness_static_chunks(c.B, c.G, c.D, T);
-    if (chunks < 1)
+    const FitnessChunks chunks = fitness_static_chunks(c.B, c.G, c.D, T);
+    if (chunks.gram < 1)
         return fail(SLIME_EINVAL,
                     "B=%d, D=%d, T=%d needs %zu bytes of partial sums, more than the %zu-byte "
                     "static scratch of slime_ca_fitness_static (use slime_ca_fitness)",
-                    c.B, c.D, T, fitness_partial_bytes(c.B, c.D, T, 1), kFitnessScratchBytes);
+                    c.B, c.D, T, fitness_partial_bytes(c.B, c.D, T, FitnessChunks{1, 1}), kFitnessScratchBytes);
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1)
         return fail(SLIME_ENODEV, "no HIP device visible");
@@ -715,7 +710,8 @@ int slime_ca_fitness_static(const slime_ca_config* config, const void* x_hist, i
     f.B = c.B;
     f.G = c.G;
     f.D = c.D;
-    f.chunks = chunks;
+    f.chunks = chunks.gram;
+    f.mom_chunks = chunks.mom;
     f.erank = erank;
     f.coh = coherence;
     f.fitness = fitness;

@@ -19,6 +19,7 @@
 // Gram and moment partials, then one workgroup per (batch, head) that reduces them in
 // fixed order, runs the cyclic Jacobi on the fp64 matrix in LDS, and finishes
 // rank, coherence and fitness.
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 
@@ -40,8 +41,6 @@ static __device__ __align__(256) unsigned char scratch[slime::kFitnessScratchByt
 namespace slime {
 namespace {
 
-constexpr int kCellsPerStage = 64;
-
 // State t of the history starts t * f.t_stride bytes after f.hist. The stride may be
 // negative: two separately allocated states form a history of two.
 template <typename T>
@@ -55,32 +54,33 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
     return v;
 }
 
-// Up to kTB states are read per pass over a chunk; their sums stay in registers.
-constexpr int kTB = 8;
+// The partial pass has two kinds of workgroups in one launch, interleaved so that the
+// matrix cores' work runs beside the other kind's streaming:
+//   moments: per (batch, chunk of cells) and every state t of the history, each head's sums
+//     S1 = sum x_t, S2 = sum x_t^2 and P = sum x_{t-1} x_t (P of state 0 is 0), which give
+//     the lag-1 moments of each consecutive pair. A workgroup reads whole cells, all heads
+//     (a state's rows are contiguous), and a thread's 16-byte pieces always belong to one
+//     head. Bound by HBM.
+//   Gram: per (batch, head, chunk) the D x D Gram partial of the last state on the fp64
+//     matrix cores (v_mfma_f64_16x16x4), the blocks on and above the diagonal only.
+// Products of the fp32 values are exact in fp64 and accumulate in fp64, so the partials
+// carry no accumulation error that the Jacobi solve could amplify on a nearly singular
+// Gram (small eigenvalues enter the rank through their square roots).
+//
+// Measured at 8 states of 16 x 128^2 x 512 bf16 (2.15 GB): 461 us = 4.66 TB/s (a copy reaches
+// 4.84), 784 us with the Gram on the VALU in the same workgroups and one head's 128-byte row
+// segments per workgroup; 2 states of 128^2 x 512 fp32: 27 us, 127 us with 128 workgroups
+// and eight states' loads whatever T.
+constexpr int kUnit = 64;  // cells per Gram step of a workgroup: 16 per wave
 
-// The 16-byte pieces of state t that thread `tid` owns in the stage whose head-h
-// slice starts `stage_off` bytes into each state: piece j is (cell, channel group)
-// = divmod(tid + 256 j, D / elements-per-piece). The uniform part of the address
-// is one scalar base per state; the per-thread part is a small byte offset that
-// does not change between stages or states. Pieces past the stage hold zeros.
-template <typename T, int D, int kPPT>
-__device__ __forceinline__ void load_pieces(const FitnessArgs& f, int t, long long stage_off, int tid,
-                                            uint4 (&x)[kPPT]) {
-    constexpr int kCE = 16 / (int)sizeof(T);
-    constexpr int kCPR = D / kCE;
-    constexpr int kPieces = kCellsPerStage * kCPR;
-    constexpr int C = kHeads * D;
-    const char* base = static_cast<const char*>(f.hist) + t * f.t_stride + stage_off;
-#pragma unroll
-    for (int j = 0; j < kPPT; ++j) {
-        const int q = tid + 256 * j;
-        if (kPieces % 256 == 0 || q < kPieces) {
-            const unsigned off = (unsigned)(((q / kCPR) * C + (q % kCPR) * kCE) * (int)sizeof(T));
-            x[j] = *reinterpret_cast<const uint4*>(base + off);
-        } else {
-            x[j] = make_uint4(0u, 0u, 0u, 0u);
-        }
-    }
+// Workgroup k of n_g Gram and n_m moment workgroups: groups of 8 (one per XCD), the kinds
+// spread evenly over the launch. Returns its kind's index; -1 past the end.
+__device__ __forceinline__ long long split_kinds(long long k, long long n_g, long long n_m, bool* gram) {
+    const long long gg = (n_g + 7) / 8, gm = (n_m + 7) / 8, g = k >> 3;
+    const long long before = g * gg / (gg + gm), after = (g + 1) * gg / (gg + gm);
+    *gram = after > before;
+    const long long idx = 8 * (*gram ? before : g - before) + (k & 7);
+    return idx < (*gram ? n_g : n_m) ? idx : -1;
 }
 
 template <typename T>
@@ -94,71 +94,72 @@ __device__ __forceinline__ void unpack_piece(const uint4& v, float (&e)[16 / siz
     }
 }
 
-// Per (batch, head, chunk of cells): the D x D Gram partial of the last state, and
-// for every state t the sums S1 = sum x_t, S2 = sum x_t^2 and P = sum x_{t-1} x_t
-// (P of state 0 is 0), which give the lag-1 moments of each consecutive pair.
-// Products of the fp32 values are exact in fp64 and accumulate in fp64, so the
-// partials carry no accumulation error that the Jacobi solve could amplify on a
-// nearly singular Gram (small eigenvalues enter the rank through their square
-// roots). Each pass over the chunk reads states tb - 1 .. tb + kTB - 1 once, with
-// 16-byte loads, all of a stage's loads in flight together; the last pass stages
-// the last state through LDS for the Gram.
+// The geometry of a moment workgroup's reads.
 template <typename T, int D>
-__global__ __launch_bounds__(256) void fitness_partial_kernel(FitnessArgs f) {
-    constexpr int H = kHeads;
-    constexpr int kCE = 16 / (int)sizeof(T);   // elements per 16-byte piece
-    constexpr int kCPR = D / kCE;               // pieces per cell of one head
-    constexpr int kPieces = kCellsPerStage * kCPR;
-    constexpr int kPPT = (kPieces + 255) / 256;  // pieces per thread
-    constexpr int kBS = 4;                      // Gram block edge per thread
-    constexpr int kBlk = D / kBS;               // blocks per side (16 at D = 64)
-    static_assert(kBlk * kBlk <= 256, "one Gram block per thread");
-    __shared__ __attribute__((aligned(16))) float sx[kCellsPerStage * D];
-    __shared__ double sred[4][3 * kTB];
+struct Rows {
+    static constexpr int kCE = 16 / (int)sizeof(T);             // elements per 16-byte piece
+    static constexpr int kPPC = kHeads * D / kCE;                // pieces per cell, a power of two
+    static constexpr int kPPH = D / kCE;                         // ... of one head
+    static constexpr int kCells = 256 / kPPC;                    // cells the workgroup reads at once
+    static constexpr int kPPT = 2;                               // pieces per thread and state in flight
+    static constexpr int kStage = kCells * kPPT;                 // cells per stage; divides 64
+    static constexpr int kHW = kPPC <= 64 ? kHeads : 64 / kPPH;  // heads in a wave
+};
 
-    const int bh = blockIdx.x, chunk = blockIdx.y;
-    const int b = bh / H, h = bh % H;
+// Sum over the lanes of a wave that hold the same head: the kPPH lanes of a cell, then the
+// wave's cells.
+template <typename R>
+__device__ __forceinline__ double head_sum(double v) {
+    if constexpr (R::kPPH >= 2) v += dpp_f64<0xB1>(v);
+    if constexpr (R::kPPH >= 4) v += dpp_f64<0x4E>(v);
+    if constexpr (R::kPPH >= 8) v += dpp_f64<0x141>(v);
+    if constexpr (R::kPPH >= 16) v += dpp_f64<0x140>(v);
+#pragma unroll
+    for (int m = R::kPPC; m < 64; m *= 2) v += __shfl_xor(v, m, 64);
+    return v;
+}
+
+// Moments of up to kTB states per pass over the chunk; each pass reads states tb - 1 ..
+// tb + kTB - 1 once, a stage's loads all in flight together.
+template <typename T, int D, int kTB>
+__device__ __forceinline__ void moments(const FitnessArgs& f, int b, int chunk, double* sred) {
+    using R = Rows<T, D>;
+    constexpr int kItems = 3 * kTB;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const long long cells = (long long)f.G * f.G;
-    const long long cpc = cells / f.chunks;
-    const long long c_begin = chunk * cpc;
-
-    const bool gact = tid < kBlk * kBlk;
-    const int bi = tid / kBlk, bj = tid % kBlk;
-    double g[kBS][kBS];
-#pragma unroll
-    for (int i = 0; i < kBS; ++i)
-#pragma unroll
-        for (int j = 0; j < kBS; ++j) g[i][j] = 0.0;
-
-    double* mp = f.mom_part + ((long long)bh * f.chunks + chunk) * f.T * 3;
+    const long long cells = (long long)f.G * f.G, stages = cells / R::kStage;
+    const long long st0 = stages * chunk / f.mom_chunks, st1 = stages * (chunk + 1) / f.mom_chunks;
+    const int row_bytes = kHeads * D * (int)sizeof(T);
+    const unsigned off = (unsigned)(tid * 16);  // cell tid / kPPC of the read, piece tid % kPPC
     for (int tb = 0; tb < f.T; tb += kTB) {
         const int tn = min(kTB, f.T - tb);  // states tb .. tb + tn - 1 in this pass
-        const bool last = tb + tn == f.T;
         double s1[kTB], s2[kTB], pr[kTB];
 #pragma unroll
         for (int k = 0; k < kTB; ++k) s1[k] = s2[k] = pr[k] = 0.0;
-        for (long long c0 = c_begin; c0 < c_begin + cpc; c0 += kCellsPerStage) {
-            const long long stage_off = (((long long)b * cells + c0) * (kHeads * D) + h * D) * (long long)sizeof(T);
-            uint4 x[kTB + 1][kPPT];  // states tb - 1 .. tb + kTB - 1
-            if (tb > 0) {
-                load_pieces<T, D, kPPT>(f, tb - 1, stage_off, tid, x[0]);
-            } else {
+        for (long long st = st0; st < st1; ++st) {
+            const long long base = (b * cells + st * R::kStage) * row_bytes;
+            uint4 x[kTB + 1][R::kPPT];  // states tb - 1 .. tb + kTB - 1
 #pragma unroll
-                for (int j = 0; j < kPPT; ++j) x[0][j] = make_uint4(0u, 0u, 0u, 0u);
+            for (int k = 0; k <= kTB; ++k)
+#pragma unroll
+                for (int j = 0; j < R::kPPT; ++j) x[k][j] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+            for (int k = 0; k <= kTB; ++k) {
+                const int t = tb + k - 1;
+                if (t < 0 || t >= f.T) continue;  // uniform; those sums are unused
+                const char* src = static_cast<const char*>(f.hist) + t * f.t_stride + base;
+#pragma unroll
+                for (int j = 0; j < R::kPPT; ++j)
+                    x[k][j] = *reinterpret_cast<const uint4*>(src + j * 4096 + off);
             }
-            // Past the last state the loads repeat it (cached); those sums are unused.
-#pragma unroll
-            for (int k = 0; k < kTB; ++k) load_pieces<T, D, kPPT>(f, min(tb + k, f.T - 1), stage_off, tid, x[k + 1]);
 #pragma unroll
             for (int k = 0; k < kTB; ++k)
 #pragma unroll
-                for (int j = 0; j < kPPT; ++j) {
-                    float a[kCE], e[kCE];
+                for (int j = 0; j < R::kPPT; ++j) {
+                    float a[R::kCE], e[R::kCE];
                     unpack_piece<T>(x[k][j], a);
                     unpack_piece<T>(x[k + 1][j], e);
 #pragma unroll
-                    for (int u = 0; u < kCE; ++u) {
+                    for (int u = 0; u < R::kCE; ++u) {
                         const double va = a[u], vb = e[u];
                         s1[k] += vb;
                         s2[k] = __builtin_fma(vb, vb, s2[k]);
@@ -167,64 +168,141 @@ __global__ __launch_bounds__(256) void fitness_partial_kernel(FitnessArgs f) {
                     // one piece at a time: the converted values stay few
                     __builtin_amdgcn_sched_barrier(0);
                 }
-            if (last) {
-                // x[tn] holds the last state: stage it as fp32 for the Gram.
-#pragma unroll
-                for (int k = 1; k <= kTB; ++k) {
-                    if (k != tn) continue;
-#pragma unroll
-                    for (int j = 0; j < kPPT; ++j) {
-                        const int q = tid + 256 * j;
-                        if (kPieces % 256 == 0 || q < kPieces) {
-                            float e[kCE];
-                            unpack_piece<T>(x[k][j], e);
-                            float* dst = sx + (q / kCPR) * D + (q % kCPR) * kCE;
-#pragma unroll
-                            for (int u = 0; u < kCE; u += 4)
-                                *reinterpret_cast<float4*>(dst + u) = make_float4(e[u], e[u + 1], e[u + 2], e[u + 3]);
-                        }
-                    }
-                }
-                __syncthreads();
-                if (gact) {
-                    for (int cell = 0; cell < kCellsPerStage; ++cell) {
-                        const float4 xi = *reinterpret_cast<const float4*>(sx + cell * D + bi * kBS);
-                        const float4 xj = *reinterpret_cast<const float4*>(sx + cell * D + bj * kBS);
-                        const double di[4] = {xi.x, xi.y, xi.z, xi.w};
-                        const double dj[4] = {xj.x, xj.y, xj.z, xj.w};
-#pragma unroll
-                        for (int i = 0; i < kBS; ++i)
-#pragma unroll
-                            for (int j = 0; j < kBS; ++j) g[i][j] = __builtin_fma(di[i], dj[j], g[i][j]);
-                    }
-                }
-                __syncthreads();
-            }
         }
-        // Block sums of this pass's states, in a fixed order (lanes, then waves).
+        // Workgroup sums per head in a fixed order (lanes, then waves).
+        const int h = (tid % R::kPPC) / R::kPPH;
+        const bool first = (lane & (R::kPPH - 1)) == 0 && lane / R::kPPH < R::kHW;
 #pragma unroll
         for (int k = 0; k < kTB; ++k) {
-            const double v[3] = {wave_sum_f64(s1[k]), wave_sum_f64(s2[k]), wave_sum_f64(pr[k])};
-            if (lane == 0) {
-                sred[wave][3 * k] = v[0];
-                sred[wave][3 * k + 1] = v[1];
-                sred[wave][3 * k + 2] = v[2];
+            const double v[3] = {head_sum<R>(s1[k]), head_sum<R>(s2[k]), head_sum<R>(pr[k])};
+            if (first) {
+#pragma unroll
+                for (int u = 0; u < 3; ++u) sred[(wave * kHeads + h) * kItems + 3 * k + u] = v[u];
             }
         }
         __syncthreads();
-        if (tid < 3 * tn) {
-            const double sum = sred[0][tid] + sred[1][tid] + sred[2][tid] + sred[3][tid];
-            mp[(long long)tb * 3 + tid] = (tb == 0 && tid == 2) ? 0.0 : sum;
+        for (int i = tid; i < kHeads * 3 * tn; i += 256) {
+            const int hh = i / (3 * tn), it = i - hh * (3 * tn);
+            double sum = 0.0;
+#pragma unroll
+            for (int w = 0; w < 4; ++w)
+                if (R::kHW == kHeads || (w * R::kHW) % kHeads == hh / R::kHW * R::kHW)
+                    sum += sred[(w * kHeads + hh) * kItems + it];
+            f.mom_part[((((long long)b * kHeads + hh) * f.mom_chunks + chunk) * f.T + tb) * 3 + it] =
+                tb == 0 && it == 2 ? 0.0 : sum;
         }
         __syncthreads();
     }
-    if (gact) {
-        double* gp = f.gram_part + ((long long)bh * f.chunks + chunk) * D * D;
+}
+
+typedef __attribute__((ext_vector_type(4))) double f64x4;
+
+// Gram partial of the last state over one chunk of one head. Lane (i = lane % 16, k = lane /
+// 16) reads channels NR i .. NR i + NR - 1 of cell k of a group of four; channel NR i + r is
+// row (and column) i of 16-wide block r, so that one register is an operand of either side
+// of v_mfma_f64_16x16x4 (row or column lane % 16, k = lane / 16; result value e of a lane:
+// row lane / 16 + 4 e, column lane % 16).
+template <typename T, int D>
+__device__ __forceinline__ void gram(const FitnessArgs& f, int bh, int chunk, double* sred) {
+    constexpr int NR = D >= 16 ? D / 16 : 1, kBlocks = NR * (NR + 1) / 2;
+    constexpr int kBytes = NR * (int)sizeof(T);  // per lane and cell: 2 to 16
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int i = lane & 15, kq = lane >> 4;
+    const long long cells = (long long)f.G * f.G, units = cells / kUnit;
+    const long long u0 = units * chunk / f.chunks, u1 = units * (chunk + 1) / f.chunks;
+    const int b = bh / kHeads, h = bh % kHeads;
+    constexpr int C = kHeads * D;
+    const bool on = D >= 16 || i < D;  // D = 8: half of the 16 rows
+    const T* src = history_state<T>(f, f.T - 1) + (long long)b * cells * C + (long long)(16 * wave + kq) * C + h * D +
+                   (on ? NR * i : 0);
+    struct Raw {
+        unsigned w[4][kBytes >= 4 ? kBytes / 4 : 1];  // four groups of four cells
+    };
+    auto load = [&](long long u, Raw& r) {
 #pragma unroll
-        for (int i = 0; i < kBS; ++i)
+        for (int g = 0; g < 4; ++g) {
+            const T* p = src + (u * kUnit + 4 * g) * C;
+            if constexpr (kBytes == 16) {
+                const uint4 v = *reinterpret_cast<const uint4*>(p);
+                r.w[g][0] = v.x, r.w[g][1] = v.y, r.w[g][2] = v.z, r.w[g][3] = v.w;
+            } else if constexpr (kBytes == 8) {
+                const uint2 v = *reinterpret_cast<const uint2*>(p);
+                r.w[g][0] = v.x, r.w[g][1] = v.y;
+            } else if constexpr (kBytes == 4) {
+                r.w[g][0] = *reinterpret_cast<const unsigned*>(p);
+            } else {
+                r.w[g][0] = *p;
+            }
+            if (!on) r.w[g][0] = 0u;
+        }
+    };
+    f64x4 acc[kBlocks];
 #pragma unroll
-            for (int j = 0; j < kBS; ++j) gp[(bi * kBS + i) * D + bj * kBS + j] = g[i][j];
+    for (int k = 0; k < kBlocks; ++k) acc[k] = f64x4{0.0, 0.0, 0.0, 0.0};
+    Raw cur, nxt;
+    if (u0 < u1) load(u0, cur);
+    for (long long u = u0; u < u1; ++u) {
+        load(u + 1 < u1 ? u + 1 : u, nxt);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            double x[NR];
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                if constexpr (sizeof(T) == 4) x[r] = __builtin_bit_cast(float, cur.w[g][r]);
+                else x[r] = r & 1 ? bf16hi(cur.w[g][r / 2]) : bf16lo(cur.w[g][r / 2]);
+            }
+            int k = 0;
+#pragma unroll
+            for (int r1 = 0; r1 < NR; ++r1)
+#pragma unroll
+                for (int r2 = r1; r2 < NR; ++r2, ++k)
+                    acc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[r1], x[r2], acc[k], 0, 0, 0);
+        }
+        cur = nxt;
     }
+    // Waves 1, 2, 3 added to wave 0 in turn, then the elements on and above the diagonal.
+    for (int w = 1; w < 4; ++w) {
+        if (wave == w) {
+#pragma unroll
+            for (int k = 0; k < kBlocks; ++k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sred[(4 * k + e) * 64 + lane] = acc[k][e];
+        }
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int k = 0; k < kBlocks; ++k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[k][e] += sred[(4 * k + e) * 64 + lane];
+        }
+        __syncthreads();
+    }
+    if (wave != 0) return;
+    double* gp = f.gram_part + ((long long)bh * f.chunks + chunk) * D * D;
+    int k = 0;
+#pragma unroll
+    for (int r1 = 0; r1 < NR; ++r1)
+#pragma unroll
+        for (int r2 = r1; r2 < NR; ++r2, ++k)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int ri = kq + 4 * e, c1 = NR * ri + r1, c2 = NR * i + r2;
+                if (D < 16 && (ri >= D || i >= D)) continue;
+                if (r1 != r2 || ri <= i) gp[c1 <= c2 ? c1 * D + c2 : c2 * D + c1] = acc[k][e];
+            }
+}
+
+template <typename T, int D, int kTB>
+__global__ __launch_bounds__(256, 2) void fitness_partial_kernel(FitnessArgs f) {
+    constexpr int NR = D >= 16 ? D / 16 : 1;
+    constexpr int kGramLds = NR * (NR + 1) / 2 * 4 * 64, kMomLds = 4 * kHeads * 3 * kTB;
+    __shared__ double sred[kGramLds > kMomLds ? kGramLds : kMomLds];
+    bool is_gram;
+    const long long n_g = (long long)f.B * kHeads * f.chunks, n_m = (long long)f.B * f.mom_chunks;
+    const long long idx = split_kinds(blockIdx.x, n_g, n_m, &is_gram);
+    if (idx < 0) return;
+    if (is_gram) gram<T, D>(f, (int)(idx / f.chunks), (int)(idx % f.chunks), sred);
+    else moments<T, D, kTB>(f, (int)(idx / f.mom_chunks), (int)(idx % f.mom_chunks), sred);
 }
 
 // Keeps the compiler from moving LDS accesses across this point. The block is one
@@ -279,6 +357,7 @@ __global__ __launch_bounds__(kFinThreads) void fitness_finalize_kernel(FitnessAr
     __shared__ __attribute__((aligned(16))) double2 cs[2][D];  // new a_i = c a_i + s a_partner
     __shared__ int flag[2];  // a step's: 0 no rotation, 1 rotations, 2 the solve has ended
     __shared__ double dg[D];  // the diagonal (wave 0 only)
+    __shared__ double msum[3 * 65];  // [state][S1, S2, P] over all chunks
     __shared__ double rho[64];
     __shared__ double sv[D], term[D];
 
@@ -302,6 +381,15 @@ __global__ __launch_bounds__(kFinThreads) void fitness_finalize_kernel(FitnessAr
             A[0][e] = f.scales ? s * gram_scale : s / ncell;
         }
         if (tid < 2) flag[tid] = 0;
+        // The moment sums: a wave per sum, its lanes striding over the chunks, then a
+        // fixed tree.
+        const double* mp = f.mom_part + (long long)bh * f.mom_chunks * f.T * 3;
+        for (int it = tid >> 6; it < 3 * f.T; it += kFinThreads / 64) {
+            double s = 0.0;
+            for (int c = lane; c < f.mom_chunks; c += 64) s += mp[(long long)c * f.T * 3 + it];
+            s = wave_sum_f64(s);
+            if (lane == 0) msum[it] = s;
+        }
     }
     __syncthreads();
 
@@ -425,19 +513,11 @@ __global__ __launch_bounds__(kFinThreads) void fitness_finalize_kernel(FitnessAr
     }
 
     // Coherence from the per-state sums: pair t = (t - 1, t) has sum a = S1(t-1),
-    // sum b = S1(t), sum ab = P(t), sum aa = S2(t-1), sum bb = S2(t); chunks in order.
+    // sum b = S1(t), sum ab = P(t), sum aa = S2(t-1), sum bb = S2(t).
     const int npair = f.T - 1;
     const double n = ncell * D;
     for (int t = lane + 1; t < f.T; t += 64) {
-        double mo[5] = {0, 0, 0, 0, 0};
-        for (int ch = 0; ch < f.chunks; ++ch) {
-            const double* qm = f.mom_part + ((long long)bh * f.chunks + ch) * f.T * 3;
-            mo[0] += qm[(t - 1) * 3];
-            mo[1] += qm[t * 3];
-            mo[2] += qm[t * 3 + 2];
-            mo[3] += qm[(t - 1) * 3 + 1];
-            mo[4] += qm[t * 3 + 1];
-        }
+        double mo[5] = {msum[(t - 1) * 3], msum[t * 3], msum[t * 3 + 2], msum[(t - 1) * 3 + 1], msum[t * 3 + 1]};
         if (f.scales) {
             const double sa = scale_of(t - 1), sb = scale_of(t);
             mo[0] *= sa;
@@ -492,7 +572,15 @@ __global__ __launch_bounds__(kFinThreads) void fitness_finalize_kernel(FitnessAr
 
 template <typename T, int D>
 hipError_t launch_td(const FitnessArgs& f, hipStream_t s) {
-    hipLaunchKernelGGL((fitness_partial_kernel<T, D>), dim3(f.B * kHeads, f.chunks), dim3(256), 0, s, f);
+    const long long n_g = (long long)f.B * kHeads * f.chunks, n_m = (long long)f.B * f.mom_chunks;
+    const dim3 grid((unsigned)(8 * ((n_g + 7) / 8 + (n_m + 7) / 8)));
+    // States per pass: a short history needs no registers for eight.
+    if (f.T <= 2)
+        hipLaunchKernelGGL((fitness_partial_kernel<T, D, 2>), grid, dim3(256), 0, s, f);
+    else if (f.T <= 4)
+        hipLaunchKernelGGL((fitness_partial_kernel<T, D, 4>), grid, dim3(256), 0, s, f);
+    else
+        hipLaunchKernelGGL((fitness_partial_kernel<T, D, 8>), grid, dim3(256), 0, s, f);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(fitness_finalize_kernel<D>, dim3(f.B * kHeads), dim3(kFinThreads), 0, s, f);
@@ -512,26 +600,33 @@ hipError_t launch_t(const FitnessArgs& f, hipStream_t s) {
 
 }  // namespace
 
-int fitness_chunks(int G) {
-    const long long stages = (long long)G * G / kCellsPerStage;
-    int c = 16;
-    while (c > 1 && (stages % c) != 0) --c;
-    return stages >= 1 ? c : 0;
+FitnessChunks fitness_chunks(int B, int G) {
+    const long long units = (long long)G * G / kUnit;
+    auto clamp = [&](long long v, long long lo, long long hi) { return v < lo ? lo : v > hi ? hi : v; };
+    FitnessChunks c;
+    // Gram: about four workgroups per CU, not more partials than the finalize reads in a few
+    // microseconds. Moments: about eight per CU. Neither splits below 64 cells.
+    c.gram = (int)std::min(units, clamp(1024 / (B * kHeads), 4, 32));
+    c.mom = (int)std::min(units, clamp(2048 / B, 1, 512));
+    return c;
 }
 
 hipError_t launch_fitness(int dtype, const FitnessArgs& f, hipStream_t s) {
     return dtype == 1 ? launch_t<bf16_t>(f, s) : launch_t<float>(f, s);
 }
 
-size_t fitness_partial_bytes(int B, int D, int T, int chunks) {
-    return (size_t)B * kHeads * chunks * ((size_t)D * D + 3 * (size_t)T) * sizeof(double);
+size_t fitness_partial_bytes(int B, int D, int T, FitnessChunks c) {
+    return (size_t)B * kHeads * ((size_t)c.gram * D * D + (size_t)c.mom * 3 * T) * sizeof(double);
 }
 
-int fitness_static_chunks(int B, int G, int D, int T) {
-    const long long stages = (long long)G * G / kCellsPerStage;
-    for (int c = fitness_chunks(G); c >= 1; --c)
-        if (stages % c == 0 && fitness_partial_bytes(B, D, T, c) <= kFitnessScratchBytes) return c;
-    return 0;
+FitnessChunks fitness_static_chunks(int B, int G, int D, int T) {
+    FitnessChunks c = fitness_chunks(B, G);
+    while (fitness_partial_bytes(B, D, T, c) > kFitnessScratchBytes) {
+        if (c.gram == 1 && c.mom == 1) return FitnessChunks{0, 0};
+        c.gram = (c.gram + 1) / 2;
+        c.mom = (c.mom + 1) / 2;
+    }
+    return c;
 }
 
 namespace {

@@ -129,9 +129,9 @@ struct FitnessArgs {
     const void* hist;   // state 0 of the history, each state [B][G][G][C]
     long long t_stride; // bytes from state t to state t + 1 (may be negative)
     int T, B, G, D;
-    double* gram_part;  // [B*H][chunks][D*D]
-    double* mom_part;   // [B*H][chunks][T][3]: sum x_t, sum x_t^2, sum x_{t-1} x_t
-    int chunks;
+    double* gram_part;  // [B*H][chunks][D*D], on and above the diagonal
+    double* mom_part;   // [B*H][mom_chunks][T][3]: sum x_t, sum x_t^2, sum x_{t-1} x_t
+    int chunks, mom_chunks;
     float* erank;       // [B][H]
     float* coh;
     float* fitness;
@@ -140,18 +140,22 @@ struct FitnessArgs {
     // values per (b, h); the moments and the last state's Gram are scaled in fp64.
     const double* scales;
 };
-int fitness_chunks(int G);
+// How many parts the cells of a batch entry are split into for the two kinds of partial
+// sums.
+struct FitnessChunks {
+    int gram, mom;
+};
+FitnessChunks fitness_chunks(int B, int G);
 hipError_t launch_fitness(int dtype, const FitnessArgs& a, hipStream_t s);
 // Allocation-free fitness (slime_ca_fitness_static): the partial sums live in a
-// static device buffer of kFitnessScratchBytes per GPU. fitness_static_chunks: the
-// largest chunk count <= fitness_chunks(G) that divides the grid's 64-cell stages
-// and whose [B*H][chunks] Gram and moment partials fit in that buffer (0: none
-// fits). fitness_static_scratch: the buffer's device address on the current device
+// static device buffer of kFitnessScratchBytes per GPU. fitness_static_chunks:
+// fitness_chunks, halved until the partials fit in that buffer (0: not even one part
+// does). fitness_static_scratch: the buffer's device address on the current device
 // (hipErrorNoBinaryForGpu unless it is a gfx950), looked up on the device's first
 // call and cached.
 constexpr size_t kFitnessScratchBytes = size_t(32) << 20;
-size_t fitness_partial_bytes(int B, int D, int T, int chunks);
-int fitness_static_chunks(int B, int G, int D, int T);
+size_t fitness_partial_bytes(int B, int D, int T, FitnessChunks c);
+FitnessChunks fitness_static_chunks(int B, int G, int D, int T);
 hipError_t fitness_static_scratch(void** ptr);
 // launch_fitness on the static scratch (f.gram_part and f.mom_part are set here).
 // Outside graph capture, a call on another stream than the previous call's waits for
