@@ -828,7 +828,7 @@ int slime_ca_backward(slime_ca* h, const void* x_in, const void* target, float* 
     const int lchunks = loss_fused ? h->tiles : backward_loss_chunks(c.G);
     const int nW = 1024;  // cell-pass workgroups per pod
     const long long rows_pod = (long long)(c.B / c.pods) * c.G * c.G;
-    const int dw_chunks = backward_dw_chunks_per_pod(c.dtype, (int)C, rows_pod);
+    const DwPlan dw = backward_dw_plan(c.dtype, (int)C, c.pods, rows_pod);
     const bool want_w = grads && (grads->WP || grads->WI || grads->WV);
     // work buffers, allocated on first use
     if (!h->Wcat) {
@@ -862,7 +862,7 @@ int slime_ca_backward(slime_ca* h, const void* x_in, const void* target, float* 
         rc = rc ? rc : dalloc_t(&h->bw_ppart, (size_t)c.pods * c.H * nW * backward_part_floats() * 4);
     if (c.growth_per_cell && !h->bw_gcell) rc = rc ? rc : dalloc_t(&h->bw_gcell, cells * c.H * 2 * 4);
     if (want_w && !h->bw_dwpart)
-        rc = rc ? rc : dalloc_t(&h->bw_dwpart, (size_t)c.pods * dw_chunks * C * 3 * C * 4);
+        rc = rc ? rc : dalloc_t(&h->bw_dwpart, (size_t)c.pods * dw.chunks_per_pod * C * 3 * C * 4);
     if (!h->Sf && !h->bw_y32) rc = rc ? rc : dalloc_t(&h->bw_y32, n * 4);
     if (rc) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -941,9 +941,10 @@ int slime_ca_backward(slime_ca* h, const void* x_in, const void* target, float* 
         d.part = h->bw_dwpart;
         d.C = (int)C;
         d.pods = c.pods;
-        d.chunks_per_pod = dw_chunks;
+        d.chunks_per_pod = dw.chunks_per_pod;
         d.rows_per_pod = rows_pod;
-        d.rows_per_chunk = backward_dw_rows_per_chunk(c.dtype, (int)C, rows_pod);
+        d.rows_per_chunk = dw.rows_per_chunk;
+        d.tile = dw.tile;
         d.gWP = grads->WP;
         d.gWI = grads->WI;
         d.gWV = grads->WV;

@@ -25,6 +25,8 @@
 // over those lanes with DPP moves inside a 16-lane row.
 // Parameter partial sums are kept per workgroup, each workgroup owning one
 // (pod, head), and added in a fixed order by the finalize kernels.
+#include <cmath>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -999,46 +1001,9 @@ __global__ __launch_bounds__(256) void bw_cell_param_finalize_kernel(BackwardArg
 }
 
 // ---- weight gradients gW_p[pod][k][j] = sum over the pod's rows of X[r][k] G_p[r][j] ----------
-// Block (k tile, j tile, chunk): a 64 x 64 output tile over kWRows rows, 4 x 4
-// per thread, operands staged through LDS 16 rows at a time; chunks are added in
-// order by bw_dw_reduce_kernel.
-constexpr int kWRows = 4096;
-
-template <typename T>
-__global__ __launch_bounds__(256) void bw_dw_partial_kernel(BackwardArgs a, DwArgs d) {
-    const int C = d.C, N3 = 3 * C;
-    const int kt = blockIdx.x, jt = blockIdx.y, chunk = blockIdx.z;
-    const long long rows = d.rows_per_pod;
-    const int pod = chunk / d.chunks_per_pod;
-    const long long r0 = (long long)pod * rows + (long long)(chunk % d.chunks_per_pod) * d.rows_per_chunk;
-    const long long r1 = min(r0 + d.rows_per_chunk, (long long)(pod + 1) * rows);
-    __shared__ float sx[16][64], sg[16][64];
-    const int tk = (threadIdx.x / 16) * 4, tj = (threadIdx.x % 16) * 4;
-    float acc[4][4] = {};
-    for (long long rb = r0; rb < r1; rb += 16) {
-        for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-            const int rr = e / 64, cc = e % 64;
-            const long long r = rb + rr;
-            sx[rr][cc] = r < r1 ? ld<T>(a.X, r * C + kt * 64 + cc) : 0.f;
-            sg[rr][cc] = r < r1 ? ld<T>(a.G3, r * N3 + jt * 64 + cc) : 0.f;
-        }
-        __syncthreads();
-#pragma unroll 4
-        for (int rr = 0; rr < 16; ++rr)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(sx[rr][tk + i], sg[rr][tj + j], acc[i][j]);
-        __syncthreads();
-    }
-    float* out = d.part + (long long)chunk * C * N3;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) out[(long long)(kt * 64 + tk + i) * N3 + jt * 64 + tj + j] = acc[i][j];
-}
-
-// bf16: the same partial sums on the matrix cores. Block (k tile, j tile, chunk):
+// Split over row chunks, added in order by bw_dw_reduce_kernel; the tile and the chunk
+// length are chosen by backward_dw_plan.
+// bf16 with C a multiple of 128. Block (k tile, j tile, chunk):
 // a 128 x 128 output tile over rows_per_chunk rows in steps of 32, wave (wk, wj)
 // owning 64 x 64 as 4 x 4 v_mfma_f32_16x16x32_bf16 blocks. Both operands are
 // column slices of row-major tiles -- out[k][j] = sum_r X[r][k] G[r][j] -- staged
@@ -1051,7 +1016,6 @@ __global__ __launch_bounds__(256) void bw_dw_partial_kernel(BackwardArgs a, DwAr
 // disjoint banks, and so do the groups, whose rows are 8 apart.
 constexpr int kDwT = 128, kDwStep = 32, kDwRowB = 2 * kDwT, kDwStages = 4;
 constexpr int kDwStageB = 2 * kDwStep * kDwRowB;  // X and G tiles, 16 KiB
-constexpr long long kDwRowsMfma = 16384;
 
 typedef short dw_v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) dw_v4i16 dw_lds_v4i16;
@@ -1285,6 +1249,70 @@ __global__ __launch_bounds__(256) void bw_dw_mfma2_kernel(BackwardArgs a, DwArgs
             }
 }
 
+// fp32, and bf16 with C = 64: 64 x 64 output tiles, wave (wk, wj) owning one 32 x 32 block
+// of v_mfma_f32_32x32x2_f32, whose operands are 32 consecutive columns of two rows: plain
+// reads of the row-major [rows][64 columns] stages, without bank conflicts (bf16 values are
+// widened as they are read: products and sums stay fp32). Slabs of 4 KiB per operand (16
+// fp32 or 32 bf16 rows) through a 4-stage ring, several workgroups per CU. Bound by the
+// fp32 matrix rate. Measured (2 x 64^2 cells, C = 256, fp32): 550 us as scalar
+// FMAs in 96 workgroups -> 33 us in 768 (99 TFLOP/s)
+constexpr int kDw64SlabB = 4096, kDw64StageB = 2 * kDw64SlabB, kDw64Stages = 4;
+
+template <typename T>
+__global__ __launch_bounds__(256) void bw_dw64_kernel(BackwardArgs a, DwArgs d) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[kDw64Stages * kDw64StageB];
+    constexpr int kRowB = 64 * (int)sizeof(T), kRows = kDw64SlabB / kRowB, kCPR = kRowB / 16, kRPI = 64 / kCPR;
+    const int C = d.C, N3 = 3 * C;
+    const int kt = blockIdx.x, jt = blockIdx.y, chunk = blockIdx.z;
+    const int pod = chunk / d.chunks_per_pod;
+    const long long r0 = (long long)pod * d.rows_per_pod + (long long)(chunk % d.chunks_per_pod) * d.rows_per_chunk;
+    const long long r1 = min(r0 + d.rows_per_chunk, (long long)(pod + 1) * d.rows_per_pod);
+    const int nsteps = (int)((r1 - r0) / kRows);  // rows are a multiple of 32 (backward_dw_plan)
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave & 1, wj = wave >> 1;
+    // Direct load: wave w fills rows kRPI w .. of each operand's slab, lane l row l / kCPR of
+    // those, 16-byte piece l % kCPR.
+    const char* Xs = reinterpret_cast<const char*>(static_cast<const T*>(a.X) + (r0 + kRPI * wave) * C + kt * 64);
+    const char* Gs = reinterpret_cast<const char*>(static_cast<const T*>(a.G3) + (r0 + kRPI * wave) * N3 + jt * 64);
+    const unsigned xoff = (unsigned)(lane / kCPR * C * (int)sizeof(T) + lane % kCPR * 16);
+    const unsigned goff = (unsigned)(lane / kCPR * N3 * (int)sizeof(T) + lane % kCPR * 16);
+    auto issue = [&](int st, int stage) {  // past the end: the last slab again
+        const long long rb = (long long)(st < nsteps ? st : nsteps - 1) * kRows;
+        const unsigned sb = lds_addr(lds + stage * kDw64StageB) + wave * 1024;
+        dma16_lds(Xs + rb * C * (int)sizeof(T), xoff, sb);
+        dma16_lds(Gs + rb * N3 * (int)sizeof(T), goff, sb + kDw64SlabB);
+    };
+    f32x16 acc = {};
+    if (nsteps > 0) {
+#pragma unroll
+        for (int st = 0; st < kDw64Stages - 1; ++st) issue(st, st);
+    }
+    const unsigned at = (unsigned)((lane >> 5) * kRowB + (lane & 31) * (int)sizeof(T));
+    const unsigned xa = at + wk * 32 * (unsigned)sizeof(T), ga = at + wj * 32 * (unsigned)sizeof(T) + kDw64SlabB;
+    for (int st = 0; st < nsteps; ++st) {
+        dw_wait<2 * (kDw64Stages - 2)>();  // this wave's loads of slab st have landed
+        dw_barrier();                      // ... and every wave's; slab st - 1's stage is free
+        issue(st + kDw64Stages - 1, (st + kDw64Stages - 1) % kDw64Stages);
+        const unsigned char* base = lds + (st % kDw64Stages) * kDw64StageB;
+        float x[kRows / 2], g[kRows / 2];
+#pragma unroll
+        for (int k = 0; k < kRows / 2; ++k) {
+            x[k] = Store<T>::to_f32(*reinterpret_cast<const T*>(base + xa + 2 * k * kRowB));
+            g[k] = Store<T>::to_f32(*reinterpret_cast<const T*>(base + ga + 2 * k * kRowB));
+        }
+#pragma unroll
+        for (int k = 0; k < kRows / 2; ++k) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[k], g[k], acc, 0, 0, 0);
+    }
+    dw_wait<0>();  // refetched slabs may still be landing in LDS
+    float* out = d.part + (long long)chunk * C * N3;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int k = kt * 64 + wk * 32 + 8 * (e / 4) + 4 * (lane >> 5) + e % 4;
+        out[(long long)k * N3 + jt * 64 + wj * 32 + (lane & 31)] = acc[e];
+    }
+}
+
 __global__ __launch_bounds__(256) void bw_dw_reduce_kernel(DwArgs d) {
     const int C = d.C, N3 = 3 * C;
     const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;  // (pod, k, j)
@@ -1292,6 +1320,7 @@ __global__ __launch_bounds__(256) void bw_dw_reduce_kernel(DwArgs d) {
     const int pod = (int)(idx / ((long long)C * N3));
     const long long kj = idx % ((long long)C * N3);
     float sum = 0.f;
+#pragma unroll 8
     for (int c = 0; c < d.chunks_per_pod; ++c)
         sum += d.part[((long long)(pod * d.chunks_per_pod + c)) * C * N3 + kj];
     const int k = (int)(kj / N3), j = (int)(kj % N3), p = j / C;
@@ -1337,16 +1366,32 @@ hipError_t launch_t(const BackwardArgs& a, hipStream_t s) {
 
 int backward_loss_chunks(int G) { return (G * G + kLossCells - 1) / kLossCells; }
 int backward_part_floats() { return kPartF; }
-static bool dw_mfma(int dtype, int C, long long rows_per_pod) {
-    return dtype == 1 && C % kDwT == 0 && rows_per_pod % kDwStep == 0;
-}
-long long backward_dw_rows_per_chunk(int dtype, int C, long long rows_per_pod) {
-    if (!dw_mfma(dtype, C, rows_per_pod)) return kWRows;
-    return rows_per_pod < kDwRowsMfma ? rows_per_pod : kDwRowsMfma;  // a multiple of kDwStep
-}
-int backward_dw_chunks_per_pod(int dtype, int C, long long rows_per_pod) {
-    const long long r = backward_dw_rows_per_chunk(dtype, C, rows_per_pod);
-    return (int)((rows_per_pod + r - 1) / r);
+
+// Tiles of 256 or 128 (bf16, bw_dw_mfma2_kernel and bw_dw_mfma_kernel) or 64 (bw_dw64_kernel),
+// and the rows a chunk sums, by the least time of: rounds of workgroups over 256 CUs at the
+// rate one tile reaches (3.9, 2.7 and 0.5 TFLOP/s per CU), plus the chunks' partials written
+// and read once at 4.8 TB/s. One chunk keeps at most 16,384 rows (4096 in 64-wide tiles), so
+// that its fp32 sums stay short, and at least 128. A large product keeps its few long
+// chunks (1,048,576 rows, C = 512: 64 chunks of 768 tiles); one grid of 16,384 rows had 12
+// workgroups.
+DwPlan backward_dw_plan(int dtype, int C, int pods, long long rows_per_pod) {
+    DwPlan best{0, 0, 0};
+    double best_t = 0.0;
+    for (int tile : {256, 128, 64}) {
+        if (C % tile != 0 || (tile == 64) != (dtype != 1 || C % 128 != 0)) continue;
+        const double rate = tile == 256 ? 3.9e12 : tile == 128 ? 2.7e12 : 0.5e12;
+        const long long most = tile == 64 ? 4096 : 16384;
+        const double tiles = (double)(C / tile) * (3 * C / tile) * pods;
+        for (long long n = (rows_per_pod + most - 1) / most;; n *= 2) {
+            const long long rows = ((rows_per_pod + n - 1) / n + 31) / 32 * 32;
+            const long long chunks = (rows_per_pod + rows - 1) / rows;
+            const double rounds = std::ceil(tiles * chunks / 256.0);
+            const double t = rounds * rows * tile * tile * 2.0 / rate + (double)chunks * pods * C * 3 * C * 8.0 / 4.8e12;
+            if (!best.tile || t < best_t) best = DwPlan{tile, rows, (int)chunks}, best_t = t;
+            if (rows <= 128) break;
+        }
+    }
+    return best;
 }
 
 hipError_t launch_backward_stencil(int dtype, const BackwardArgs& a, hipStream_t s) {
@@ -1354,17 +1399,15 @@ hipError_t launch_backward_stencil(int dtype, const BackwardArgs& a, hipStream_t
 }
 
 hipError_t launch_backward_dw(int dtype, const BackwardArgs& a, const DwArgs& d, hipStream_t s) {
-    const dim3 grid(d.C / 64, 3 * d.C / 64, d.pods * d.chunks_per_pod);
-    if (dw_mfma(dtype, d.C, d.rows_per_pod) && d.C % kDw2T == 0)
-        hipLaunchKernelGGL(bw_dw_mfma2_kernel, dim3(d.C / kDw2T, 3 * d.C / kDw2T, d.pods * d.chunks_per_pod),
-                           dim3(256), 0, s, a, d);
-    else if (dw_mfma(dtype, d.C, d.rows_per_pod))
-        hipLaunchKernelGGL(bw_dw_mfma_kernel, dim3(d.C / kDwT, 3 * d.C / kDwT, d.pods * d.chunks_per_pod),
-                           dim3(256), 0, s, a, d);
+    const dim3 grid(d.C / d.tile, 3 * d.C / d.tile, d.pods * d.chunks_per_pod);
+    if (d.tile == 256)
+        hipLaunchKernelGGL(bw_dw_mfma2_kernel, grid, dim3(256), 0, s, a, d);
+    else if (d.tile == 128)
+        hipLaunchKernelGGL(bw_dw_mfma_kernel, grid, dim3(256), 0, s, a, d);
     else if (dtype == 1)
-        hipLaunchKernelGGL((bw_dw_partial_kernel<bf16_t>), grid, dim3(256), 0, s, a, d);
+        hipLaunchKernelGGL((bw_dw64_kernel<bf16_t>), grid, dim3(256), 0, s, a, d);
     else
-        hipLaunchKernelGGL((bw_dw_partial_kernel<float>), grid, dim3(256), 0, s, a, d);
+        hipLaunchKernelGGL((bw_dw64_kernel<float>), grid, dim3(256), 0, s, a, d);
     const long long n = (long long)d.pods * d.C * 3 * d.C;
     hipLaunchKernelGGL(bw_dw_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d);
     return hipGetLastError();
