@@ -13,13 +13,11 @@
 // The toroidal halo tile follows slime/kernels/triton_impl.cu:90-105.
 //
 // One workgroup owns a 4x8 cell tile of one batch and walks the 8 heads. Per
-// head it stages the 6x10 halo of X_h and V_h (fp32, X already multiplied by
-// the deferred mass scale), I_h and the centre P_h (storage type, rows padded by
-// 16 B) in LDS; computes the 32x9 attention weights; then each thread sweeps a
-// run of 4 cells of one tile row for two adjacent channels with a 3x3 register
-// window (each halo value is read from LDS 3 times per run, not 9 per cell) and
-// accumulates its share of all eight mixed outputs Y_o in registers (64 per
-// thread, which keeps the kernel at 2+ waves per SIMD without spills). After the last head the outputs are rounded to
+// head it stages the 6x10 halo of X_h, V_h and I_h and the centre P_h in LDS (storage
+// type, by direct global->LDS loads); computes the 32x9 attention weights; then each
+// thread takes two neighbouring cells of one tile row for two adjacent channels and
+// accumulates its share of all eight mixed outputs Y_o in registers (32 per thread).
+// After the last head the outputs are rounded to
 // the storage type, written once, and the tile's per-head sums of the scaled
 // input and of the stored output go to global partial buffers (wave64 DPP
 // reductions, then a cross-wave pass through LDS).
@@ -39,7 +37,7 @@ constexpr int kHaloX = kTileX + 2;     // halo rows are 10 cells wide, 6 rows ta
 constexpr int kHaloCells = (kTileY + 2) * kHaloX;  // 60
 constexpr int kHaloPad = 64;           // halo cells reserved per array
 constexpr int kTileCells = kTileY * kTileX;        // 32
-constexpr int kRun = 4;                // cells per thread along x in phase B
+constexpr int kRun = 2;                // cells per thread along x in phase B
 constexpr int kAStride = 12;           // floats per cell in the attention buffer
 
 __device__ __forceinline__ int wrapi(int v, int G) { return v < 0 ? v + G : (v >= G ? v - G : v); }
@@ -60,21 +58,25 @@ struct Layout {
     static constexpr int kCPR = D / kCE;                     // chunks per (cell, head) row
     static constexpr int kRowB = D * (int)sizeof(T);         // bytes per (cell, head) row
     static constexpr int kSwz = (kCPR < 8 ? kCPR : 8) - 1;   // chunk XOR mask (I and P rows)
-    static constexpr int kThreads = (4 * D) < 64 ? 64 : 4 * D;
-    static constexpr int kActive = 4 * D;                    // threads with a phase-B task
+    static constexpr int kThreads = kTileCells / kRun * (D / 2);  // one phase-B task each
     static constexpr int kWaves = kThreads / 64;
-    static constexpr int kTPC = kThreads / kTileCells;       // phase-A threads per cell
+    static constexpr int kTPC = D / 8 < 2 ? 2 : D / 8;       // phase-A threads per cell
+    static_assert(kThreads % 64 == 0 && kTileCells * kTPC <= kThreads, "whole waves, phase A fits");
     // Direct global->LDS staging: one wave instruction fills 1 KiB = kCPI rows.
     static constexpr int kCPI = 64 / kCPR;                   // cells per DMA instruction
     static constexpr int kPCells = kCPI > kTileCells ? kCPI : kTileCells;  // P rows (padded)
     static constexpr int kHG = kHaloPad / kCPI;              // instruction groups per halo array
     static constexpr int kPG = kPCells / kCPI;               // instruction groups of the P tile
     static constexpr int kIA = kHG / kWaves;                 // per wave, per halo array
-    static constexpr int kPA = kPG / kWaves;                 // per wave, P tile
-    static_assert(kHG % kWaves == 0 && kPG % kWaves == 0, "DMA groups must split over waves");
+    static_assert(kHG % kWaves == 0 && kPG <= kWaves, "DMA groups must split over waves");
+    static constexpr int kLoads = 3 * kIA + 1;               // per wave and head (wave w >= kPG
+                                                             // repeats P group w % kPG)
     static constexpr int kBufB = (3 * kHaloPad + kPCells) * kRowB;
     static constexpr int offX = 0, offV = kHaloPad * kRowB, offI = 2 * kHaloPad * kRowB,
                          offP = 3 * kHaloPad * kRowB;
+    // Staging buffers: see stencil_kernel.
+    static constexpr int kFull = sizeof(T) == 2 ? 2 : 1;
+    static constexpr int kDeep = 150 * 1024 / kBufB < kHeads ? 150 * 1024 / kBufB : kHeads;
 };
 
 // Direct global->LDS loads: dma16_lds, dma16_lds_nt, wait_vm0 (common.hpp); the kernel
@@ -172,21 +174,64 @@ __device__ __forceinline__ float group_max(float v) {
     return v;
 }
 
+// One step of a butterfly sum of kN*2 per-lane values: lanes whose bit `bit` is
+// set keep the upper half, the others the lower half, each adding the partner
+// lane's copy (DPP kCtrl, whose partner differs from the lane in that bit and in
+// no bit a previous step used).
+template <int kN, int kCtrl>
+__device__ __forceinline__ void fold_half(double (&v)[16], int lane, int bit) {
+    const bool up = (lane >> bit) & 1;
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+        const double keep = up ? v[i + kN] : v[i];
+        const double send = up ? v[i] : v[i + kN];
+        v[i] = keep + dpp_f64<kCtrl>(send);
+    }
+}
+
+// Waits until at most `heads` heads' loads of this wave are in flight.
+template <int kLoads>
+__device__ __forceinline__ void wait_heads(int heads) {
+#define SLIME_WAIT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | ((((n) >> 4) & 3) << 14) | 0x0F70)
+    static_assert(6 * kLoads < 64, "vmcnt has 6 bits");
+    switch (heads) {
+        case 6: SLIME_WAIT(6 * kLoads); break;
+        case 5: SLIME_WAIT(5 * kLoads); break;
+        case 4: SLIME_WAIT(4 * kLoads); break;
+        case 3: SLIME_WAIT(3 * kLoads); break;
+        case 2: SLIME_WAIT(2 * kLoads); break;
+        case 1: SLIME_WAIT(kLoads); break;
+        default: SLIME_WAIT(0); break;
+    }
+#undef SLIME_WAIT
+}
+
 // TY: storage type of the unscaled output; fp32 when the caller rescales it into
 // the final bf16 state (one rounding instead of two).
-template <typename T, int D, typename TY>
-__global__ __launch_bounds__((Layout<T, D>::kThreads), 2) void stencil_kernel(StencilArgs a) {
+//
+// kBufs: how a head's data meets its compute. 1: one buffer in two halves -- I and P of
+// the next head load during phase B, which no longer reads them, X and V during phase A --
+// so that two workgroups of a CU (57 KiB each for fp32, D = 64) cover each other. 2 or
+// more: a ring, the loads of the next kBufs - 1 heads in flight; eight buffers hold the
+// whole tile, so that a grid with no second workgroup to overlap pays one memory round
+// trip instead of eight. launch_tdy picks.
+//
+// What bounds it: VALU and LDS issue with four waves per SIMD (two cells per thread keep
+// the output accumulators at 32 and the kernel at 128 registers).
+// Measured: 1 x 128^2 x 512 fp32 57 -> 37 us (4.6 TB/s of the five planes; one workgroup of 4
+// waves per CU and four cells per thread before), 8 x 104^2 x 256 bf16 85 -> 76 us,
+// 1 x 32^2 x 64 fp32 (32 tiles, eight buffers) 17 -> 14 us.
+template <typename T, int D, typename TY, int kBufs>
+__global__ __launch_bounds__((Layout<T, D>::kThreads), (kBufs == Layout<T, D>::kFull ? 4 : 2))
+void stencil_kernel(StencilArgs a) {
     using L = Layout<T, D>;
     constexpr int H = kHeads;
     constexpr int C = H * D;
     constexpr int kPairs = D / 2;
-    // Two staging buffers as separate LDS objects: the compiler can then tell that
-    // reading one does not depend on the direct loads landing in the other.
-    __shared__ __attribute__((aligned(16))) unsigned char bufA[L::kBufB];
-    __shared__ __attribute__((aligned(16))) unsigned char bufB[L::kBufB];
-    __shared__ __attribute__((aligned(16))) float sAtt[2][kTileCells * kAStride];
+    __shared__ __attribute__((aligned(1024))) unsigned char stage[kBufs * L::kBufB];
+    __shared__ __attribute__((aligned(16))) float sA[kTileCells * kAStride];
     __shared__ __attribute__((aligned(16))) float sMS[H * kTileCells * 2];
-    __shared__ double sR[L::kWaves * 16];
+    __shared__ double sR[L::kThreads];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -208,8 +253,9 @@ __global__ __launch_bounds__((Layout<T, D>::kThreads), 2) void stencil_kernel(St
     // g*kCPI + l/kCPR, physical chunk l%kCPR. X and V rows are stored linearly; I
     // and P rows are XOR-swizzled by cell (the score phase reads whole rows of
     // neighbouring cells), so those lanes fetch logical chunk (l%kCPR) ^ (cell&kSwz).
-    // Wave w issues groups g = w + k*kWaves. Per-lane element offsets, head 0:
-    int hoff_lin[L::kIA], hoff_swz[L::kIA], poff[L::kPA];
+    // Wave w issues groups g = w + k*kWaves. Per-lane byte offsets in the batch entry, head 0:
+    unsigned boff_lin[L::kIA], boff_swz[L::kIA], boff_p;
+    const int pgrp = wave % L::kPG;
     {
         const int ch = lane % L::kCPR;
 #pragma unroll
@@ -217,49 +263,41 @@ __global__ __launch_bounds__((Layout<T, D>::kThreads), 2) void stencil_kernel(St
             const int cell = (wave + k * L::kWaves) * L::kCPI + lane / L::kCPR;
             const int gc = cell < kHaloCells ? cell : kHaloCells - 1;  // padding rows
             const int gy = wrapi(ty0 + gc / kHaloX - 1, G), gx = wrapi(tx0 + gc % kHaloX - 1, G);
-            const int base = (gy * G + gx) * C;
-            hoff_lin[k] = base + ch * L::kCE;
-            hoff_swz[k] = base + (ch ^ (cell & L::kSwz)) * L::kCE;
+            const unsigned base = (unsigned)((gy * G + gx) * C);
+            boff_lin[k] = (base + ch * L::kCE) * (unsigned)sizeof(T);
+            boff_swz[k] = (base + (ch ^ (cell & L::kSwz)) * L::kCE) * (unsigned)sizeof(T);
         }
-#pragma unroll
-        for (int k = 0; k < L::kPA; ++k) {
-            const int cell = (wave + k * L::kWaves) * L::kCPI + lane / L::kCPR;
-            const int gc = cell < kTileCells ? cell : kTileCells - 1;  // padding rows
-            poff[k] = ((ty0 + gc / kTileX) * G + tx0 + gc % kTileX) * C +
-                      (ch ^ (cell & L::kSwz)) * L::kCE;
-        }
+        const int cell = pgrp * L::kCPI + lane / L::kCPR;
+        const int gc = cell < kTileCells ? cell : kTileCells - 1;  // padding rows
+        boff_p = (unsigned)(((ty0 + gc / kTileX) * G + tx0 + gc % kTileX) * C + (ch ^ (cell & L::kSwz)) * L::kCE) *
+                 (unsigned)sizeof(T);
     }
     const char* srcX = reinterpret_cast<const char*>(static_cast<const T*>(a.X) + bbase);
     const char* srcV = reinterpret_cast<const char*>(static_cast<const T*>(a.V) + bbase);
     const char* srcI = reinterpret_cast<const char*>(static_cast<const T*>(a.I) + bbase);
     const char* srcP = reinterpret_cast<const char*>(static_cast<const T*>(a.P) + bbase);
-    // Byte offsets (within the batch entry) of this lane's 16-byte pieces.
-    unsigned boff_lin[L::kIA], boff_swz[L::kIA], boff_p[L::kPA];
+    auto issue_pi = [&](int h, int slot) {
+        const unsigned hb = (unsigned)(h * D * (int)sizeof(T)), sb = lds_addr(stage) + slot * L::kBufB;
 #pragma unroll
-    for (int k = 0; k < L::kIA; ++k) {
-        boff_lin[k] = (unsigned)hoff_lin[k] * (unsigned)sizeof(T);
-        boff_swz[k] = (unsigned)hoff_swz[k] * (unsigned)sizeof(T);
-    }
-#pragma unroll
-    for (int k = 0; k < L::kPA; ++k) boff_p[k] = (unsigned)poff[k] * (unsigned)sizeof(T);
-    auto issue_head = [&](int h, unsigned char* buf) {
-        const unsigned hb = (unsigned)(h * D * (int)sizeof(T));
+        for (int k = 0; k < L::kIA; ++k)
+            dma16_lds(srcI, boff_swz[k] + hb, sb + L::offI + (wave + k * L::kWaves) * 1024);
+        dma16_lds(srcP, boff_p + hb, sb + L::offP + pgrp * 1024);
+    };
+    auto issue_xv = [&](int h, int slot) {
+        const unsigned hb = (unsigned)(h * D * (int)sizeof(T)), sb = lds_addr(stage) + slot * L::kBufB;
 #pragma unroll
         for (int k = 0; k < L::kIA; ++k) {
-            const unsigned row = lds_addr(buf) + (wave + k * L::kWaves) * 1024;
+            const unsigned row = sb + (wave + k * L::kWaves) * 1024;
             dma16_lds(srcX, boff_lin[k] + hb, row + L::offX);
             dma16_lds(srcV, boff_lin[k] + hb, row + L::offV);
-            dma16_lds(srcI, boff_swz[k] + hb, row + L::offI);
         }
-#pragma unroll
-        for (int k = 0; k < L::kPA; ++k)
-            dma16_lds(srcP, boff_p[k] + hb, lds_addr(buf) + L::offP + (wave + k * L::kWaves) * 1024);
     };
 
     // Per-head parameters (and per-cell growth parameters) go to LDS once, before
     // any direct load is issued: reading them later from global memory would make
     // the in-order vector-memory counter wait for the next head's staging.
-    __shared__ float sK[H * 9], sMW[H * H], sGa[H], sGb[H], sScale[H], sScaleLo[H];
+    __shared__ __attribute__((aligned(16))) float sMW[H * H];
+    __shared__ float sK[H * 9], sGa[H], sGb[H], sScale[H], sScaleLo[H];
     {
         for (int i = tid; i < H * 9; i += L::kThreads) sK[i] = a.K[pod * H * 9 + i];
         for (int i = tid; i < H * H; i += L::kThreads) {
@@ -285,20 +323,25 @@ __global__ __launch_bounds__((Layout<T, D>::kThreads), 2) void stencil_kernel(St
             sMS[(h * kTileCells + cell) * 2 + 1] = a.sigma[pi];
         }
     }
-    issue_head(0, bufA);
+    if constexpr (kBufs == 1) {
+        issue_pi(0, 0);
+    } else {
+#pragma unroll
+        for (int h = 0; h < kBufs - 1; ++h) issue_pi(h, h), issue_xv(h, h);
+    }
 
-    // ---- phase-B task: a run of 4 cells of one tile row, two adjacent channels ----
-    const bool active = tid < L::kActive;
+    // ---- phase-B task: two cells of one tile row, two adjacent channels ----------------
     const int cp = tid % kPairs;
-    const int grp = tid / kPairs;  // 0..7 when active
-    const int ry = grp >> 1;
-    const int rx0 = (grp & 1) * kRun;
+    const int grp = tid / kPairs;  // 0..15
+    const int ry = grp >> 2;
+    const int rx0 = (grp & 3) * kRun;
     const int c0 = 2 * cp;
     // LDS byte offset of this thread's pair in halo cell (ry, rx0); a window column
     // moves by kRowB bytes, a window row by 10 kRowB.
     const int pbase = (ry * kHaloX + rx0) * L::kRowB + c0 * (int)sizeof(T);
 
-    // ---- phase-A task: one cell, chunk group g of kTPC --------------------------------
+    // ---- phase-A task: one cell, chunk group ag of kTPC --------------------------------
+    const bool scores = tid < kTileCells * L::kTPC;
     const int acell = tid / L::kTPC, ag = tid % L::kTPC;
     const int acy = acell / kTileX, acx = acell % kTileX;
 
@@ -313,14 +356,23 @@ __global__ __launch_bounds__((Layout<T, D>::kThreads), 2) void stencil_kernel(St
     constexpr float kLog2e = 1.4426950408889634f;
     const Growth gc = growth_args(a.growth_fn, 0.f, 1.f, a.dt);  // c0, c1, c2 of the function
 
-    auto do_head = [&](int h, const unsigned char* buf, unsigned char* nxt) {
-        float* sA = sAtt[h & 1];
-        wait_vm0();       // this wave's loads of head h have landed
-        __syncthreads();  // ... and every other wave's; head h-1 is fully consumed
-        if (h + 1 < H) issue_head(h + 1, nxt);
+    int slot = 0, fill = kBufs - 1;
+#pragma unroll 1
+    for (int h = 0; h < H; ++h) {
+        // This wave's loads of head h (for one buffer: its I and P) have landed ...
+        if constexpr (kBufs <= 2) wait_vm0();
+        else wait_heads<L::kLoads>(min(kBufs - 2, H - 1 - h));
+        lds_barrier();  // ... and every other wave's; head h-1 is fully consumed
+        if constexpr (kBufs == 1) {
+            issue_xv(h, 0);
+        } else if (h + kBufs - 1 < H) {
+            issue_pi(h + kBufs - 1, fill);
+            issue_xv(h + kBufs - 1, fill);
+        }
+        const unsigned char* buf = stage + slot * L::kBufB;
 
         // ---- phase A: attention scores (S4) and softmax --------------------------------
-        {
+        if (scores) {
             float s[9];
 #pragma unroll
             for (int k = 0; k < 9; ++k) s[k] = 0.f;
@@ -354,48 +406,29 @@ __global__ __launch_bounds__((Layout<T, D>::kThreads), 2) void stencil_kernel(St
                 for (int k = 0; k < 9; ++k) sA[acell * kAStride + k] = s[k] * inv;
             }
         }
+        if constexpr (kBufs == 1) wait_vm0();  // X and V of head h
         lds_barrier();
+        if constexpr (kBufs == 1) {
+            if (h + 1 < H) issue_pi(h + 1, 0);
+        }
 
         // ---- phase B: potential, growth, propagation, update, head mixing --------------
+        const float s_in = sScale[h], s_lo = sScaleLo[h];
+        float coef[kRun][2], xc[kRun][2];
         float xacc = 0.f;
-        if (active) {
-            const float s_in = sScale[h], s_lo = sScaleLo[h];
-            float kw[9];
-#pragma unroll
-            for (int k = 0; k < 9; ++k) kw[k] = sK[h * 9 + k];
-            float mw[H];
-#pragma unroll
-            for (int o = 0; o < H; ++o) mw[o] = sMW[h * H + o];
-            float ga = 0.f, gb = 0.f;
-            if (!a.per_cell) {
-                ga = sGa[h];
-                gb = sGb[h];
-            }
+        {
             const unsigned char* px = buf + L::offX + pbase;
-            const unsigned char* pvv = buf + L::offV + pbase;
-
-            float2 xw[3][3], vw[3][3];
+            float2 w[3][kRun + 2];
 #pragma unroll
             for (int dy = 0; dy < 3; ++dy)
 #pragma unroll
-                for (int dx = 0; dx < 2; ++dx) {
-                    const int o = (dy * kHaloX + dx) * L::kRowB;
-                    xw[dy][dx] = lds_pair<T>(px + o);
-                    vw[dy][dx] = lds_pair<T>(pvv + o);
-                }
+                for (int dx = 0; dx < kRun + 2; ++dx) w[dy][dx] = lds_pair<T>(px + (dy * kHaloX + dx) * L::kRowB);
+            float kw[9];
+#pragma unroll
+            for (int k = 0; k < 9; ++k) kw[k] = sK[h * 9 + k];
+            float ga = sGa[h], gb = sGb[h];
 #pragma unroll
             for (int x = 0; x < kRun; ++x) {
-#pragma unroll
-                for (int dy = 0; dy < 3; ++dy) {
-                    const int o = (dy * kHaloX + x + 2) * L::kRowB;
-                    xw[dy][2] = lds_pair<T>(px + o);
-                    vw[dy][2] = lds_pair<T>(pvv + o);
-                }
-                const float* ap = sA + (ry * kTileX + rx0 + x) * kAStride;
-                const float4 a0 = reinterpret_cast<const float4*>(ap)[0];
-                const float4 a1 = reinterpret_cast<const float4*>(ap)[1];
-                const float a8 = ap[8];
-                const float aw[9] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w, a8};
                 if (a.per_cell) {
                     const int cell = ry * kTileX + rx0 + x;
                     const float2 ms = *reinterpret_cast<const float2*>(sMS + (h * kTileCells + cell) * 2);
@@ -403,50 +436,64 @@ __global__ __launch_bounds__((Layout<T, D>::kThreads), 2) void stencil_kernel(St
                     ga = gr.ga;
                     gb = gr.gb;
                 }
-                float z[2];
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
-                    float u = 0.f, vt = 0.f;
+                    float u = 0.f;
 #pragma unroll
                     for (int k = 0; k < 9; ++k) {
-                        const float2 xv = xw[k / 3][k % 3];
-                        const float2 vv = vw[k / 3][k % 3];
+                        const float2 xv = w[k / 3][x + k % 3];
                         u = __builtin_fmaf(kw[k], e ? xv.y : xv.x, u);
-                        vt = __builtin_fmaf(aw[k], e ? vv.y : vv.x, vt);
                     }
                     const float us = u * s_in;
                     const float tg = __builtin_fmaf(us, ga, -gb);
                     const float ex = exp2_fast(-tg * tg);
-                    const float coef = __builtin_fmaf(ex, __builtin_fmaf(gc.c2, us, gc.c1), gc.c0);  // dt * g
-                    const float xv = e ? xw[1][1].y : xw[1][1].x;
-                    const float xc = __builtin_fmaf(xv, s_lo, xv * s_in);
-                    z[e] = __builtin_fmaf(coef, vt, xc);
-                    xacc += xc;
+                    coef[x][e] = __builtin_fmaf(ex, __builtin_fmaf(gc.c2, us, gc.c1), gc.c0);  // dt * g
+                    const float xv = e ? w[1][x + 1].y : w[1][x + 1].x;
+                    xc[x][e] = __builtin_fmaf(xv, s_lo, xv * s_in);
+                    xacc += xc[x][e];
                 }
-#pragma unroll
-                for (int o = 0; o < H; ++o) {
-                    y[o][x][0] = __builtin_fmaf(mw[o], z[0], y[o][x][0]);
-                    y[o][x][1] = __builtin_fmaf(mw[o], z[1], y[o][x][1]);
-                }
-#pragma unroll
-                for (int dy = 0; dy < 3; ++dy) {
-                    xw[dy][0] = xw[dy][1];
-                    xw[dy][1] = xw[dy][2];
-                    vw[dy][0] = vw[dy][1];
-                    vw[dy][1] = vw[dy][2];
-                }
-                // Keep the scheduler from hoisting later cells' LDS reads over this
-                // one: the output accumulators already take a large share of a
-                // 2-waves-per-SIMD register budget.
-                __builtin_amdgcn_sched_barrier(0);
             }
+        }
+        {
+            const unsigned char* pv = buf + L::offV + pbase;
+            float2 w[3][kRun + 2];
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+                for (int dx = 0; dx < kRun + 2; ++dx) w[dy][dx] = lds_pair<T>(pv + (dy * kHaloX + dx) * L::kRowB);
+            float z[kRun][2];
+#pragma unroll
+            for (int x = 0; x < kRun; ++x) {
+                const float* ap = sA + (ry * kTileX + rx0 + x) * kAStride;
+                const float4 a0 = reinterpret_cast<const float4*>(ap)[0];
+                const float4 a1 = reinterpret_cast<const float4*>(ap)[1];
+                const float a8 = ap[8];
+                const float aw[9] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w, a8};
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    float vt = 0.f;
+#pragma unroll
+                    for (int k = 0; k < 9; ++k) {
+                        const float2 vv = w[k / 3][x + k % 3];
+                        vt = __builtin_fmaf(aw[k], e ? vv.y : vv.x, vt);
+                    }
+                    z[x][e] = __builtin_fmaf(coef[x][e], vt, xc[x][e]);
+                }
+            }
+            const float4 m0 = reinterpret_cast<const float4*>(sMW)[2 * h], m1 = reinterpret_cast<const float4*>(sMW)[2 * h + 1];
+            const float mw[H] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+#pragma unroll
+            for (int o = 0; o < H; ++o)
+#pragma unroll
+                for (int x = 0; x < kRun; ++x) {
+                    y[o][x][0] = __builtin_fmaf(mw[o], z[x][0], y[o][x][0]);
+                    y[o][x][1] = __builtin_fmaf(mw[o], z[x][1], y[o][x][1]);
+                }
         }
 #pragma unroll
         for (int j = 0; j < H; ++j) xin[j] = (j == h) ? xacc : xin[j];
-    };
-    for (int h = 0; h < H; h += 2) {
-        do_head(h, bufA, bufB);
-        do_head(h + 1, bufB, bufA);
+        slot = slot + 1 == kBufs ? 0 : slot + 1;
+        fill = fill + 1 == kBufs ? 0 : fill + 1;
     }
 
     // ---- phase C: store Y and the tile's mass partial sums ------------------------------
@@ -454,34 +501,36 @@ __global__ __launch_bounds__((Layout<T, D>::kThreads), 2) void stencil_kernel(St
     float ysum[H];
 #pragma unroll
     for (int o = 0; o < H; ++o) ysum[o] = 0.f;
-    if (active) {
 #pragma unroll
-        for (int x = 0; x < kRun; ++x) {
-            const long long base = bbase + ((long long)(ty0 + ry) * G + tx0 + rx0 + x) * C + c0;
+    for (int x = 0; x < kRun; ++x) {
+        const long long base = bbase + ((long long)(ty0 + ry) * G + tx0 + rx0 + x) * C + c0;
 #pragma unroll
-            for (int o = 0; o < H; ++o) {
-                const float r0 = Store<TY>::round(y[o][x][0]);
-                const float r1 = Store<TY>::round(y[o][x][1]);
-                ysum[o] += r0 + r1;
-                Store<TY>::store2(Yg + base + o * D, r0, r1);
-            }
+        for (int o = 0; o < H; ++o) {
+            const float r0 = Store<TY>::round(y[o][x][0]);
+            const float r1 = Store<TY>::round(y[o][x][1]);
+            ysum[o] += r0 + r1;
+            Store<TY>::store2(Yg + base + o * D, r0, r1);
         }
     }
     // Each lane's few values are summed in fp32; lanes, waves and tiles add in fp64,
     // so the sums stay accurate when the state's values are large and of both signs.
+    // The butterfly leaves lane l holding its 16-lane row's sum of value l & 15.
+    double red[16];  // [0, 8): sum of scaled X per head; [8, 16): sum of stored Y
 #pragma unroll
-    for (int j = 0; j < H; ++j) {
-        const double sx = wave_sum64(xin[j]);
-        const double sy = wave_sum64(ysum[j]);
-        if (lane == 0) {
-            sR[wave * 16 + j] = sx;
-            sR[wave * 16 + H + j] = sy;
-        }
+    for (int o = 0; o < H; ++o) {
+        red[o] = xin[o];
+        red[H + o] = ysum[o];
     }
+    fold_half<8, 0x140>(red, lane, 3);  // row_mirror: partner l ^ 15
+    fold_half<4, 0x141>(red, lane, 2);  // row_half_mirror: partner l ^ 7
+    fold_half<2, 0x4E>(red, lane, 1);   // quad_perm [2,3,0,1]: partner l ^ 2
+    fold_half<1, 0xB1>(red, lane, 0);   // quad_perm [1,0,3,2]: partner l ^ 1
+    sR[tid] = red[0];
     __syncthreads();
     if (tid < 2 * H) {
         double sum = 0.0;
-        for (int w = 0; w < L::kWaves; ++w) sum += sR[w * 16 + tid];
+#pragma unroll
+        for (int r = 0; r < L::kThreads / 16; ++r) sum += sR[r * 16 + tid];
         const int j = tid % H;
         double* dst = tid < H ? a.part_in : a.part_out;
         dst[((long long)b * H + j) * tpb + tile] = sum;
@@ -568,21 +617,6 @@ __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
 __device__ __forceinline__ void split_bf16(float v, bf16_t& hi, bf16_t& lo) {
     hi = f32_to_bf16(v);
     lo = f32_to_bf16(v - bf16_to_f32(hi));
-}
-
-// One step of a butterfly sum of kN*2 per-lane values: lanes whose bit `bit` is
-// set keep the upper half, the others the lower half, each adding the partner
-// lane's copy (DPP kCtrl, whose partner differs from the lane in that bit and in
-// no bit a previous step used).
-template <int kN, int kCtrl>
-__device__ __forceinline__ void fold_half(double (&v)[16], int lane, int bit) {
-    const bool up = (lane >> bit) & 1;
-#pragma unroll
-    for (int i = 0; i < kN; ++i) {
-        const double keep = up ? v[i + kN] : v[i];
-        const double send = up ? v[i] : v[i + kN];
-        v[i] = keep + dpp_f64<kCtrl>(send);
-    }
 }
 
 // Halo row of neighbour k of tile cell c (4 x 8 tile, 6 x 10 halo).
@@ -1176,11 +1210,19 @@ __global__ __launch_bounds__(mf::kThreads, 2) void stencil_mfma_kernel(StencilAr
     }
 }
 
+// One workgroup per tile. With no more tiles than CUs nothing overlaps a workgroup's loads
+// but its own pipeline, so it gets as deep a ring as LDS holds; otherwise the buffers leave
+// room for four waves per SIMD.
 template <typename T, int D, typename TY>
 hipError_t launch_tdy(const StencilArgs& a, hipStream_t s) {
     using L = Layout<T, D>;
-    const int tiles = (a.G / kTileY) * (a.G / kTileX);
-    hipLaunchKernelGGL((stencil_kernel<T, D, TY>), dim3(a.B * tiles), dim3(L::kThreads), 0, s, a);
+    int n_cu = 0;
+    if (hipError_t e = device_cu_count(&n_cu); e != hipSuccess) return e;
+    const int tiles = a.B * (a.G / kTileY) * (a.G / kTileX);
+    if (tiles <= n_cu)
+        hipLaunchKernelGGL((stencil_kernel<T, D, TY, L::kDeep>), dim3(tiles), dim3(L::kThreads), 0, s, a);
+    else
+        hipLaunchKernelGGL((stencil_kernel<T, D, TY, L::kFull>), dim3(tiles), dim3(L::kThreads), 0, s, a);
     return hipGetLastError();
 }
 
