@@ -105,8 +105,9 @@ hipError_t launch_stencil(int dtype, const StencilArgs& a, hipStream_t s);
 // scale[b][h] = |sum_out| > 1e-6 ? sum_in / sum_out : 1, reduced in fixed order,
 // written as two floats per (b, h): scale_out[0][b][h] the fp32 rounding of the
 // fp64 ratio, scale_out[1][b][h] the fp32 rounding of the rest. A scale applied
-// as x * hi + x * lo carries no rounding bias from step to step, so the mass of a
-// long chain of steps does not drift with the rounding of the ratio.
+// as fma(x, hi, x * lo) carries no rounding bias from step to step, so the mass of a
+// long chain of steps does not drift with the rounding of the ratio (added to an
+// already rounded x * hi, x * lo is mostly below half a unit and rounds away).
 // scale64_out (may be nullptr): the same factor as one fp64 value per (b, h).
 hipError_t launch_mass_finalize(const double* part_in, const double* part_out, int BH, int tiles,
                                 double* mass_in, double* mass_out, float* scale_out,

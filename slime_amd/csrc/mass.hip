@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256) void rescale_kernel(const TI* x, const float* 
         v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = __builtin_fmaf(v[i], s_lo, v[i] * s);
+    for (int i = 0; i < 4; ++i) v[i] = __builtin_fmaf(v[i], s, v[i] * s_lo);
     if constexpr (sizeof(T) == 2) {
         reinterpret_cast<uint2*>(y)[q] = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
     } else {
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256) void cell_conserve_kernel(const TX* X, const f
         float sx = 0.f, sy = 0.f;
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            sx += __builtin_fmaf(xv[q], s_lo, xv[q] * s_hi);
+            sx += __builtin_fmaf(xv[q], s_hi, xv[q] * s_lo);
             sy += yv[q];
         }
         // the D / 8 consecutive lanes of one (cell, head) share their sums

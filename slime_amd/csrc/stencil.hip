@@ -449,7 +449,7 @@ void stencil_kernel(StencilArgs a) {
                     const float ex = exp2_fast(-tg * tg);
                     coef[x][e] = __builtin_fmaf(ex, __builtin_fmaf(gc.c2, us, gc.c1), gc.c0);  // dt * g
                     const float xv = e ? w[1][x + 1].y : w[1][x + 1].x;
-                    xc[x][e] = __builtin_fmaf(xv, s_lo, xv * s_in);
+                    xc[x][e] = __builtin_fmaf(xv, s_in, xv * s_lo);
                     xacc += xc[x][e];
                 }
             }
@@ -1025,7 +1025,7 @@ __global__ __launch_bounds__(mf::kThreads, 2) void stencil_mfma_kernel(StencilAr
                             coef[mb][e] = __builtin_fmaf(ex[mb][e], __builtin_fmaf(c2s, u[mb][e], c1), c0);
                         else
                             coef[mb][e] = __builtin_fmaf(ex[mb][e], two_dt, -dt);
-                        xcs[mb][e] = __builtin_fmaf(xv[e], s_lo, xv[e] * s_in);
+                        xcs[mb][e] = __builtin_fmaf(xv[e], s_in, xv[e] * s_lo);
                         xacc += xcs[mb][e];
                     }
                 }
