@@ -32,6 +32,7 @@ struct slime_ca {
 
     float* Wtm = nullptr;      // [pods][3C][C] fp32 masters, transposed (n-major)
     void* Wt = nullptr;        // [B][3C][C] per-batch scaled, transposed
+    void* W1 = nullptr;        // [pods][3C][C] as Wtm, unscaled, in the handle's dtype
     float* K = nullptr;        // [pods][H][9]
     float* mu = nullptr;       // [pods][H] or [pods][G][G][H]
     float* sigma = nullptr;
@@ -46,7 +47,6 @@ struct slime_ca {
     double* part_in = nullptr;  // [B*H][tiles]
     double* part_out = nullptr;
     float* scale[2] = {nullptr, nullptr};  // [2][B*H]: high parts, then low parts
-    float* unit_scale = nullptr;           // [2][B*H]: 1.0, then 0.0
     double* mass_in = nullptr;             // [B*H]
     double* mass_out = nullptr;
 
@@ -183,8 +183,8 @@ hipError_t timed(slime_ca* h, std::vector<std::pair<size_t, size_t>>& log, hipSt
 void release(slime_ca* h) {
     for (hipEvent_t e : h->ev_pool) (void)hipEventDestroy(e);
     h->ev_pool.clear();
-    void* ptrs[] = {h->Wtm, h->Wt, h->K, h->mu, h->sigma, h->M, h->kband, h->sched, h->P, h->I, h->V,
-                    h->S[0], h->S[1], h->Sf, h->part_in, h->part_out, h->scale[0], h->scale[1], h->unit_scale,
+    void* ptrs[] = {h->Wtm, h->Wt, h->W1, h->K, h->mu, h->sigma, h->M, h->kband, h->sched, h->P, h->I, h->V,
+                    h->S[0], h->S[1], h->Sf, h->part_in, h->part_out, h->scale[0], h->scale[1],
                     h->mass_in, h->mass_out, h->gram_part, h->mom_part, h->sweeps, h->org_fit, h->view,
                     h->Wcat, h->Ipre, h->bw_lpart, h->bw_coef, h->bw_loss, h->bw_gU, h->bw_gVt,
                     h->bw_att, h->bw_gS, h->bw_G3, h->bw_gXd, h->bw_ppart, h->bw_gcell,
@@ -222,34 +222,39 @@ class DeviceScope {
     bool restore_ = false;
 };
 
-// S1 for one step: per-batch weights (scaled by the deferred mass scale of x),
-// then the projection GEMM(s).
+// S1 for one step, then the projection GEMM(s). Weights that the deferred mass scale of x
+// does not touch come from W1, one copy per pod: all of them when x_scale is NULL (a state
+// as its caller holds it), and the second and third plane of the chained forms. Scaled
+// ones are written per batch entry first.
 // With `pre` (parallel projections only), I before its GELU is also written there.
 int run_project(slime_ca* h, const void* x, const float* x_scale, void* P, void* I, void* V,
                 hipStream_t s, void* pre = nullptr) {
     const slime_ca_config& c = h->cfg;
-    const int C = h->C;
-    WeightPrepArgs w{};
-    w.Wtm = h->Wtm;
-    w.scale = x_scale;
-    w.Wt = h->Wt;
-    w.B = c.B;
-    w.C = C;
-    w.D = c.D;
-    w.per_pod = c.B / c.pods;
-    w.nplanes = 3;
-    w.scaled_planes = c.pvi_chain ? 1u : 7u;
-    HIP_TRY(launch_weight_prep(c.dtype, w, s));
-
+    const int C = h->C, cells = c.G * c.G, per_pod = c.B / c.pods;
+    if (x_scale) {
+        WeightPrepArgs w{};
+        w.Wtm = h->Wtm;
+        w.scale = x_scale;
+        w.Wt = h->Wt;
+        w.B = c.B;
+        w.C = C;
+        w.D = c.D;
+        w.per_pod = per_pod;
+        w.nplanes = c.pvi_chain ? 1 : 3;
+        HIP_TRY(launch_weight_prep(c.dtype, w, s));
+    }
     GemmArgs g{};
-    g.rows_per_batch = c.G * c.G;
-    g.M = c.B * c.G * c.G;
+    g.M = c.B * cells;
     g.K = C;
     g.ncol = C;
     g.bt_batch_stride = 3LL * C * C;
+    auto weights = [&](bool scaled, int plane) {
+        g.Bt = static_cast<const char*>(scaled ? h->Wt : h->W1) + (size_t)plane * C * C * h->elem;
+        g.rows_per_batch = scaled ? cells : per_pod * cells;
+    };
     if (!c.pvi_chain) {
         g.A = x;
-        g.Bt = h->Wt;
+        weights(x_scale != nullptr, 0);
         g.N = 3 * C;
         g.out[0] = P;
         g.out[1] = I;
@@ -273,7 +278,7 @@ int run_project(slime_ca* h, const void* x, const float* x_scale, void* P, void*
         g.N = C;
         for (int p = 0; p < 3; ++p) {
             g.A = ins[p];
-            g.Bt = static_cast<const char*>(h->Wt) + (size_t)p * C * C * h->elem;
+            weights(p == 0 && x_scale != nullptr, p);
             g.out[0] = outs[p];
             g.act[0] = acts[p];
             HIP_TRY(timed(h, h->gemm_ev, s, [&] { return launch_gemm(c.dtype, g, s); }));
@@ -399,6 +404,7 @@ int slime_ca_create(const slime_ca_config* config, slime_ca** out) {
     rc = 0;
     rc = rc ? rc : dalloc_t(&h->Wtm, (size_t)c.pods * 3 * C * C * 4);
     rc = rc ? rc : dalloc(&h->Wt, (size_t)c.B * 3 * C * C * h->elem);
+    rc = rc ? rc : dalloc(&h->W1, (size_t)c.pods * 3 * C * C * h->elem);
     rc = rc ? rc : dalloc_t(&h->K, (size_t)c.pods * c.H * 9 * 4);
     rc = rc ? rc : dalloc_t(&h->mu, n_param_growth(c) * 4);
     rc = rc ? rc : dalloc_t(&h->sigma, n_param_growth(c) * 4);
@@ -418,7 +424,6 @@ int slime_ca_create(const slime_ca_config* config, slime_ca** out) {
     // scales: [2][B*H] fp32, the high parts then the low parts (scale = hi + lo)
     rc = rc ? rc : dalloc_t(&h->scale[0], 2 * BH * 4);
     rc = rc ? rc : dalloc_t(&h->scale[1], 2 * BH * 4);
-    rc = rc ? rc : dalloc_t(&h->unit_scale, 2 * BH * 4);
     rc = rc ? rc : dalloc_t(&h->mass_in, BH * 8);
     rc = rc ? rc : dalloc_t(&h->mass_out, BH * 8);
     rc = rc ? rc : dalloc_t(&h->sweeps, BH * sizeof(int));
@@ -427,11 +432,7 @@ int slime_ca_create(const slime_ca_config* config, slime_ca** out) {
         delete h;
         return rc;
     }
-    float* ones = new float[2 * BH];
-    for (size_t i = 0; i < 2 * BH; ++i) ones[i] = i < BH ? 1.0f : 0.0f;
-    hipError_t e = hipMemcpy(h->unit_scale, ones, 2 * BH * 4, hipMemcpyHostToDevice);
-    delete[] ones;
-    if (e == hipSuccess) e = hipMemset(h->mass_in, 0, BH * 8);
+    hipError_t e = hipMemset(h->mass_in, 0, BH * 8);
     if (e == hipSuccess) e = hipMemset(h->mass_out, 0, BH * 8);
     if (e == hipSuccess && h->sched) e = hipMemset(h->sched, 0, 16 * sizeof(unsigned));
     if (e != hipSuccess) {
@@ -507,6 +508,19 @@ int slime_ca_set_params(slime_ca* h, const slime_ca_params* p) {
             HIP_TRY(hipMemcpy(h->Wtm + (size_t)q * 3 * CC, t.data(), 3 * CC * 4,
                               hipMemcpyHostToDevice));
         }
+    }
+    // The unscaled copy that the GEMMs read: laid out once here, on the stream the uploads use.
+    {
+        WeightPrepArgs w{};
+        w.Wtm = h->Wtm;
+        w.Wt = h->W1;
+        w.B = c.pods;
+        w.C = h->C;
+        w.D = c.D;
+        w.per_pod = 1;
+        w.nplanes = 3;
+        HIP_TRY(launch_weight_prep(c.dtype, w, nullptr));
+        HIP_TRY(hipStreamSynchronize(nullptr));
     }
     // [W_P | W_I | W_V] by input channel, for the backward's dX GEMM (uploaded by
     // slime_ca_backward when first needed).
@@ -585,7 +599,7 @@ int slime_ca_step(slime_ca* h, const void* x_in, void* x_out, int n_steps, void*
         return SLIME_OK;
     }
     const void* cur = x_in;
-    const float* cur_scale = h->unit_scale;
+    const float* cur_scale = nullptr;  // the caller's state is complete
     // Intermediate outputs stay unscaled in the storage type: the next step applies
     // the conservation factor in fp32 as it reads them. The last step writes fp32
     // (bf16 state) so the final rescale rounds once.
@@ -660,7 +674,7 @@ int slime_ca_rollout(slime_ca* h, void* hist, int T, double* scales, void* strea
     // Step t reads state t-1 as stored, with its factor folded into the weights and
     // the stencil's loads, and stores state t before its own rescale; the factor goes
     // to the handle (for step t+1) and to scales[t].
-    const float* cur_scale = h->unit_scale;
+    const float* cur_scale = nullptr;  // hist[0] is complete
     for (int t = 1; t < T; ++t) {
         const void* cur = base + (size_t)(t - 1) * state_bytes;
         void* y = base + (size_t)t * state_bytes;

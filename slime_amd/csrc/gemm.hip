@@ -89,18 +89,16 @@ constexpr int kPrepBatches = 8;  // batches per thread
 // 16-byte (bf16) or two 16-byte (fp32) stores.
 template <typename T>
 __global__ __launch_bounds__(256) void weight_prep_kernel(WeightPrepArgs w) {
-    const long long per_b = (long long)w.nplanes * w.C * w.C;
+    const long long per_b = (long long)w.nplanes * w.C * w.C, stride = 3LL * w.C * w.C;
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const int pods = w.B / w.per_pod;
     if (q * 8 >= per_b * pods) return;
     const int pod = (int)(q * 8 / per_b);
     const long long r = q * 8 - (long long)pod * per_b;
     const int k = (int)(r % w.C);
-    const int p = (int)(r / ((long long)w.C * w.C));
-    const float* src = w.Wtm + (long long)pod * per_b + r;
+    const float* src = w.Wtm + (long long)pod * stride + r;
     const float4 v0 = *reinterpret_cast<const float4*>(src);
     const float4 v1 = *reinterpret_cast<const float4*>(src + 4);
-    const bool scaled = w.scale && ((w.scaled_planes >> p) & 1u);
     const int heads = w.C / w.D, head = k / w.D;
     const int b0 = blockIdx.y * kPrepBatches;
     const int b1 = min(w.per_pod, b0 + kPrepBatches);
@@ -109,17 +107,17 @@ __global__ __launch_bounds__(256) void weight_prep_kernel(WeightPrepArgs w) {
         const int b = pod * w.per_pod + bb;
         // scale = hi + lo, applied as w * hi + w * lo with one rounding (the stencil
         // applies the same factor to its reads of the state)
-        const float s = scaled ? w.scale[b * heads + head] : 1.0f;
-        const float sl = scaled ? w.scale[(long long)w.B * heads + b * heads + head] : 0.0f;
+        const float s = w.scale ? w.scale[b * heads + head] : 1.0f;
+        const float sl = w.scale ? w.scale[(long long)w.B * heads + b * heads + head] : 0.0f;
         float o[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = __builtin_fmaf(o[e], s, o[e] * sl);
         if constexpr (sizeof(T) == 2) {
-            *reinterpret_cast<uint4*>(static_cast<T*>(w.Wt) + (long long)b * per_b + r) =
+            *reinterpret_cast<uint4*>(static_cast<T*>(w.Wt) + (long long)b * stride + r) =
                 make_uint4(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]),
                            pack_bf16x2(o[6], o[7]));
         } else {
-            float* dst = static_cast<float*>(w.Wt) + (long long)b * per_b + r;
+            float* dst = static_cast<float*>(w.Wt) + (long long)b * stride + r;
             *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
             *reinterpret_cast<float4*>(dst + 4) = make_float4(o[4], o[5], o[6], o[7]);
         }

@@ -18,7 +18,7 @@ struct GemmArgs {
     const void* A;             // [M][K] rows (cells), K contiguous
     const void* Bt;            // per batch [N][K], K contiguous
     long long bt_batch_stride; // elements between consecutive batches' Bt
-    int rows_per_batch;        // rows of A that share one Bt (G*G)
+    int rows_per_batch;        // rows of A that share one Bt
     int M, N, K;
     void* out[3];              // output planes [M][ncol]
     int ncol;                  // columns per plane
@@ -49,14 +49,13 @@ hipError_t launch_neighbourhood_sum(int dtype, const void* X, void* S, int B, in
                                     hipStream_t s);
 
 // ---- per-batch scaled, transposed weights -------------------------------------
-// Wt[b][p*C + n][k] = cvt( scale_p(b, k) * Wtm[pod(b)][p*C + n][k] ), where the
-// mass scale applies only to planes that consume the state (scale[b][k / D]).
+// Wt[b][n][k] = cvt( scale(b, k) * Wtm[pod(b)][n][k] ) for the first nplanes * C of the 3C
+// rows n (the planes that consume the state): the mass scale of channel k, scale[b][k / D].
 struct WeightPrepArgs {
-    const float* Wtm;     // [pods][nplanes*C][C] fp32 masters, already transposed
-    const float* scale;   // [2][B][H] high then low parts (scale = hi + lo), or nullptr
-    void* Wt;             // [B][nplanes*C][C]
+    const float* Wtm;     // [pods][3C][C] fp32 masters, already transposed
+    const float* scale;   // [2][B][H] high then low parts (scale = hi + lo), or nullptr: 1
+    void* Wt;             // [B][3C][C]
     int B, C, D, per_pod, nplanes;
-    unsigned scaled_planes;  // bit p set: plane p is multiplied by the scale
 };
 hipError_t launch_weight_prep(int dtype, const WeightPrepArgs& a, hipStream_t s);
 
