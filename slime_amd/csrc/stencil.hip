@@ -69,14 +69,13 @@ struct Layout {
     static constexpr int kPG = kPCells / kCPI;               // instruction groups of the P tile
     static constexpr int kIA = kHG / kWaves;                 // per wave, per halo array
     static_assert(kHG % kWaves == 0 && kPG <= kWaves, "DMA groups must split over waves");
-    static constexpr int kLoads = 3 * kIA + 1;               // per wave and head (wave w >= kPG
-                                                             // repeats P group w % kPG)
     static constexpr int kBufB = (3 * kHaloPad + kPCells) * kRowB;
     static constexpr int offX = 0, offV = kHaloPad * kRowB, offI = 2 * kHaloPad * kRowB,
                          offP = 3 * kHaloPad * kRowB;
-    // Staging buffers: see stencil_kernel.
+    // Staging buffers and heads at once: see stencil_kernel.
     static constexpr int kFull = sizeof(T) == 2 ? 2 : 1;
-    static constexpr int kDeep = 150 * 1024 / kBufB < kHeads ? 150 * 1024 / kBufB : kHeads;
+    static constexpr int kPar = D == 64 ? 1 : 1024 / kThreads < kHeads ? 1024 / kThreads : kHeads;
+    static constexpr int kParTiles = D == 8 ? 4 : D == 16 && sizeof(T) == 2 ? 2 : 1;  // per CU
 };
 
 // Direct global->LDS loads: dma16_lds, dma16_lds_nt, wait_vm0 (common.hpp); the kernel
@@ -189,53 +188,44 @@ __device__ __forceinline__ void fold_half(double (&v)[16], int lane, int bit) {
     }
 }
 
-// Waits until at most `heads` heads' loads of this wave are in flight.
-template <int kLoads>
-__device__ __forceinline__ void wait_heads(int heads) {
-#define SLIME_WAIT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | ((((n) >> 4) & 3) << 14) | 0x0F70)
-    static_assert(6 * kLoads < 64, "vmcnt has 6 bits");
-    switch (heads) {
-        case 6: SLIME_WAIT(6 * kLoads); break;
-        case 5: SLIME_WAIT(5 * kLoads); break;
-        case 4: SLIME_WAIT(4 * kLoads); break;
-        case 3: SLIME_WAIT(3 * kLoads); break;
-        case 2: SLIME_WAIT(2 * kLoads); break;
-        case 1: SLIME_WAIT(kLoads); break;
-        default: SLIME_WAIT(0); break;
-    }
-#undef SLIME_WAIT
-}
-
 // TY: storage type of the unscaled output; fp32 when the caller rescales it into
 // the final bf16 state (one rounding instead of two).
 //
 // kBufs: how a head's data meets its compute. 1: one buffer in two halves -- I and P of
 // the next head load during phase B, which no longer reads them, X and V during phase A --
-// so that two workgroups of a CU (57 KiB each for fp32, D = 64) cover each other. 2 or
-// more: a ring, the loads of the next kBufs - 1 heads in flight; eight buffers hold the
-// whole tile, so that a grid with no second workgroup to overlap pays one memory round
-// trip instead of eight. launch_tdy picks.
+// so that two workgroups of a CU (57 KiB each for fp32, D = 64) cover each other. 2: the
+// next head's data load into the other buffer while this one computes.
+//
+// kPar: heads computed at once. 1: the workgroup walks the 8 heads, each thread adding its
+// share of all eight outputs in registers. More: kPar groups of threads take heads of their
+// own, the updated states Z meet in LDS, and each group mixes its share of the outputs, in
+// the same order and with the same bits; a grid of few tiles then has kPar times the
+// wavefronts and 1 / kPar of the serial chain. launch_tdy picks.
 //
 // What bounds it: VALU and LDS issue with four waves per SIMD (two cells per thread keep
 // the output accumulators at 32 and the kernel at 128 registers).
 // Measured: 1 x 128^2 x 512 fp32 57 -> 37 us (4.6 TB/s of the five planes; one workgroup of 4
-// waves per CU and four cells per thread before), 8 x 104^2 x 256 bf16 85 -> 76 us,
-// 1 x 32^2 x 64 fp32 (32 tiles, eight buffers) 17 -> 14 us.
-template <typename T, int D, typename TY, int kBufs>
-__global__ __launch_bounds__((Layout<T, D>::kThreads), (kBufs == Layout<T, D>::kFull ? 4 : 2))
+// waves per CU and four cells per thread before), 8 x 104^2 x 256 bf16 85 -> 76 us.
+template <typename T, int D, typename TY, int kBufs, int kPar>
+__global__ __launch_bounds__((Layout<T, D>::kThreads * kPar), (kPar == 1 ? 4 : 2))
 void stencil_kernel(StencilArgs a) {
     using L = Layout<T, D>;
+    static_assert(kPar == 1 || kBufs == 1, "parallel heads stage one buffer each");
     constexpr int H = kHeads;
     constexpr int C = H * D;
     constexpr int kPairs = D / 2;
-    __shared__ __attribute__((aligned(1024))) unsigned char stage[kBufs * L::kBufB];
-    __shared__ __attribute__((aligned(16))) float sA[kTileCells * kAStride];
+    constexpr int kRounds = H / kPar;
+    constexpr int kAll = L::kThreads * kPar;  // threads
+    __shared__ __attribute__((aligned(1024))) unsigned char stage[kBufs * kPar * L::kBufB];
+    __shared__ __attribute__((aligned(16))) float sAtt[kPar * kTileCells * kAStride];
     __shared__ __attribute__((aligned(16))) float sMS[H * kTileCells * 2];
-    __shared__ double sR[L::kThreads];
+    __shared__ double sR[kPar > 1 ? L::kWaves * kPar * 2 * kRounds : L::kThreads];
 
-    const int tid = threadIdx.x;
+    const int gw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scalar LDS addresses
+    const int group = kPar > 1 ? gw / L::kWaves : 0;                  // of heads
+    const int wave = gw - group * L::kWaves, tid = threadIdx.x - group * L::kThreads;  // in the group
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar LDS addresses
+    float* sA = sAtt + group * kTileCells * kAStride;
     const int G = a.G;
     const int tiles_x = G / kTileX;
     const int tpb = (G / kTileY) * tiles_x;
@@ -293,41 +283,40 @@ void stencil_kernel(StencilArgs a) {
         }
     };
 
-    // Per-head parameters (and per-cell growth parameters) go to LDS once, before
-    // any direct load is issued: reading them later from global memory would make
-    // the in-order vector-memory counter wait for the next head's staging.
+    if constexpr (kPar > 1) issue_xv(group, group);
+    issue_pi(group, group);
+    if constexpr (kBufs > 1) issue_xv(0, 0);
+
+    // Per-head parameters (and per-cell growth parameters) go to LDS once: reading them
+    // later from global memory would make the in-order vector-memory counter wait for
+    // the next head's staging.
     __shared__ __attribute__((aligned(16))) float sMW[H * H];
     __shared__ float sK[H * 9], sGa[H], sGb[H], sScale[H], sScaleLo[H];
     {
-        for (int i = tid; i < H * 9; i += L::kThreads) sK[i] = a.K[pod * H * 9 + i];
-        for (int i = tid; i < H * H; i += L::kThreads) {
+        const int all = threadIdx.x;
+        for (int i = all; i < H * 9; i += kAll) sK[i] = a.K[pod * H * 9 + i];
+        for (int i = all; i < H * H; i += kAll) {
             const int hh = i / H, o = i % H;  // sMW[h][o] = M[o][h]
             sMW[i] = a.M[(pod * H + o) * H + hh];
         }
-        if (tid < H) {
-            sScale[tid] = a.scale_in ? a.scale_in[b * H + tid] : 1.0f;
-            sScaleLo[tid] = a.scale_in ? a.scale_in[a.B * H + b * H + tid] : 0.0f;
+        if (all < H) {
+            sScale[all] = a.scale_in ? a.scale_in[b * H + all] : 1.0f;
+            sScaleLo[all] = a.scale_in ? a.scale_in[a.B * H + b * H + all] : 0.0f;
             if (!a.per_cell) {
-                const Growth gr = growth_args(a.growth_fn, a.mu[pod * H + tid], a.sigma[pod * H + tid], a.dt);
-                sGa[tid] = gr.ga;
-                sGb[tid] = gr.gb;
+                const Growth gr = growth_args(a.growth_fn, a.mu[pod * H + all], a.sigma[pod * H + all], a.dt);
+                sGa[all] = gr.ga;
+                sGb[all] = gr.gb;
             }
         }
-    }
-    if (a.per_cell) {
-        for (int i = tid; i < kTileCells * H; i += L::kThreads) {
-            const int cell = i / H, h = i % H;
-            const long long pi =
-                (((long long)pod * G + ty0 + cell / kTileX) * G + tx0 + cell % kTileX) * H + h;
-            sMS[(h * kTileCells + cell) * 2 + 0] = a.mu[pi];
-            sMS[(h * kTileCells + cell) * 2 + 1] = a.sigma[pi];
+        if (a.per_cell) {
+            for (int i = all; i < kTileCells * H; i += kAll) {
+                const int cell = i / H, h = i % H;
+                const long long pi =
+                    (((long long)pod * G + ty0 + cell / kTileX) * G + tx0 + cell % kTileX) * H + h;
+                sMS[(h * kTileCells + cell) * 2 + 0] = a.mu[pi];
+                sMS[(h * kTileCells + cell) * 2 + 1] = a.sigma[pi];
+            }
         }
-    }
-    if constexpr (kBufs == 1) {
-        issue_pi(0, 0);
-    } else {
-#pragma unroll
-        for (int h = 0; h < kBufs - 1; ++h) issue_pi(h, h), issue_xv(h, h);
     }
 
     // ---- phase-B task: two cells of one tile row, two adjacent channels ----------------
@@ -345,29 +334,29 @@ void stencil_kernel(StencilArgs a) {
     const int acell = tid / L::kTPC, ag = tid % L::kTPC;
     const int acy = acell / kTileX, acx = acell % kTileX;
 
-    float y[H][kRun][2];
+    float y[kPar > 1 ? 1 : H][kRun][2];
 #pragma unroll
-    for (int o = 0; o < H; ++o)
+    for (int o = 0; o < (kPar > 1 ? 1 : H); ++o)
 #pragma unroll
         for (int x = 0; x < kRun; ++x) y[o][x][0] = y[o][x][1] = 0.f;
-    float xin[H] = {};
+    float xin[kRounds] = {};
+    float4 zr[kPar > 1 ? kRounds : 1];  // parallel heads: this thread's Z of each round
 
     const float inv_sqrt_d = 1.0f / __builtin_sqrtf((float)D);
     constexpr float kLog2e = 1.4426950408889634f;
     const Growth gc = growth_args(a.growth_fn, 0.f, 1.f, a.dt);  // c0, c1, c2 of the function
 
-    int slot = 0, fill = kBufs - 1;
 #pragma unroll 1
-    for (int h = 0; h < H; ++h) {
-        // This wave's loads of head h (for one buffer: its I and P) have landed ...
-        if constexpr (kBufs <= 2) wait_vm0();
-        else wait_heads<L::kLoads>(min(kBufs - 2, H - 1 - h));
-        lds_barrier();  // ... and every other wave's; head h-1 is fully consumed
+    for (int r = 0; r < kRounds; ++r) {
+        const int h = r * kPar + group;
+        const int slot = kBufs > 1 ? (r & 1) : group;
+        wait_vm0();     // this wave's loads of head h (for one buffer: its I and P) have landed ...
+        lds_barrier();  // ... and every other wave's; the head before is fully consumed
         if constexpr (kBufs == 1) {
-            issue_xv(h, 0);
-        } else if (h + kBufs - 1 < H) {
-            issue_pi(h + kBufs - 1, fill);
-            issue_xv(h + kBufs - 1, fill);
+            if (kPar == 1 || r > 0) issue_xv(h, slot);
+        } else if (r + 1 < kRounds) {
+            issue_pi(h + 1, slot ^ 1);
+            issue_xv(h + 1, slot ^ 1);
         }
         const unsigned char* buf = stage + slot * L::kBufB;
 
@@ -409,7 +398,7 @@ void stencil_kernel(StencilArgs a) {
         if constexpr (kBufs == 1) wait_vm0();  // X and V of head h
         lds_barrier();
         if constexpr (kBufs == 1) {
-            if (h + 1 < H) issue_pi(h + 1, 0);
+            if (r + 1 < kRounds) issue_pi(h + kPar, slot);
         }
 
         // ---- phase B: potential, growth, propagation, update, head mixing --------------
@@ -480,60 +469,103 @@ void stencil_kernel(StencilArgs a) {
                     z[x][e] = __builtin_fmaf(coef[x][e], vt, xc[x][e]);
                 }
             }
-            const float4 m0 = reinterpret_cast<const float4*>(sMW)[2 * h], m1 = reinterpret_cast<const float4*>(sMW)[2 * h + 1];
-            const float mw[H] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+            if constexpr (kPar > 1) {
+                static_assert(kRun == 2, "a thread's Z is one float4");
 #pragma unroll
-            for (int o = 0; o < H; ++o)
+                for (int j = 0; j < kRounds; ++j)
+                    if (j == r) zr[j] = make_float4(z[0][0], z[0][1], z[1][0], z[1][1]);
+            } else {
+                const float4 m0 = reinterpret_cast<const float4*>(sMW)[2 * h], m1 = reinterpret_cast<const float4*>(sMW)[2 * h + 1];
+                const float mw[H] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
 #pragma unroll
-                for (int x = 0; x < kRun; ++x) {
-                    y[o][x][0] = __builtin_fmaf(mw[o], z[x][0], y[o][x][0]);
-                    y[o][x][1] = __builtin_fmaf(mw[o], z[x][1], y[o][x][1]);
-                }
+                for (int o = 0; o < H; ++o)
+#pragma unroll
+                    for (int x = 0; x < kRun; ++x) {
+                        y[o][x][0] = __builtin_fmaf(mw[o], z[x][0], y[o][x][0]);
+                        y[o][x][1] = __builtin_fmaf(mw[o], z[x][1], y[o][x][1]);
+                    }
+            }
         }
 #pragma unroll
-        for (int j = 0; j < H; ++j) xin[j] = (j == h) ? xacc : xin[j];
-        slot = slot + 1 == kBufs ? 0 : slot + 1;
-        fill = fill + 1 == kBufs ? 0 : fill + 1;
+        for (int j = 0; j < kRounds; ++j) xin[j] = (j == r) ? xacc : xin[j];
     }
 
     // ---- phase C: store Y and the tile's mass partial sums ------------------------------
-    TY* Yg = static_cast<TY*>(a.Y);
-    float ysum[H];
-#pragma unroll
-    for (int o = 0; o < H; ++o) ysum[o] = 0.f;
-#pragma unroll
-    for (int x = 0; x < kRun; ++x) {
-        const long long base = bbase + ((long long)(ty0 + ry) * G + tx0 + rx0 + x) * C + c0;
-#pragma unroll
-        for (int o = 0; o < H; ++o) {
-            const float r0 = Store<TY>::round(y[o][x][0]);
-            const float r1 = Store<TY>::round(y[o][x][1]);
-            ysum[o] += r0 + r1;
-            Store<TY>::store2(Yg + base + o * D, r0, r1);
-        }
-    }
     // Each lane's few values are summed in fp32; lanes, waves and tiles add in fp64,
     // so the sums stay accurate when the state's values are large and of both signs.
-    // The butterfly leaves lane l holding its 16-lane row's sum of value l & 15.
-    double red[16];  // [0, 8): sum of scaled X per head; [8, 16): sum of stored Y
+    TY* Yg = static_cast<TY*>(a.Y);
+    const long long ybase = bbase + ((long long)(ty0 + ry) * G + tx0 + rx0) * C + c0;
+    auto store = [&](int o, const float (&v)[kRun][2]) {  // returns the stored values' sum
+        float sum = 0.f;
 #pragma unroll
-    for (int o = 0; o < H; ++o) {
-        red[o] = xin[o];
-        red[H + o] = ysum[o];
-    }
-    fold_half<8, 0x140>(red, lane, 3);  // row_mirror: partner l ^ 15
-    fold_half<4, 0x141>(red, lane, 2);  // row_half_mirror: partner l ^ 7
-    fold_half<2, 0x4E>(red, lane, 1);   // quad_perm [2,3,0,1]: partner l ^ 2
-    fold_half<1, 0xB1>(red, lane, 0);   // quad_perm [1,0,3,2]: partner l ^ 1
-    sR[tid] = red[0];
-    __syncthreads();
-    if (tid < 2 * H) {
-        double sum = 0.0;
+        for (int x = 0; x < kRun; ++x) {
+            const float r0 = Store<TY>::round(v[x][0]);
+            const float r1 = Store<TY>::round(v[x][1]);
+            sum += r0 + r1;
+            Store<TY>::store2(Yg + ybase + (long long)x * C + o * D, r0, r1);
+        }
+        return sum;
+    };
+    if constexpr (kPar > 1) {
+        // Z of every head, in the staging buffers, which no group reads any more.
+        static_assert(H * L::kThreads * (int)sizeof(float4) <= kPar * L::kBufB, "Z fits the staging buffers");
+        float4* sZ = reinterpret_cast<float4*>(stage);
+        lds_barrier();
 #pragma unroll
-        for (int r = 0; r < L::kThreads / 16; ++r) sum += sR[r * 16 + tid];
-        const int j = tid % H;
-        double* dst = tid < H ? a.part_in : a.part_out;
-        dst[((long long)b * H + j) * tpb + tile] = sum;
+        for (int r = 0; r < kRounds; ++r) sZ[(r * kPar + group) * L::kThreads + tid] = zr[r];
+        lds_barrier();
+        // This group's outputs o = group * kRounds + r.
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) {
+            const int o = group * kRounds + r;
+            float v[kRun][2] = {};
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                const float4 z = sZ[h * L::kThreads + tid];
+                const float mw = sMW[h * H + o];
+                v[0][0] = __builtin_fmaf(mw, z.x, v[0][0]);
+                v[0][1] = __builtin_fmaf(mw, z.y, v[0][1]);
+                v[1][0] = __builtin_fmaf(mw, z.z, v[1][0]);
+                v[1][1] = __builtin_fmaf(mw, z.w, v[1][1]);
+            }
+            const double sy = wave_sum64(store(o, v)), sx = wave_sum64(xin[r]);
+            if (lane == 0) {
+                sR[(gw * kRounds + r) * 2] = sx;
+                sR[(gw * kRounds + r) * 2 + 1] = sy;
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < 2 * H) {
+            const int j = threadIdx.x % H, out = threadIdx.x / H;
+            const int g = out ? j / kRounds : j % kPar, r = out ? j % kRounds : j / kPar;
+            double sum = 0.0;
+#pragma unroll
+            for (int w = 0; w < L::kWaves; ++w) sum += sR[((g * L::kWaves + w) * kRounds + r) * 2 + out];
+            double* dst = out ? a.part_out : a.part_in;
+            dst[((long long)b * H + j) * tpb + tile] = sum;
+        }
+    } else {
+        // The butterfly leaves lane l holding its 16-lane row's sum of value l & 15.
+        double red[16];  // [0, 8): sum of scaled X per head; [8, 16): sum of stored Y
+#pragma unroll
+        for (int o = 0; o < H; ++o) {
+            red[o] = xin[o];
+            red[H + o] = store(o, y[o]);
+        }
+        fold_half<8, 0x140>(red, lane, 3);  // row_mirror: partner l ^ 15
+        fold_half<4, 0x141>(red, lane, 2);  // row_half_mirror: partner l ^ 7
+        fold_half<2, 0x4E>(red, lane, 1);   // quad_perm [2,3,0,1]: partner l ^ 2
+        fold_half<1, 0xB1>(red, lane, 0);   // quad_perm [1,0,3,2]: partner l ^ 1
+        sR[tid] = red[0];
+        __syncthreads();
+        if (tid < 2 * H) {
+            double sum = 0.0;
+#pragma unroll
+            for (int r = 0; r < L::kThreads / 16; ++r) sum += sR[r * 16 + tid];
+            const int j = tid % H;
+            double* dst = tid < H ? a.part_in : a.part_out;
+            dst[((long long)b * H + j) * tpb + tile] = sum;
+        }
     }
 }
 
@@ -1210,19 +1242,26 @@ __global__ __launch_bounds__(mf::kThreads, 2) void stencil_mfma_kernel(StencilAr
     }
 }
 
-// One workgroup per tile. With no more tiles than CUs nothing overlaps a workgroup's loads
-// but its own pipeline, so it gets as deep a ring as LDS holds; otherwise the buffers leave
-// room for four waves per SIMD.
+// One workgroup per tile. Heads in parallel (D < 64) while the tiles leave the card room for
+// it: up to kParTiles tiles per CU. Measured, full / parallel in us:
+//   D = 8   fp32 32 tiles 11.7 / 5.5, 1024 tiles 16.2 / 15.7, 1600 tiles 21.3 / 23.4
+//   D = 16  bf16 162 tiles 13.5 / 7.2, 576 tiles 16.1 / 14.7, 1600 tiles 26.5 / 30.1
+//           fp32 162 tiles 14.4 / 8.2, 576 tiles 18.3 / 23.5
+//   D = 32  fp32 162 tiles 16.2 / 11.8, 288 tiles 19.1 / 23.0
+//   D = 64  fp32 32 tiles 18.5 / 18.2, 162 tiles 19.4 / 20.6: never
 template <typename T, int D, typename TY>
 hipError_t launch_tdy(const StencilArgs& a, hipStream_t s) {
     using L = Layout<T, D>;
-    int n_cu = 0;
-    if (hipError_t e = device_cu_count(&n_cu); e != hipSuccess) return e;
     const int tiles = a.B * (a.G / kTileY) * (a.G / kTileX);
-    if (tiles <= n_cu)
-        hipLaunchKernelGGL((stencil_kernel<T, D, TY, L::kDeep>), dim3(tiles), dim3(L::kThreads), 0, s, a);
-    else
-        hipLaunchKernelGGL((stencil_kernel<T, D, TY, L::kFull>), dim3(tiles), dim3(L::kThreads), 0, s, a);
+    if constexpr (L::kPar > 1) {
+        int n_cu = 0;
+        if (hipError_t e = device_cu_count(&n_cu); e != hipSuccess) return e;
+        if (tiles <= L::kParTiles * n_cu) {
+            hipLaunchKernelGGL((stencil_kernel<T, D, TY, 1, L::kPar>), dim3(tiles), dim3(L::kThreads * L::kPar), 0, s, a);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((stencil_kernel<T, D, TY, L::kFull, 1>), dim3(tiles), dim3(L::kThreads), 0, s, a);
     return hipGetLastError();
 }
 

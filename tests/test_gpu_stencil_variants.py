@@ -1,0 +1,44 @@
+"""The generic stencil's forms at the sizes where the choice between them changes: the same
+cells computed with heads in parallel (one small grid) and one head after the other (a batch
+of copies of that grid, past the rule's tile counts) give the same bits, output and conserved
+sums, since both mix the heads in the same order; the small grid is checked against the
+oracle elsewhere (test_gpu_parity)."""
+import numpy as np
+import pytest
+
+from slime_amd import Pseudopod, make_params, make_state
+from slime_amd.synthetic import CAConfig
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.mark.parametrize("dtype,D,G,copies,per_cell", [
+    ("fp32", 8, 8, 600, False), ("bf16", 8, 16, 160, True),    # 2 and 8 tiles; 1200 and 1280
+    ("fp32", 16, 16, 40, True), ("bf16", 16, 24, 40, False),   # 8 and 18 tiles; 320 and 720
+    ("fp32", 32, 40, 6, False), ("bf16", 32, 16, 40, True),    # 50 and 8 tiles; 300 and 320
+])
+def test_parallel_heads_match_serial_heads(dtype, D, G, copies, per_cell):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    print(f"[case] {dtype} D={D} G={G} x{copies} per_cell={per_cell}", flush=True)
+    cfg = CAConfig("var", B=1, G=G, H=8, D=D, dtype=dtype, steps=1, w_std=0.1, growth_per_cell=per_cell)
+    p = make_params(cfg, seed=3)
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    x = torch.from_numpy(make_state(cfg, seed=4)).cuda().to(dt)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    P, I, V = (torch.randn(x.shape, generator=g, device="cuda").to(dt) for _ in range(3))
+    outs, masses = [], []
+    for B in (1, copies):
+        with Pseudopod(B, G, 8, D, dtype, growth_per_cell=per_cell) as e:
+            e.set_params(p)
+            y = e.flow_lenia(*(t.expand(B, -1, -1, -1).contiguous() for t in (x, P, I, V)))
+            mi, mo = e.mass()
+            outs.append(y)
+            masses.append((mi, mo))
+    assert torch.isfinite(outs[0].float()).all()
+    assert torch.equal(outs[1], outs[0].expand_as(outs[1]))
+    for one, many in zip(masses[0], masses[1]):
+        # fp64 sums of the same lane sums, trees of another shape: 2^-48 of the sums' size
+        np.testing.assert_allclose(many, np.broadcast_to(one, many.shape), rtol=2.0 ** -40)
