@@ -288,12 +288,14 @@ int run_project(slime_ca* h, const void* x, const float* x_scale, void* P, void*
 }
 
 // S2-S6 plus the mass partials and S7 finalize: y_raw gets the unscaled output,
-// out_scale the per-(b, head) conservation factor.
+// out_scale the per-(b, head) conservation factor. With y_out (a call's last step) the
+// factor is also applied, y_out = out_scale * y_raw in the storage type.
 // loss_T, loss_part: the backward's tape step on the MFMA stencil (bf16, D = 64), which
 // also sums Y^2, Y T and T^2 per (b, head, tile) into loss_part (StencilArgs).
 int run_stencil(slime_ca* h, const void* x, const float* x_scale, const void* P, const void* I,
                 const void* V, void* y_raw, int y_f32, float* out_scale, hipStream_t s,
-                double* out_scale64 = nullptr, const void* loss_T = nullptr, double* loss_part = nullptr) {
+                double* out_scale64 = nullptr, const void* loss_T = nullptr, double* loss_part = nullptr,
+                void* y_out = nullptr) {
     const slime_ca_config& c = h->cfg;
     StencilArgs a{};
     a.X = x;
@@ -323,8 +325,12 @@ int run_stencil(slime_ca* h, const void* x, const float* x_scale, const void* P,
     HIP_TRY(timed(h, h->stencil_ev, s, [&] { return launch_stencil(c.dtype, a, s); }));
     if (c.conservation == 1)
         HIP_TRY(launch_cell_conserve(c.dtype, x, x_scale, y_raw, y_f32, h->part_out, c.B, c.G, c.D, s));
-    HIP_TRY(launch_mass_finalize(h->part_in, h->part_out, c.B * c.H, h->tiles, h->mass_in,
-                                 h->mass_out, out_scale, out_scale64, s));
+    if (y_out)
+        HIP_TRY(launch_mass_rescale(c.dtype, h->part_in, h->part_out, h->tiles, h->mass_in, h->mass_out,
+                                    out_scale, y_raw, y_f32, y_out, c.B, c.G, h->C, c.D, s));
+    else
+        HIP_TRY(launch_mass_finalize(h->part_in, h->part_out, c.B * c.H, h->tiles, h->mass_in,
+                                     h->mass_out, out_scale, out_scale64, s));
     return SLIME_OK;
 }
 
@@ -509,7 +515,8 @@ int slime_ca_set_params(slime_ca* h, const slime_ca_params* p) {
                               hipMemcpyHostToDevice));
         }
     }
-    // The unscaled copy that the GEMMs read: laid out once here, on the stream the uploads use.
+    // The unscaled copy that the GEMMs read: laid out once here, on the stream of the uploads,
+    // whose later copies wait for it.
     {
         WeightPrepArgs w{};
         w.Wtm = h->Wtm;
@@ -520,7 +527,6 @@ int slime_ca_set_params(slime_ca* h, const slime_ca_params* p) {
         w.per_pod = 1;
         w.nplanes = 3;
         HIP_TRY(launch_weight_prep(c.dtype, w, nullptr));
-        HIP_TRY(hipStreamSynchronize(nullptr));
     }
     // [W_P | W_I | W_V] by input channel, for the backward's dX GEMM (uploaded by
     // slime_ca_backward when first needed).
@@ -575,11 +581,8 @@ int slime_ca_flow_lenia(slime_ca* h, const void* x_in, const void* P, const void
     const slime_ca_config& c = h->cfg;
     // The output is rescaled once from an fp32 copy, so a bf16 state is rounded once.
     void* raw = h->Sf ? static_cast<void*>(h->Sf) : h->S[0];
-    rc = run_stencil(h, x_in, nullptr, P, I, V, raw, h->Sf != nullptr, h->scale[0], s);
-    if (rc) return rc;
-    HIP_TRY(launch_rescale(c.dtype, raw, h->Sf != nullptr, h->scale[0], y_out, c.B, c.G, h->C,
-                           c.D, s));
-    return SLIME_OK;
+    return run_stencil(h, x_in, nullptr, P, I, V, raw, h->Sf != nullptr, h->scale[0], s, nullptr, nullptr,
+                       nullptr, y_out);
 }
 
 int slime_ca_step(slime_ca* h, const void* x_in, void* x_out, int n_steps, void* stream) {
@@ -603,7 +606,6 @@ int slime_ca_step(slime_ca* h, const void* x_in, void* x_out, int n_steps, void*
     // Intermediate outputs stay unscaled in the storage type: the next step applies
     // the conservation factor in fp32 as it reads them. The last step writes fp32
     // (bf16 state) so the final rescale rounds once.
-    int cur_f32 = 0;
     for (int i = 0; i < n_steps; ++i) {
         const bool last = i == n_steps - 1;
         const int y_f32 = last && h->Sf != nullptr;
@@ -611,13 +613,12 @@ int slime_ca_step(slime_ca* h, const void* x_in, void* x_out, int n_steps, void*
         float* ys = h->scale[i & 1];
         rc = run_project(h, cur, cur_scale, h->P, h->I, h->V, s);
         if (rc) return rc;
-        rc = run_stencil(h, cur, cur_scale, h->P, h->I, h->V, y, y_f32, ys, s);
+        rc = run_stencil(h, cur, cur_scale, h->P, h->I, h->V, y, y_f32, ys, s, nullptr, nullptr, nullptr,
+                         last ? x_out : nullptr);
         if (rc) return rc;
         cur = y;
-        cur_f32 = y_f32;
         cur_scale = ys;
     }
-    HIP_TRY(launch_rescale(c.dtype, cur, cur_f32, cur_scale, x_out, c.B, c.G, h->C, c.D, s));
     return SLIME_OK;
 }
 

@@ -124,6 +124,11 @@ hipError_t launch_cell_conserve(int dtype, const void* x, const float* scale, vo
 hipError_t launch_rescale(int dtype, const void* x, int x_f32, const float* scale, void* y, int B,
                           int G, int C, int D, hipStream_t s);
 
+// launch_mass_finalize and launch_rescale together, in one launch for small grids.
+hipError_t launch_mass_rescale(int dtype, const double* part_in, const double* part_out, int tiles, double* mass_in,
+                               double* mass_out, float* scale, const void* x, int x_f32, void* y, int B, int G, int C,
+                               int D, hipStream_t s);
+
 // ---- E1-E5 fitness --------------------------------------------------------------------
 struct FitnessArgs {
     const void* hist;   // state 0 of the history, each state [B][G][G][C]

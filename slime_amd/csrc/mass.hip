@@ -41,53 +41,62 @@ hipError_t device_cu_count(int* n_cu) {
 
 namespace {
 
-__global__ __launch_bounds__(64) void mass_finalize_kernel(const double* part_in,
-                                                           const double* part_out, int tiles,
-                                                           double* mass_in, double* mass_out,
-                                                           float* scale_out, double* scale64_out) {
-    // One wave per (b, h): lanes stride over tiles, then a fixed-shape tree.
-    __shared__ double s_in[64], s_out[64];
-    const int bh = blockIdx.x, lane = threadIdx.x;
+// The S7 factor of one (b, h) from its sums, as the pair hi + lo.
+struct Factor {
+    float hi, lo;
+};
+__device__ __forceinline__ Factor factor_of(double in, double out) {
+    const double r = fabs(out) > 1e-6 ? in / out : 1.0;
+    const float hi = (float)r;
+    return {hi, (float)(r - (double)hi)};
+}
+
+// Sum of a wave's values, lane l + w added to lane l for w = 32, 16, ... 1: in lane 0.
+__device__ __forceinline__ double wave_tree(double v) {
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) v += __shfl_down(v, w, 64);
+    return v;
+}
+
+struct MassOut {
+    double *mass_in, *mass_out;
+    float* scale;      // [2][BH]
+    double* scale64;   // may be nullptr
+};
+__device__ __forceinline__ void write_factor(const MassOut& m, int bh, int BH, double in, double out) {
+    const Factor f = factor_of(in, out);
+    const double r = (double)f.hi + (double)f.lo;
+    m.scale[bh] = f.hi;
+    m.scale[BH + bh] = f.lo;
+    if (m.scale64) m.scale64[bh] = r;
+    m.mass_in[bh] = in;
+    m.mass_out[bh] = r * out;
+}
+
+// One workgroup per (b, h): threads stride over the tiles, then fixed trees over lanes and
+// waves (with at most 64 tiles the sums of one wave, as mass_rescale_kernel forms them).
+// Latency bound: 8192 tiles (512^2) 8 us, 60 us in one wave.
+__global__ __launch_bounds__(256) void mass_finalize_kernel(const double* part_in, const double* part_out,
+                                                            int tiles, MassOut m) {
+    __shared__ double s[2][4];
+    const int bh = blockIdx.x, tid = threadIdx.x;
     double si = 0.0, so = 0.0;
-    for (int t = lane; t < tiles; t += 64) {
+#pragma unroll 4
+    for (int t = tid; t < tiles; t += 256) {
         si += part_in[(long long)bh * tiles + t];
         so += part_out[(long long)bh * tiles + t];
     }
-    s_in[lane] = si;
-    s_out[lane] = so;
+    si = wave_tree(si);
+    so = wave_tree(so);
+    if ((tid & 63) == 0) s[0][tid >> 6] = si, s[1][tid >> 6] = so;
     __syncthreads();
-    for (int w = 32; w > 0; w >>= 1) {
-        if (lane < w) {
-            s_in[lane] += s_in[lane + w];
-            s_out[lane] += s_out[lane + w];
-        }
-        __syncthreads();
-    }
-    if (lane == 0) {
-        const double in = s_in[0], out = s_out[0];
-        const double r = fabs(out) > 1e-6 ? in / out : 1.0;
-        const float hi = (float)r, lo = (float)(r - (double)hi);
-        scale_out[bh] = hi;
-        scale_out[gridDim.x + bh] = lo;
-        if (scale64_out) scale64_out[bh] = (double)hi + (double)lo;
-        mass_in[bh] = in;
-        mass_out[bh] = ((double)hi + (double)lo) * out;
-    }
+    if (tid == 0)
+        write_factor(m, bh, gridDim.x, s[0][0] + s[0][1] + s[0][2] + s[0][3], s[1][0] + s[1][1] + s[1][2] + s[1][3]);
 }
 
+// Four consecutive elements times the factor; they never straddle two heads (D >= 8).
 template <typename TI, typename T>
-__global__ __launch_bounds__(256) void rescale_kernel(const TI* x, const float* scale, T* y,
-                                                      long long nquads, int C, int D,
-                                                      long long cells_per_batch, int bh_total) {
-    // Four consecutive elements per thread; they never straddle two heads (D >= 8).
-    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= nquads) return;
-    const long long e0 = q * 4;
-    const long long cell = e0 / C;
-    const int ch = (int)(e0 - cell * C);
-    const int b = (int)(cell / cells_per_batch);
-    const long long si = (long long)b * (C / D) + ch / D;
-    const float s = scale[si], s_lo = scale[bh_total + si];
+__device__ __forceinline__ void rescale_quad(const TI* x, T* y, long long q, float s, float s_lo) {
     float v[4];
     if constexpr (sizeof(TI) == 2) {
         const uint2 w = reinterpret_cast<const uint2*>(x)[q];
@@ -105,13 +114,61 @@ __global__ __launch_bounds__(256) void rescale_kernel(const TI* x, const float* 
     }
 }
 
+template <typename TI, typename T>
+__global__ __launch_bounds__(256) void rescale_kernel(const TI* x, const float* scale, T* y,
+                                                      long long nquads, int C, int D,
+                                                      long long cells_per_batch, int bh_total) {
+    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= nquads) return;
+    const long long e0 = q * 4;
+    const long long cell = e0 / C;
+    const int ch = (int)(e0 - cell * C);
+    const int b = (int)(cell / cells_per_batch);
+    const long long si = (long long)b * (C / D) + ch / D;
+    rescale_quad(x, y, q, scale[si], scale[bh_total + si]);
+}
+
+// mass_finalize_kernel and rescale_kernel in one launch, for grids of at most 64 tiles: every
+// workgroup (1024 elements of one batch entry, all heads: 64 G^2 elements are a multiple)
+// forms the entry's eight factors from the partials itself, two heads per wave, and the
+// entry's first workgroup writes them. One wave's tree over the tiles, so the factors have
+// the bits of mass_finalize_kernel.
+template <typename TI, typename T>
+__global__ __launch_bounds__(256) void mass_rescale_kernel(const double* part_in, const double* part_out, int tiles,
+                                                           MassOut m, const TI* x, T* y, int C, int D,
+                                                           int wgs_per_batch, int BH) {
+    __shared__ Factor f[kHeads];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int b = blockIdx.x / wgs_per_batch;
+    double si[2], so[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const long long at = ((long long)b * kHeads + 2 * wave + u) * tiles + lane;
+        si[u] = lane < tiles ? part_in[at] : 0.0;
+        so[u] = lane < tiles ? part_out[at] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int h = 2 * wave + u;
+        const double in = wave_tree(si[u]), out = wave_tree(so[u]);
+        if (lane == 0) {
+            f[h] = factor_of(in, out);
+            if (blockIdx.x % wgs_per_batch == 0) write_factor(m, b * kHeads + h, BH, in, out);
+        }
+    }
+    __syncthreads();
+    const long long q = (long long)blockIdx.x * 256 + tid;
+    const Factor k = f[(int)(q * 4 % C) / D];
+    rescale_quad(x, y, q, k.hi, k.lo);
+}
+
 }  // namespace
 
 hipError_t launch_mass_finalize(const double* part_in, const double* part_out, int BH, int tiles,
                                 double* mass_in, double* mass_out, float* scale_out,
                                 double* scale64_out, hipStream_t s) {
-    hipLaunchKernelGGL(mass_finalize_kernel, dim3(BH), dim3(64), 0, s, part_in, part_out, tiles,
-                       mass_in, mass_out, scale_out, scale64_out);
+    hipLaunchKernelGGL(mass_finalize_kernel, dim3(BH), dim3(256), 0, s, part_in, part_out, tiles,
+                       MassOut{mass_in, mass_out, scale_out, scale64_out});
     return hipGetLastError();
 }
 
@@ -233,6 +290,36 @@ hipError_t launch_rescale(int dtype, const void* x, int x_f32, const float* scal
                            static_cast<const float*>(x), scale, static_cast<float*>(y), nquads, C,
                            D, cells, bh);
     return hipGetLastError();
+}
+
+namespace {
+template <typename TI, typename T>
+hipError_t launch_fused_t(const double* part_in, const double* part_out, int tiles, const MassOut& m, const void* x,
+                          void* y, int B, int C, int D, int wgs, hipStream_t s) {
+    hipLaunchKernelGGL((mass_rescale_kernel<TI, T>), dim3((unsigned)(B * wgs)), dim3(256), 0, s, part_in, part_out,
+                       tiles, m, static_cast<const TI*>(x), static_cast<T*>(y), C, D, wgs, B * kHeads);
+    return hipGetLastError();
+}
+}  // namespace
+
+// One launch while the partials that every workgroup reads again stay small beside the
+// data: at most 64 tiles, and 16 MiB of partial reads in all. Small grids are bound by
+// their launches (a step of 32^2 x 64 fp32: 20.9 -> 17.1 us); a batch of 64 grids of 32^2 x
+// 512 would read 134 MB of partials beside 201 MB of data.
+hipError_t launch_mass_rescale(int dtype, const double* part_in, const double* part_out, int tiles, double* mass_in,
+                               double* mass_out, float* scale, const void* x, int x_f32, void* y, int B, int G, int C,
+                               int D, hipStream_t s) {
+    const long long wgs = (long long)G * G * C / 1024;
+    const MassOut m{mass_in, mass_out, scale, nullptr};
+    if (tiles <= 64 && B * wgs * tiles * 2 * kHeads * 8 <= (16 << 20)) {
+        if (dtype == 1 && x_f32)
+            return launch_fused_t<float, bf16_t>(part_in, part_out, tiles, m, x, y, B, C, D, (int)wgs, s);
+        if (dtype == 1) return launch_fused_t<bf16_t, bf16_t>(part_in, part_out, tiles, m, x, y, B, C, D, (int)wgs, s);
+        return launch_fused_t<float, float>(part_in, part_out, tiles, m, x, y, B, C, D, (int)wgs, s);
+    }
+    const hipError_t e =
+        launch_mass_finalize(part_in, part_out, B * kHeads, tiles, mass_in, mass_out, scale, nullptr, s);
+    return e != hipSuccess ? e : launch_rescale(dtype, x, x_f32, scale, y, B, G, C, D, s);
 }
 
 }  // namespace slime
