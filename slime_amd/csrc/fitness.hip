@@ -325,7 +325,7 @@ __device__ __forceinline__ void lds_barrier() {
 // (failed_attempts/pseudopod.cu:391-436) and skips |a_pq| <= 1e-6. That absolute
 // threshold makes the converged diagonal depend on the order when the Gram is nearly
 // singular, so the order is kept. What bounds it is the chain of a rotation's fp64
-// operations (four hardware estimates in a row with their refinements, ~600 cycles), so
+// operations (two hardware estimates in a row with their refinements, ~450 cycles), so
 // the solve runs the cyclic order as a wave front (jacobi_wave.hpp): the up to D / 2
 // rotations of a step share no index, commute, and run in the lanes of one wave, D steps
 // to a sweep instead of D (D - 1) / 2 rotations; every rotation sees the values that the
@@ -343,9 +343,10 @@ __device__ __forceinline__ void lds_barrier() {
 // the one that rotated nothing (every later sweep would repeat it up to the limit, and
 // 30 sweeps are reported, as the reference runs them), or the 30th.
 //
-// Measured on 128 Grams of 64 x 64 (16 pods x 8 heads, ~11.7k rotations each): 377 us,
-// 2920 us as one rotation at a time. A step takes the chain's latency plus one LDS round
-// trip and the barrier; the update waves (one item each) stay below that.
+// Measured on 128 Grams of 64 x 64 (16 pods x 8 heads, ~11.7k rotations each): 315 us,
+// 2920 us as one rotation at a time. A step (~1300 cycles) is shared between the chain and
+// the update's LDS traffic (48 KB of the CU's 128 B per cycle): halving the chain's hardware
+// estimates took 5 %, two or four items per update thread cost 5 and 14 %.
 constexpr int kFinUpdate = 512;                // threads that apply the rotations
 constexpr int kFinThreads = 64 + kFinUpdate;   // wave 0 computes them
 
@@ -396,26 +397,27 @@ __global__ __launch_bounds__(kFinThreads) void fitness_finalize_kernel(FitnessAr
     int cur = 0;
     if (tid >= 64) {
         // ---- apply step T to the matrix ----------------------------------------------------
-        // One item per thread (D = 64), and threads 0 .. S - 1 a rotated pair's own element.
+        // One item (the block of slots d1 and d2) per thread, and in the first S threads the own
+        // element of slot d1's pair.
         static_assert(S * S / 2 <= kFinUpdate, "one work item per thread");
         const int u = tid - 64;
-        int d1, d2;
-        const bool act = u < S * S / 2 && item(u, S, &d1, &d2), pairs = u < S;
+        const int d1 = u & (S - 1), o = u / S + 1, d2 = (d1 + o) & (S - 1);  // jacobi_wave::item
+        const bool act = o <= S / 2 && (o < S / 2 || d1 < S / 2), pairs = u < S;
         for (int T = 0;; ++T) {
             const int sig = T & (D - 1);
             const double* M = A[cur];
             double* W = A[cur ^ 1];
             const double2* r = cs[T & 1];
-            int i1 = 0, j1 = 1, i2 = 0, j2 = 1, pi = 0, pj = 1;
-            if (act) slot(sig, d1, D, &i1, &j1), slot(sig, d2, D, &i2, &j2);
-            if (pairs) slot(sig, u, D, &pi, &pj);
+            int i1, j1, i2, j2;
+            slot(sig, d1, D, &i1, &j1);
+            slot(sig, d2, D, &i2, &j2);
             const int ea = upper(i1, i2, D), eb = upper(i1, j2, D), ec = upper(j1, i2, D), ed = upper(j1, j2, D);
-            const int ep = upper(pi, pj, D);
+            const int ep = upper(i1, j1, D);
             // all reads at once, before the step is known to rotate anything
             const int fl = flag[T & 1];
             const double2 r1 = r[i1], r2 = r[i2];
             const double a = M[ea], b = M[eb], c = M[ec], d = M[ed];
-            const double ps = r[pi].y, pv = M[ep];
+            const double own = M[ep];
             if (fl == 2) return;
             if (fl) {
                 if (act) {
@@ -426,7 +428,7 @@ __global__ __launch_bounds__(kFinThreads) void fitness_finalize_kernel(FitnessAr
                     W[ec] = r2.x * cr + r2.y * dr;
                     W[ed] = r2.x * dr - r2.y * cr;
                 }
-                if (pairs) W[ep] = ps != 0.0 ? 0.0 : pv;
+                if (pairs) W[ep] = r1.y != 0.0 ? 0.0 : own;  // a rotated pair's element is zero now
                 cur ^= 1;
             }
             lds_barrier();
@@ -551,7 +553,7 @@ __global__ __launch_bounds__(kFinThreads) void fitness_finalize_kernel(FitnessAr
 #pragma unroll 8
     for (int i = 0; i < D; ++i) sum += sv[i];
     if (own) {
-        const double pr = sv[lane] / (sum + 1e-7);
+        const double pr = div_rn(sv[lane], sum + 1e-7);
         term[lane] = -pr * log(pr + 1e-7);
     }
     lds_order();
