@@ -74,3 +74,24 @@ def test_projections_match_fp64(dtype, B, G, D, pods, chain):
         ins = [xs[b], P[b] if chain else x[b], I[b] if chain else x[b]]
         for got, src, wk, act, name in zip((P, I, V), ins, w, (1, 2, 0), "PIV"):
             _check(got[b].reshape(G * G, C), src.reshape(G * G, C), wk, act, bf16, (name, b))
+
+
+@pytest.mark.parametrize("dtype,G,D", [("fp32", 24, 16), ("bf16", 40, 64), ("fp32", 16, 64)])
+def test_project_takes_a_state_inside_another_buffer(dtype, G, D):
+    """A contiguous state that starts one element into its buffer, which no 16-byte load fits."""
+    C, bf16 = 8 * D, dtype == "bf16"
+    rng = np.random.default_rng(D)
+    p = {k: rng.normal(0, 0.1, (1, C, C)).astype(np.float32) for k in ("WP", "WI", "WV")}
+    if bf16:
+        p = {k: round_bf16(v) for k, v in p.items()}
+    p.update(K=np.zeros((1, 8, 9)), M=np.eye(8)[None], mu=np.full((1, 8), 0.2), sigma=np.full((1, 8), 0.05))
+    dt = torch.bfloat16 if bf16 else torch.float32
+    buf = torch.randn(1 + G * G * C, generator=torch.Generator(device="cuda").manual_seed(1), device="cuda").to(dt)
+    x = buf[1:].view(1, G, G, C)
+    assert x.is_contiguous() and x.data_ptr() % 16
+    with Pseudopod(1, G, 8, D, dtype) as e:
+        e.set_params(p)
+        outs = e.project(x)
+        torch.cuda.synchronize()
+    for got, k, act in zip(outs, ("WP", "WI", "WV"), (1, 2, 0)):
+        _check(got.reshape(G * G, C), x.reshape(G * G, C), torch.from_numpy(p[k][0]).cuda(), act, bf16, k)
