@@ -322,9 +322,10 @@ int run_stencil(slime_ca* h, const void* x, const float* x_scale, const void* P,
     a.growth_fn = c.growth_fn;
     a.T = loss_T;
     a.loss_part = loss_part;
+    const bool conserve_pass = c.conservation == 1 && c.dtype == SLIME_BF16 && c.D == 64;
+    a.cell_conserve = c.conservation == 1 && !conserve_pass;
     HIP_TRY(timed(h, h->stencil_ev, s, [&] { return launch_stencil(c.dtype, a, s); }));
-    if (c.conservation == 1)
-        HIP_TRY(launch_cell_conserve(c.dtype, x, x_scale, y_raw, y_f32, h->part_out, c.B, c.G, c.D, s));
+    if (conserve_pass) HIP_TRY(launch_cell_conserve(x, x_scale, y_raw, y_f32, h->part_out, c.B, c.G, s));
     if (y_out)
         HIP_TRY(launch_mass_rescale(c.dtype, h->part_in, h->part_out, h->tiles, h->mass_in, h->mass_out,
                                     out_scale, y_raw, y_f32, y_out, c.B, c.G, h->C, c.D, s));

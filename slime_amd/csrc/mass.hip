@@ -191,7 +191,8 @@ hipError_t launch_fill_f64(double* p, int n, double v, hipStream_t s) {
 // deferred per-(b, head) factor applied (hi + lo), as the stencil reads it. One
 // workgroup per stencil tile (4 x 8 cells) rewrites that tile's part_out sums from the
 // renormalised values, so the per-(b, head) factor S7 then computes from the partials
-// is 1 up to rounding (or corrects the cells the guard skipped).
+// is 1 up to rounding (or corrects the cells the guard skipped). The generic stencil does
+// this itself; this pass serves the matrix-core one (bf16, D = 64).
 namespace {
 constexpr int kCcTileY = 4, kCcTileX = 8, kCcCells = kCcTileY * kCcTileX;
 
@@ -246,29 +247,19 @@ __global__ __launch_bounds__(256) void cell_conserve_kernel(const TX* X, const f
     }
 }
 
-template <typename TX, typename TY>
-hipError_t launch_cc_t(const void* x, const float* scale, void* y, double* part_out, int B, int G, int D,
-                       hipStream_t s) {
-    const dim3 grid((unsigned)(B * (G / kCcTileY) * (G / kCcTileX)));
-    const TX* xp = static_cast<const TX*>(x);
-    TY* yp = static_cast<TY*>(y);
-    switch (D) {
-        case 8: hipLaunchKernelGGL((cell_conserve_kernel<TX, TY, 8>), grid, dim3(256), 0, s, xp, scale, yp, part_out, B, G); break;
-        case 16: hipLaunchKernelGGL((cell_conserve_kernel<TX, TY, 16>), grid, dim3(256), 0, s, xp, scale, yp, part_out, B, G); break;
-        case 32: hipLaunchKernelGGL((cell_conserve_kernel<TX, TY, 32>), grid, dim3(256), 0, s, xp, scale, yp, part_out, B, G); break;
-        case 64: hipLaunchKernelGGL((cell_conserve_kernel<TX, TY, 64>), grid, dim3(256), 0, s, xp, scale, yp, part_out, B, G); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
 }  // namespace
 
-hipError_t launch_cell_conserve(int dtype, const void* x, const float* scale, void* y, int y_f32,
-                                double* part_out, int B, int G, int D, hipStream_t s) {
-    if (dtype == 1)
-        return y_f32 ? launch_cc_t<bf16_t, float>(x, scale, y, part_out, B, G, D, s)
-                     : launch_cc_t<bf16_t, bf16_t>(x, scale, y, part_out, B, G, D, s);
-    return launch_cc_t<float, float>(x, scale, y, part_out, B, G, D, s);
+hipError_t launch_cell_conserve(const void* x, const float* scale, void* y, int y_f32, double* part_out, int B, int G,
+                                hipStream_t s) {
+    const dim3 grid((unsigned)(B * (G / kCcTileY) * (G / kCcTileX)));
+    const bf16_t* xp = static_cast<const bf16_t*>(x);
+    if (y_f32)
+        hipLaunchKernelGGL((cell_conserve_kernel<bf16_t, float, 64>), grid, dim3(256), 0, s, xp, scale,
+                           static_cast<float*>(y), part_out, B, G);
+    else
+        hipLaunchKernelGGL((cell_conserve_kernel<bf16_t, bf16_t, 64>), grid, dim3(256), 0, s, xp, scale,
+                           static_cast<bf16_t*>(y), part_out, B, G);
+    return hipGetLastError();
 }
 
 hipError_t launch_rescale(int dtype, const void* x, int x_f32, const float* scale, void* y, int B,

@@ -166,6 +166,13 @@ __device__ __forceinline__ float group_sum(float v) {
 }
 
 template <int kN>
+__device__ __forceinline__ float group_sum16(float v) {  // kN up to 16
+    v = group_sum<(kN < 8 ? kN : 8)>(v);
+    if constexpr (kN >= 16) v += dpp_f32<0x140>(v);  // row_mirror
+    return v;
+}
+
+template <int kN>
 __device__ __forceinline__ float group_max(float v) {
     if constexpr (kN >= 2) v = fmaxf(v, dpp_f32<0xB1>(v));
     if constexpr (kN >= 4) v = fmaxf(v, dpp_f32<0x4E>(v));
@@ -202,11 +209,17 @@ __device__ __forceinline__ void fold_half(double (&v)[16], int lane, int bit) {
 // the same order and with the same bits; a grid of few tiles then has kPar times the
 // wavefronts and 1 / kPar of the serial chain. launch_tdy picks.
 //
+// kCons: conservation 1 (slime/core/pseudopod.cu:160-165,196-203): each cell's output head is
+// multiplied by the ratio of its input's head sum to its own (1 when the latter's magnitude
+// is at most 1e-6) before it is rounded and stored. The sums over a head's channels run over
+// the lanes that hold them and meet in LDS. 1 x 128^2 x 512 fp32: 27 us for a pass of its own,
+// 4 us here (32 -> 36 us).
+//
 // What bounds it: VALU and LDS issue with four waves per SIMD (two cells per thread keep
 // the output accumulators at 32 and the kernel at 128 registers).
 // Measured: 1 x 128^2 x 512 fp32 57 -> 37 us (4.6 TB/s of the five planes; one workgroup of 4
 // waves per CU and four cells per thread before), 8 x 104^2 x 256 bf16 85 -> 76 us.
-template <typename T, int D, typename TY, int kBufs, int kPar>
+template <typename T, int D, typename TY, int kBufs, int kPar, bool kCons>
 __global__ __launch_bounds__((Layout<T, D>::kThreads * kPar), (kPar == 1 ? 4 : 2))
 void stencil_kernel(StencilArgs a) {
     using L = Layout<T, D>;
@@ -220,6 +233,11 @@ void stencil_kernel(StencilArgs a) {
     __shared__ __attribute__((aligned(16))) float sAtt[kPar * kTileCells * kAStride];
     __shared__ __attribute__((aligned(16))) float sMS[H * kTileCells * 2];
     __shared__ double sR[kPar > 1 ? L::kWaves * kPar * 2 * kRounds : L::kThreads];
+    // Conservation per cell: head sums of the input and the output, in kParts parts of up to
+    // 16 lanes, and the factors.
+    constexpr int kLanes = kPairs < 16 ? kPairs : 16, kParts = kPairs / kLanes;
+    __shared__ float sXS[kCons ? H * kTileCells * kParts : 1], sYS[kCons ? H * kTileCells * kParts : 1];
+    __shared__ __attribute__((aligned(16))) float sF[kCons ? kTileCells * H : 1];  // [cell][head]
 
     const int gw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scalar LDS addresses
     const int group = kPar > 1 ? gw / L::kWaves : 0;                  // of heads
@@ -346,6 +364,38 @@ void stencil_kernel(StencilArgs a) {
     constexpr float kLog2e = 1.4426950408889634f;
     const Growth gc = growth_args(a.growth_fn, 0.f, 1.f, a.dt);  // c0, c1, c2 of the function
 
+    // This thread's cells' sums over head h's channels, in parts.
+    auto head_sums = [&](float* dst, int h, const float (&v)[kRun][2]) {
+#pragma unroll
+        for (int x = 0; x < kRun; ++x) {
+            const float sum = group_sum16<kLanes>(v[x][0] + v[x][1]);
+            if (cp % kLanes == 0) dst[(h * kTileCells + ry * kTileX + rx0 + x) * kParts + cp / kLanes] = sum;
+        }
+    };
+    // The factors of every (cell, head) from the sums in LDS, which every thread has written.
+    auto factors = [&] {
+        lds_barrier();
+        for (int i = threadIdx.x; i < kTileCells * H; i += kAll) {
+            const int cell = i / H, h = i % H;
+            float sx = 0.f, sy = 0.f;
+#pragma unroll
+            for (int u = 0; u < kParts; ++u) {
+                sx += sXS[(h * kTileCells + cell) * kParts + u];
+                sy += sYS[(h * kTileCells + cell) * kParts + u];
+            }
+            sF[i] = fabsf(sy) > 1e-6f ? sx / sy : 1.0f;
+        }
+        lds_barrier();
+    };
+    auto apply = [&](int o, float (&v)[kRun][2]) {
+#pragma unroll
+        for (int x = 0; x < kRun; ++x) {
+            const float f = sF[(ry * kTileX + rx0 + x) * H + o];
+            v[x][0] *= f;
+            v[x][1] *= f;
+        }
+    };
+
 #pragma unroll 1
     for (int r = 0; r < kRounds; ++r) {
         const int h = r * kPar + group;
@@ -443,6 +493,10 @@ void stencil_kernel(StencilArgs a) {
                 }
             }
         }
+        if constexpr (kCons) {
+            head_sums(sXS, h, xc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         {
             const unsigned char* pv = buf + L::offV + pbase;
             float2 w[3][kRun + 2];
@@ -515,20 +569,27 @@ void stencil_kernel(StencilArgs a) {
         for (int r = 0; r < kRounds; ++r) sZ[(r * kPar + group) * L::kThreads + tid] = zr[r];
         lds_barrier();
         // This group's outputs o = group * kRounds + r.
+        float v[kRounds][kRun][2] = {};
 #pragma unroll
         for (int r = 0; r < kRounds; ++r) {
             const int o = group * kRounds + r;
-            float v[kRun][2] = {};
 #pragma unroll
             for (int h = 0; h < H; ++h) {
                 const float4 z = sZ[h * L::kThreads + tid];
                 const float mw = sMW[h * H + o];
-                v[0][0] = __builtin_fmaf(mw, z.x, v[0][0]);
-                v[0][1] = __builtin_fmaf(mw, z.y, v[0][1]);
-                v[1][0] = __builtin_fmaf(mw, z.z, v[1][0]);
-                v[1][1] = __builtin_fmaf(mw, z.w, v[1][1]);
+                v[r][0][0] = __builtin_fmaf(mw, z.x, v[r][0][0]);
+                v[r][0][1] = __builtin_fmaf(mw, z.y, v[r][0][1]);
+                v[r][1][0] = __builtin_fmaf(mw, z.z, v[r][1][0]);
+                v[r][1][1] = __builtin_fmaf(mw, z.w, v[r][1][1]);
             }
-            const double sy = wave_sum64(store(o, v)), sx = wave_sum64(xin[r]);
+            if constexpr (kCons) head_sums(sYS, o, v[r]);
+        }
+        if constexpr (kCons) factors();
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) {
+            const int o = group * kRounds + r;
+            if constexpr (kCons) apply(o, v[r]);
+            const double sy = wave_sum64(store(o, v[r])), sx = wave_sum64(xin[r]);
             if (lane == 0) {
                 sR[(gw * kRounds + r) * 2] = sx;
                 sR[(gw * kRounds + r) * 2 + 1] = sy;
@@ -545,6 +606,19 @@ void stencil_kernel(StencilArgs a) {
             dst[((long long)b * H + j) * tpb + tile] = sum;
         }
     } else {
+        if constexpr (kCons) {
+#pragma unroll
+            for (int o = 0; o < H; ++o) {
+                head_sums(sYS, o, y[o]);
+                __builtin_amdgcn_sched_barrier(0);  // one output's lane sums at a time: registers
+            }
+            factors();
+#pragma unroll
+            for (int o = 0; o < H; ++o) {
+                apply(o, y[o]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
         // The butterfly leaves lane l holding its 16-lane row's sum of value l & 15.
         double red[16];  // [0, 8): sum of scaled X per head; [8, 16): sum of stored Y
 #pragma unroll
@@ -1249,7 +1323,7 @@ __global__ __launch_bounds__(mf::kThreads, 2) void stencil_mfma_kernel(StencilAr
 //           fp32 162 tiles 14.4 / 8.2, 576 tiles 18.3 / 23.5
 //   D = 32  fp32 162 tiles 16.2 / 11.8, 288 tiles 19.1 / 23.0
 //   D = 64  fp32 32 tiles 18.5 / 18.2, 162 tiles 19.4 / 20.6: never
-template <typename T, int D, typename TY>
+template <typename T, int D, typename TY, bool kCons>
 hipError_t launch_tdy(const StencilArgs& a, hipStream_t s) {
     using L = Layout<T, D>;
     const int tiles = a.B * (a.G / kTileY) * (a.G / kTileX);
@@ -1257,11 +1331,11 @@ hipError_t launch_tdy(const StencilArgs& a, hipStream_t s) {
         int n_cu = 0;
         if (hipError_t e = device_cu_count(&n_cu); e != hipSuccess) return e;
         if (tiles <= L::kParTiles * n_cu) {
-            hipLaunchKernelGGL((stencil_kernel<T, D, TY, 1, L::kPar>), dim3(tiles), dim3(L::kThreads * L::kPar), 0, s, a);
+            hipLaunchKernelGGL((stencil_kernel<T, D, TY, 1, L::kPar, kCons>), dim3(tiles), dim3(L::kThreads * L::kPar), 0, s, a);
             return hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((stencil_kernel<T, D, TY, L::kFull, 1>), dim3(tiles), dim3(L::kThreads), 0, s, a);
+    hipLaunchKernelGGL((stencil_kernel<T, D, TY, L::kFull, 1, kCons>), dim3(tiles), dim3(L::kThreads), 0, s, a);
     return hipGetLastError();
 }
 
@@ -1291,9 +1365,11 @@ hipError_t launch_mfma(const StencilArgs& a, hipStream_t s) {
 template <typename T, int D>
 hipError_t launch_td(const StencilArgs& a, hipStream_t s) {
     if constexpr (sizeof(T) == 2 && D == 64)
-        return a.y_f32 ? launch_mfma<float>(a, s) : launch_mfma<bf16_t>(a, s);
+        return a.cell_conserve ? hipErrorInvalidValue : a.y_f32 ? launch_mfma<float>(a, s) : launch_mfma<bf16_t>(a, s);
+    else if (a.cell_conserve)
+        return a.y_f32 ? launch_tdy<T, D, float, true>(a, s) : launch_tdy<T, D, T, true>(a, s);
     else
-        return a.y_f32 ? launch_tdy<T, D, float>(a, s) : launch_tdy<T, D, T>(a, s);
+        return a.y_f32 ? launch_tdy<T, D, float, false>(a, s) : launch_tdy<T, D, T, false>(a, s);
 }
 
 template <typename T>
