@@ -66,12 +66,12 @@ bool fits256(int dtype, const GemmArgs& a) {
 
 // The tile whose rounds over the card take least time: ceil(tiles / CUs) rounds of
 // tile^2 products each, at the rate the kernel reaches once it fills the card. Measured on
-// K = 512 forward products (TFLOP/s, 256 / 128 / 64 wide): bf16 915 / 690 / 560 at 65,536
-// rows or more, fp32 139 / 132 / 127; so the 256-wide kernel keeps what it tiles and
+// K = 512 forward products (TFLOP/s, 256 / 128 / 64 wide): bf16 915 / 730 / 610 at 65,536
+// rows, fp32 139 / 137 / 131; so the 256-wide kernel keeps what it tiles and
 // fills, and a batch that leaves its last round mostly empty goes to the smaller tiles:
-// 16,384 x 1536 x 512 in fp32 (384 tiles of 256 on 256 CUs) 272 -> 198 us in 1536 tiles of
+// 16,384 x 1536 x 512 in fp32 (384 tiles of 256 on 256 CUs) 272 -> 192 us in 1536 tiles of
 // 128; 8192 x 768 x 256 80 -> 31 us in tiles of 64. Shapes that 256 does not divide ran one
-// thread per output before (0.55 TFLOP/s): 73,984 x 1536 x 512 bf16 211 ms -> 0.18 ms.
+// thread per output before (0.55 TFLOP/s): 73,984 x 1536 x 512 bf16 211 ms -> 0.17 ms.
 int gemm_tile(int dtype, const GemmArgs& a, int n_cu) {
     int best = 0;
     double best_t = 0.0;
@@ -80,7 +80,7 @@ int gemm_tile(int dtype, const GemmArgs& a, int n_cu) {
         const long long rows = (a.rows_per_batch + tile - 1) / tile;  // per batch
         const long long ntiles = a.M / a.rows_per_batch * rows * (a.N / tile);
         const long long rounds = (ntiles + n_cu - 1) / n_cu;
-        const double rate = tile == 256 ? 1.0 : dtype == 1 ? (tile == 128 ? 0.75 : 0.6) : (tile == 128 ? 0.95 : 0.9);
+        const double rate = tile == 256 ? 1.0 : dtype == 1 ? (tile == 128 ? 0.8 : 0.66) : (tile == 128 ? 0.98 : 0.94);
         const double t = (double)rounds * tile * tile / rate;
         if (!best || t < best_t) best = tile, best_t = t;
     }

@@ -9,9 +9,11 @@
 // a tile moved back to the batch's end (gemm_small_addr.hpp) instead of a masked one.
 //
 // What bounds it: 128-wide bf16 tiles read 16 KiB of fragments from LDS per 128 cycles of
-// MFMAs, the LDS rate, and reach 690 TFLOP/s at 65,536 x 1536 x 512; fp32 tiles are bound
-// by the matrix cores (132 of 157 TFLOP/s); the smallest products (M <= 1024, K <= 192)
-// take 4 us, a launch and two memory round trips. The choice of tile: gemm_tile (gemm.hip).
+// MFMAs, the LDS rate, and reach 730 TFLOP/s at 65,536 x 1536 x 512; fp32 tiles are bound
+// by the matrix cores (137 of 157 TFLOP/s); the smallest products (M <= 1024, K <= 192)
+// take 4 us, a launch and two memory round trips. Three stages (48 KiB, three workgroups
+// per CU) instead of four: 16,384 x 1536 x 512 fp32 197 -> 192 us, 65,536 x 384 x 128 bf16
+// 20.5 -> 18.8 us, no shape slower. The choice of tile: gemm_tile (gemm.hip).
 #include "common.hpp"
 #include "gemm_small_addr.hpp"
 #include "kernels.hpp"
@@ -109,10 +111,10 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(GemmArgs g, voi
     for (int ks = 0; ks < kStages - 1 && ks < nk; ++ks) issue(ks, ks);
     int rd = 0, wr = kStages - 1;
     for (int ks = 0; ks < nk; ++ks) {
-        // The slabs issued after slab ks: kStages - 2, fewer at the end.
+        // The slabs issued after slab ks: one, none at the end.
         const int younger = nk - 1 - ks;
-        if (kStages > 3 && younger >= 2) wait_vm<2 * S::kDps>();
-        else if (younger >= 1) wait_vm<S::kDps>();
+        static_assert(kStages == 3, "one slab is younger than the one waited for");
+        if (younger >= 1) wait_vm<S::kDps>();
         else wait_vm<0>();
         lds_barrier();  // slab ks is in LDS; every wave has read slab ks - 1, whose stage is free
         if (ks + kStages - 1 < nk) issue(ks + kStages - 1, wr);
@@ -174,7 +176,7 @@ hipError_t launch_mode(int tile, const GemmArgs& a, void* aux, hipStream_t s) {
     const int ntiles = a.M / a.rows_per_batch * tiles_per_batch(tile, a.rows_per_batch) * (a.N / tile);
     const dim3 grid(8 * ((ntiles + 7) / 8));
     if (tile == 128)
-        hipLaunchKernelGGL((gemm_small_kernel<T, 128, 64, 4, kMode>), grid, dim3(kThreads), 0, s, a, aux);
+        hipLaunchKernelGGL((gemm_small_kernel<T, 128, 64, 3, kMode>), grid, dim3(kThreads), 0, s, a, aux);
     else
         hipLaunchKernelGGL((gemm_small_kernel<T, 64, 128, 3, kMode>), grid, dim3(kThreads), 0, s, a, aux);
     return hipGetLastError();
