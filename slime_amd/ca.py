@@ -29,9 +29,16 @@ def _ptr(t) -> ctypes.c_void_p:
 
 
 def _stream(stream=None) -> ctypes.c_void_p:
+    """The stream's handle; of the current stream of the current device when None. The raw
+    handle is asked for directly where torch offers it: the Stream object that
+    current_stream() builds takes 3 us, a fifth of a small step's call."""
+    if stream is not None:
+        return ctypes.c_void_p(stream.cuda_stream)
     torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(raw(torch.cuda.current_device()))
 
 
 class Pseudopod:
