@@ -516,8 +516,8 @@ int slime_ca_set_params(slime_ca* h, const slime_ca_params* p) {
                               hipMemcpyHostToDevice));
         }
     }
-    // The unscaled copy that the GEMMs read: laid out once here, on the stream of the uploads,
-    // whose later copies wait for it.
+    // The unscaled copy that the GEMMs read: laid out once here, on the stream of the uploads
+    // (waited for below, since a step may come on a stream that does not wait for that one).
     {
         WeightPrepArgs w{};
         w.Wtm = h->Wtm;
@@ -551,6 +551,7 @@ int slime_ca_set_params(slime_ca* h, const slime_ca_params* p) {
     HIP_TRY(hipMemcpy(h->mu, p->mu, ng * 4, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(h->sigma, p->sigma, ng * 4, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(h->M, p->M, (size_t)c.pods * c.H * c.H * 4, hipMemcpyHostToDevice));
+    HIP_TRY(hipStreamSynchronize(nullptr));
     h->params_set = true;
     return SLIME_OK;
 }

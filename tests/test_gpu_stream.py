@@ -16,3 +16,29 @@ def test_stream_handle_is_the_current_streams():
         assert _stream().value == s.cuda_stream
     assert _stream(s).value == s.cuda_stream
     assert (_stream().value or 0) == torch.cuda.current_stream().cuda_stream
+
+
+def test_new_parameters_reach_a_step_on_a_side_stream():
+    """set_params lays the weights out on the device; a projection that follows at once on a
+    stream of its own reads the new ones."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import numpy as np
+    from slime_amd import Pseudopod
+    G, D = 32, 64
+    C = 8 * D
+    rng = np.random.default_rng(5)
+    z = np.zeros
+    ca = Pseudopod(1, G, 8, D, "fp32", 0.1)
+    x = torch.from_numpy(rng.random((1, G, G, C), dtype=np.float32)).cuda()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    for s in (1.0, 2.0, 0.5, 4.0):  # W = s I: V = s X exactly, for powers of two
+        w = (s * np.eye(C, dtype=np.float32))[None]
+        ca.set_params(dict(WP=w, WI=w, WV=w, K=z((1, 8, 9), np.float32), mu=z((1, 8), np.float32),
+                           sigma=np.ones((1, 8), np.float32), M=np.eye(8, dtype=np.float32)[None]))
+        with torch.cuda.stream(side):
+            P, I, V = ca.project(x)
+        side.synchronize()
+        assert torch.equal(V, s * x)
+        assert torch.equal(P, s * x)
