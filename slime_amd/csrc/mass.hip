@@ -223,7 +223,7 @@ __global__ __launch_bounds__(256) void cell_conserve_kernel(const TX* X, const f
         float sx = 0.f, sy = 0.f;
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            sx += __builtin_fmaf(xv[q], s_hi, xv[q] * s_lo);
+            sx += __builtin_fmaf(xv[q], s_lo, xv[q] * s_hi);
             sy += yv[q];
         }
         // the D / 8 consecutive lanes of one (cell, head) share their sums
