@@ -35,7 +35,9 @@
  *     calling thread.
  *   - State tensors are device pointers, channels-last [B][G][G][C] with
  *     C = H * D, element type = the handle's dtype (fp32, or bf16 as raw 16-bit
- *     words). Arithmetic is fp32 (fp64 for reductions and the Jacobi solve).
+ *     words). They may start at any element of an allocation; a call copies one that
+ *     does not start at a multiple of 16 bytes into a buffer of the handle, or out of
+ *     one. Arithmetic is fp32 (fp64 for reductions and the Jacobi solve).
  *   - Parameters are host fp32 arrays, row-major:
  *       WP, WI, WV   [pods][C][C]   row k = input channel, column n = output channel
  *       K            [pods][H][9]   tap k = 3*(dy+1)+(dx+1), toroidal neighbours

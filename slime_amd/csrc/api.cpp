@@ -222,6 +222,26 @@ class DeviceScope {
     bool restore_ = false;
 };
 
+// The kernels move state tensors in 16-byte pieces, inputs by direct global->LDS loads, whose
+// addresses must then be multiples of 16; a caller's tensor may start at any element of its
+// buffer. Such an input is copied into `spare`, a buffer of the handle that the call does
+// not use otherwise, and such an output is written to one and copied out at the end.
+bool piece_aligned(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+int aligned_input(slime_ca* h, const void** x, void* spare, hipStream_t s) {
+    if (piece_aligned(*x)) return SLIME_OK;
+    HIP_TRY(launch_copy(h->elem, *x, spare, h->state_elems, s));
+    *x = spare;
+    return SLIME_OK;
+}
+
+// y, or `spare` in its place; give_back then copies it to y.
+void* aligned_output(void* y, void* spare) { return piece_aligned(y) ? y : spare; }
+int give_back(slime_ca* h, const void* from, void* y, size_t elem, hipStream_t s) {
+    if (from != y) HIP_TRY(launch_copy(elem, from, y, h->state_elems, s));
+    return SLIME_OK;
+}
+
 // S1 for one step, then the projection GEMM(s). Weights that the deferred mass scale of x
 // does not touch come from W1, one copy per pod: all of them when x_scale is NULL (a state
 // as its caller holds it), and the second and third plane of the chained forms. Scaled
@@ -566,7 +586,14 @@ int slime_ca_project(slime_ca* h, const void* x_in, void* P, void* I, void* V, v
         return fail(SLIME_EINVAL, "P, I and V must be distinct from x_in and from each other");
     hipStream_t s = static_cast<hipStream_t>(stream);
     h->last_stream = s;
-    return run_project(h, x_in, nullptr, P, I, V, s);
+    void* outs[3] = {P, I, V};
+    void* own[3] = {h->P, h->I, h->V};
+    void* to[3];
+    for (int i = 0; i < 3; ++i) to[i] = aligned_output(outs[i], own[i]);
+    rc = aligned_input(h, &x_in, h->S[0], s);
+    if (!rc) rc = run_project(h, x_in, nullptr, to[0], to[1], to[2], s);
+    for (int i = 0; i < 3 && !rc; ++i) rc = give_back(h, to[i], outs[i], h->elem, s);
+    return rc;
 }
 
 int slime_ca_flow_lenia(slime_ca* h, const void* x_in, const void* P, const void* I, const void* V,
@@ -583,8 +610,15 @@ int slime_ca_flow_lenia(slime_ca* h, const void* x_in, const void* P, const void
     const slime_ca_config& c = h->cfg;
     // The output is rescaled once from an fp32 copy, so a bf16 state is rounded once.
     void* raw = h->Sf ? static_cast<void*>(h->Sf) : h->S[0];
-    return run_stencil(h, x_in, nullptr, P, I, V, raw, h->Sf != nullptr, h->scale[0], s, nullptr, nullptr,
-                       nullptr, y_out);
+    void* y = aligned_output(y_out, h->P);  // written after the stencil has read P
+    rc = aligned_input(h, &x_in, h->S[1], s);
+    if (!rc) rc = aligned_input(h, &P, h->P, s);
+    if (!rc) rc = aligned_input(h, &I, h->I, s);
+    if (!rc) rc = aligned_input(h, &V, h->V, s);
+    if (!rc)
+        rc = run_stencil(h, x_in, nullptr, P, I, V, raw, h->Sf != nullptr, h->scale[0], s, nullptr, nullptr,
+                         nullptr, y);
+    return rc ? rc : give_back(h, y, y_out, h->elem, s);
 }
 
 int slime_ca_step(slime_ca* h, const void* x_in, void* x_out, int n_steps, void* stream) {
@@ -603,6 +637,9 @@ int slime_ca_step(slime_ca* h, const void* x_in, void* x_out, int n_steps, void*
                                    hipMemcpyDeviceToDevice, s));
         return SLIME_OK;
     }
+    rc = aligned_input(h, &x_in, h->S[1], s);  // the first step writes S[0]
+    if (rc) return rc;
+    void* out = aligned_output(x_out, h->P);  // written after the last stencil has read P
     const void* cur = x_in;
     const float* cur_scale = nullptr;  // the caller's state is complete
     // Intermediate outputs stay unscaled in the storage type: the next step applies
@@ -616,12 +653,12 @@ int slime_ca_step(slime_ca* h, const void* x_in, void* x_out, int n_steps, void*
         rc = run_project(h, cur, cur_scale, h->P, h->I, h->V, s);
         if (rc) return rc;
         rc = run_stencil(h, cur, cur_scale, h->P, h->I, h->V, y, y_f32, ys, s, nullptr, nullptr, nullptr,
-                         last ? x_out : nullptr);
+                         last ? out : nullptr);
         if (rc) return rc;
         cur = y;
         cur_scale = ys;
     }
-    return SLIME_OK;
+    return give_back(h, out, x_out, h->elem, s);
 }
 
 int slime_ca_mass(slime_ca* h, double* h_in, double* h_out) {
@@ -678,14 +715,19 @@ int slime_ca_rollout(slime_ca* h, void* hist, int T, double* scales, void* strea
     // the stencil's loads, and stores state t before its own rescale; the factor goes
     // to the handle (for step t+1) and to scales[t].
     const float* cur_scale = nullptr;  // hist[0] is complete
+    const void* cur = base;
+    rc = aligned_input(h, &cur, h->S[0], s);
+    if (rc) return rc;
     for (int t = 1; t < T; ++t) {
-        const void* cur = base + (size_t)(t - 1) * state_bytes;
-        void* y = base + (size_t)t * state_bytes;
+        void* state = base + (size_t)t * state_bytes;  // states are whole 16-byte pieces long
+        void* y = aligned_output(state, h->S[t & 1]);
         float* ys = h->scale[t & 1];
         rc = run_project(h, cur, cur_scale, h->P, h->I, h->V, s);
         if (rc) return rc;
         rc = run_stencil(h, cur, cur_scale, h->P, h->I, h->V, y, 0, ys, s, scales + (size_t)t * BH);
+        if (!rc) rc = give_back(h, y, state, h->elem, s);
         if (rc) return rc;
+        cur = y;
         cur_scale = ys;
     }
     return SLIME_OK;
@@ -885,6 +927,10 @@ int slime_ca_backward(slime_ca* h, const void* x_in, const void* target, float* 
     hipStream_t s = static_cast<hipStream_t>(stream);
     h->last_stream = s;
 
+    rc = aligned_input(h, &x_in, h->S[0], s);
+    if (!rc) rc = aligned_input(h, &target, h->S[1], s);
+    if (rc) return rc;
+
     // forward tape: P, I, V and I before its GELU; the unscaled fp32 output and the scale
     rc = run_project(h, x_in, nullptr, h->P, h->I, h->V, s, h->Ipre);
     if (rc) return rc;
@@ -950,8 +996,11 @@ int slime_ca_backward(slime_ca* h, const void* x_in, const void* target, float* 
         g.K = (int)(3 * C);
         g.ncol = (int)C;
         g.act[0] = 0;
-        g.out[0] = grad_x;  // grad_x = gXd + the GEMM, from its epilogue
+        // grad_x = gXd + the GEMM, from its epilogue; nothing reads gU any more
+        g.out[0] = aligned_output(grad_x, h->bw_gU);
         HIP_TRY(launch_gemm_add_f32(c.dtype, g, h->bw_gXd, s));
+        rc = give_back(h, g.out[0], grad_x, 4, s);
+        if (rc) return rc;
     }
     if (want_w) {
         DwArgs d{};

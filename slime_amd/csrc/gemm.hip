@@ -31,29 +31,6 @@
 namespace slime {
 namespace {
 
-// For operands that are not aligned to the 16 bytes the tile kernels load and store at once (a
-// state that starts inside another buffer): one thread per output, fp32 accumulation.
-template <typename T>
-__global__ __launch_bounds__(256) void gemm_unaligned_kernel(GemmArgs g) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long long)g.M * g.N) return;
-    const int m = (int)(idx / g.N), n = (int)(idx % g.N);
-    const T* a = static_cast<const T*>(g.A) + (long long)m * g.K;
-    const T* b = static_cast<const T*>(g.Bt) + (long long)(m / g.rows_per_batch) * g.bt_batch_stride +
-                 (long long)n * g.K;
-    float acc = 0.f;
-    for (int k = 0; k < g.K; ++k) acc = __builtin_fmaf(Store<T>::to_f32(a[k]), Store<T>::to_f32(b[k]), acc);
-    const int plane = n / g.ncol, col = n % g.ncol;
-    static_cast<T*>(g.out[plane])[(long long)m * g.ncol + col] =
-        Store<T>::from_f32(apply_act(acc, g.act[plane]));
-}
-
-bool aligned16(const GemmArgs& a) {
-    uintptr_t p = reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.Bt);
-    for (int i = 0; i < a.N / a.ncol; ++i) p |= reinterpret_cast<uintptr_t>(a.out[i]);
-    return p % 16 == 0;
-}
-
 // The 256 x 256 kernel's shapes: whole tiles in M, N, the planes and the batches, and K in
 // whole groups of 4 slabs (4 x 64 bytes: 128 bf16 or 64 fp32).
 bool fits256(int dtype, const GemmArgs& a) {
@@ -88,14 +65,6 @@ int gemm_tile(int dtype, const GemmArgs& a, int n_cu) {
 }
 
 hipError_t launch_gemm(int dtype, const GemmArgs& a, hipStream_t s) {
-    if (!aligned16(a)) {
-        const dim3 grid((unsigned)(((long long)a.M * a.N + 255) / 256));
-        if (dtype == 1)
-            hipLaunchKernelGGL(gemm_unaligned_kernel<bf16_t>, grid, dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL(gemm_unaligned_kernel<float>, grid, dim3(256), 0, s, a);
-        return hipGetLastError();
-    }
     int n_cu = 0;
     if (hipError_t e = device_cu_count(&n_cu); e != hipSuccess) return e;
     const int tile = gemm_tile(dtype, a, n_cu);

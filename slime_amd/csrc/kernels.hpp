@@ -27,6 +27,7 @@ struct GemmArgs {
 // The tile that a launch on n_cu compute units uses: 256 (gemm_tile.hpp), 128 or 64
 // (gemm_small.hip); 0 when none fits the shape. dtype: 0 fp32, 1 bf16.
 int gemm_tile(int dtype, const GemmArgs& a, int n_cu);
+// Every operand and output of the three launches starts at a multiple of 16 bytes.
 hipError_t launch_gemm(int dtype, const GemmArgs& a, hipStream_t s);
 // One output plane (N = ncol, identity) written as fp32 out[0] = A Bt^T + add, add of
 // out[0]'s layout and another buffer.
@@ -124,6 +125,8 @@ hipError_t launch_fill_f64(double* p, int n, double v, hipStream_t s);
 // of part_out ([B][H][tiles], the stencil's layout) are rewritten from the result.
 hipError_t launch_cell_conserve(const void* x, const float* scale, void* y, int y_f32, double* part_out, int B, int G,
                                 hipStream_t s);
+// y[i] = x[i] for n elements of 2 or 4 bytes, either side at any element's address.
+hipError_t launch_copy(size_t elem, const void* x, void* y, long long n, hipStream_t s);
 // y[i] = cvt((scale[0][b][h] + scale[1][b][h]) * x[i]) over the whole state; x is
 // fp32 when x_f32 is set, else in the storage type.
 hipError_t launch_rescale(int dtype, const void* x, int x_f32, const float* scale, void* y, int B,

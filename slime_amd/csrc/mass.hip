@@ -114,6 +114,19 @@ __device__ __forceinline__ void rescale_quad(const TI* x, T* y, long long q, flo
     }
 }
 
+// Element by element, so that neither side needs an alignment: 8 per thread, a wave's
+// accesses contiguous.
+constexpr int kCopyPer = 8;
+template <typename T>
+__global__ __launch_bounds__(256) void copy_kernel(const T* x, T* y, long long n) {
+    const long long i0 = (long long)blockIdx.x * (256 * kCopyPer) + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kCopyPer; ++k) {
+        const long long i = i0 + k * 256;
+        if (i < n) y[i] = x[i];
+    }
+}
+
 template <typename TI, typename T>
 __global__ __launch_bounds__(256) void rescale_kernel(const TI* x, const float* scale, T* y,
                                                       long long nquads, int C, int D,
@@ -259,6 +272,17 @@ hipError_t launch_cell_conserve(const void* x, const float* scale, void* y, int 
     else
         hipLaunchKernelGGL((cell_conserve_kernel<bf16_t, bf16_t, 64>), grid, dim3(256), 0, s, xp, scale,
                            static_cast<bf16_t*>(y), part_out, B, G);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy(size_t elem, const void* x, void* y, long long n, hipStream_t s) {
+    const dim3 grid((unsigned)((n + 256 * kCopyPer - 1) / (256 * kCopyPer)));
+    if (elem == 2)
+        hipLaunchKernelGGL(copy_kernel<uint16_t>, grid, dim3(256), 0, s, static_cast<const uint16_t*>(x),
+                           static_cast<uint16_t*>(y), n);
+    else
+        hipLaunchKernelGGL(copy_kernel<uint32_t>, grid, dim3(256), 0, s, static_cast<const uint32_t*>(x),
+                           static_cast<uint32_t*>(y), n);
     return hipGetLastError();
 }
 
