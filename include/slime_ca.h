@@ -353,7 +353,8 @@ int slime_snapshot_json(const slime_ca* ca, const float* chemical_concentration,
                         const slime_pool* pool, int generation, double elapsed, char* buf,
                         size_t cap, size_t* written);
 
-/* 1 when this build runs S1 on the MFMA tile kernel for the handle's shape. */
+/* 1 when this build runs S1 on matrix-core tiles for the handle's shape: every shape that
+ * slime_ca_create takes. */
 int slime_ca_uses_mfma(const slime_ca* ca);
 
 const char* slime_ca_last_error(void);

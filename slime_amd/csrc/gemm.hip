@@ -24,44 +24,14 @@
 // range, N fastest, so a cell block and one batch's weights are re-read from that
 // XCD's L2.
 // The tile kernel and its helpers are in gemm_tile.hpp (also built, with an adding
-// fp32 epilogue, by gemm_add.hip); this file holds the choice between it and the smaller
-// tiles of gemm_small.hip, the launchers and the weight folding.
+// fp32 epilogue, by gemm_add.hip); this file holds the launchers and the weight folding;
+// the choice between it and the smaller tiles of gemm_small.hip is in gemm_rule.hpp.
+#include "gemm_rule.hpp"
 #include "gemm_tile.hpp"
 
 namespace slime {
-namespace {
-
-// The 256 x 256 kernel's shapes: whole tiles in M, N, the planes and the batches, and K in
-// whole groups of 4 slabs (4 x 64 bytes: 128 bf16 or 64 fp32).
-bool fits256(int dtype, const GemmArgs& a) {
-    const int k_group = dtype == 1 ? 128 : 64;
-    return a.M % kBM == 0 && a.N % kBN == 0 && a.ncol % kBN == 0 && a.K % k_group == 0 &&
-           a.rows_per_batch % kBM == 0;
-}
-
-}  // namespace
-
-// The tile whose rounds over the card take least time: ceil(tiles / CUs) rounds of
-// tile^2 products each, at the rate the kernel reaches once it fills the card. Measured on
-// K = 512 forward products (TFLOP/s, 256 / 128 / 64 wide): bf16 915 / 730 / 610 at 65,536
-// rows, fp32 139 / 137 / 131; so the 256-wide kernel keeps what it tiles and
-// fills, and a batch that leaves its last round mostly empty goes to the smaller tiles:
-// 16,384 x 1536 x 512 in fp32 (384 tiles of 256 on 256 CUs) 272 -> 192 us in 1536 tiles of
-// 128; 8192 x 768 x 256 80 -> 31 us in tiles of 64. Shapes that 256 does not divide ran one
-// thread per output before (0.55 TFLOP/s): 73,984 x 1536 x 512 bf16 211 ms -> 0.17 ms.
 int gemm_tile(int dtype, const GemmArgs& a, int n_cu) {
-    int best = 0;
-    double best_t = 0.0;
-    for (int tile : {256, 128, 64}) {
-        if (tile == 256 ? !fits256(dtype, a) : !gemm_small_fits(dtype, tile, a)) continue;
-        const long long rows = (a.rows_per_batch + tile - 1) / tile;  // per batch
-        const long long ntiles = a.M / a.rows_per_batch * rows * (a.N / tile);
-        const long long rounds = (ntiles + n_cu - 1) / n_cu;
-        const double rate = tile == 256 ? 1.0 : dtype == 1 ? (tile == 128 ? 0.8 : 0.66) : (tile == 128 ? 0.98 : 0.94);
-        const double t = (double)rounds * tile * tile / rate;
-        if (!best || t < best_t) best = tile, best_t = t;
-    }
-    return best;
+    return gemm_rule::pick({dtype, a.M, a.N, a.K, a.ncol, a.rows_per_batch}, n_cu);
 }
 
 hipError_t launch_gemm(int dtype, const GemmArgs& a, hipStream_t s) {

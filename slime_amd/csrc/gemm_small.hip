@@ -13,8 +13,9 @@
 // by the matrix cores (137 of 157 TFLOP/s); the smallest products (M <= 1024, K <= 192)
 // take 4 us, a launch and two memory round trips. Three stages (48 KiB, three workgroups
 // per CU) instead of four: 16,384 x 1536 x 512 fp32 197 -> 192 us, 65,536 x 384 x 128 bf16
-// 20.5 -> 18.8 us, no shape slower. The choice of tile: gemm_tile (gemm.hip).
+// 20.5 -> 18.8 us, no shape slower. The choice of tile: gemm_rule.hpp.
 #include "common.hpp"
+#include "gemm_rule.hpp"
 #include "gemm_small_addr.hpp"
 #include "kernels.hpp"
 
@@ -75,7 +76,7 @@ __device__ __forceinline__ void store_block(T* out, int ncol, int lane, float (&
     }
 }
 
-template <typename T, int BT, int SB, int kStages, Mode kMode>
+template <typename T, int BT, int SB, Mode kMode>
 __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(GemmArgs g, void* aux) {
     using S = Shape<BT, SB>;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[kStages * S::kStageB];
@@ -111,10 +112,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(GemmArgs g, voi
     for (int ks = 0; ks < kStages - 1 && ks < nk; ++ks) issue(ks, ks);
     int rd = 0, wr = kStages - 1;
     for (int ks = 0; ks < nk; ++ks) {
-        // The slabs issued after slab ks: one, none at the end.
-        const int younger = nk - 1 - ks;
-        static_assert(kStages == 3, "one slab is younger than the one waited for");
-        if (younger >= 1) wait_vm<S::kDps>();
+        static_assert(kStages == 3, "one slab is younger than the one waited for, none at the end");
+        if (younger_slabs(ks, nk) > 0) wait_vm<S::kDps>();
         else wait_vm<0>();
         lds_barrier();  // slab ks is in LDS; every wave has read slab ks - 1, whose stage is free
         if (ks + kStages - 1 < nk) issue(ks + kStages - 1, wr);
@@ -176,9 +175,9 @@ hipError_t launch_mode(int tile, const GemmArgs& a, void* aux, hipStream_t s) {
     const int ntiles = a.M / a.rows_per_batch * tiles_per_batch(tile, a.rows_per_batch) * (a.N / tile);
     const dim3 grid(8 * ((ntiles + 7) / 8));
     if (tile == 128)
-        hipLaunchKernelGGL((gemm_small_kernel<T, 128, 64, 3, kMode>), grid, dim3(kThreads), 0, s, a, aux);
+        hipLaunchKernelGGL((gemm_small_kernel<T, 128, 64, kMode>), grid, dim3(kThreads), 0, s, a, aux);
     else
-        hipLaunchKernelGGL((gemm_small_kernel<T, 64, 128, 3, kMode>), grid, dim3(kThreads), 0, s, a, aux);
+        hipLaunchKernelGGL((gemm_small_kernel<T, 64, 128, kMode>), grid, dim3(kThreads), 0, s, a, aux);
     return hipGetLastError();
 }
 
@@ -190,12 +189,8 @@ hipError_t launch_small(int dtype, int tile, const GemmArgs& a, void* aux, hipSt
 
 }  // namespace
 
-// Whole tiles of columns inside a plane, at least one tile of rows per batch, whole slabs
-// (64 or 128 bytes) of K.
 bool gemm_small_fits(int dtype, int tile, const GemmArgs& a) {
-    const int slab = (tile == 128 ? 64 : 128) / (dtype == 1 ? 2 : 4);
-    return a.N % tile == 0 && a.ncol % tile == 0 && a.rows_per_batch >= tile &&
-           a.M % a.rows_per_batch == 0 && a.K % slab == 0;
+    return gemm_rule::fits_small(tile, {dtype, a.M, a.N, a.K, a.ncol, a.rows_per_batch});
 }
 
 hipError_t launch_gemm_small(int dtype, int tile, const GemmArgs& a, hipStream_t s) {

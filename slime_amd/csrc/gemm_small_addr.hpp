@@ -1,8 +1,9 @@
 // gemm_small_addr.hpp — the address arithmetic of the 128- and 64-wide tile GEMM
 // (gemm_small.hip): the tile walk with its overlapping last tile per batch, the direct
-// loads and the operand fragment reads. Plain C++ with no HIP types, shared with the
-// host replay tests/gemm_small_replay.cpp, which checks every address of a launch
-// against its buffer and every fragment read against the row and chunk its MFMA needs.
+// loads, the operand fragment reads and the ring's waits. Plain C++ with no HIP types, shared
+// with the host replay tests/gemm_small_replay.cpp, which checks every address of a launch
+// against its buffer, every fragment read against the row and chunk its MFMA needs and
+// every wait against the order in which the wave's loads complete.
 #pragma once
 
 #include "gemm_addr.hpp"
@@ -11,6 +12,13 @@ namespace slime {
 namespace gemm_small {
 
 constexpr int kThreads = 256, kWaves = 4;
+constexpr int kStages = 3;  // LDS ring: slab ks in stage ks % kStages
+
+// The slabs whose loads a wave has issued after slab ks's when it waits for that one: the
+// prologue issues kStages - 1 slabs, step ks slab ks + kStages - 1 after its wait.
+SLIME_HD constexpr int younger_slabs(int ks, int nk) {
+    return nk - 1 - ks < kStages - 2 ? nk - 1 - ks : kStages - 2;
+}
 
 // BT x BT output tile (cells x output channels), K in slabs of SB bytes per row.
 template <int BT, int SB>

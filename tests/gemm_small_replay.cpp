@@ -5,11 +5,15 @@
 // For every workgroup, wave and lane of one launch it checks that each direct load reads
 // inside A or Bt and fills its own 16 bytes of a stage, that every fragment read finds the
 // row and 16-byte chunk its MFMA needs, that each tile lies inside one batch and one output
-// plane, that the tiles are visited once, and that they cover every output row and column.
+// plane, that the tiles are visited once, and that they cover every output row and column;
+// and, for one wave's walk over the K slabs, that each vmcnt wait covers its slab under
+// in-order completion of the wave's direct loads (no looser, no stricter), that a step reads
+// the stage which holds its slab, and that no load fills a stage still to be read.
 //
 // Usage: gemm_small_replay TILE SLAB M N K elem rows_per_batch bt_batch_stride bt_elems ncol [plant]
 //   plant "past-end": model the last tile of a batch as starting at its grid position (a
 //   planted mistake: it would read past a ragged batch's end)
+//   plant "loose-wait": model every wait one slab looser than the kernel's
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -26,14 +30,45 @@ namespace {
     std::exit(1);
 }
 
+// The kernel's K loop as one wave sees it: kDps direct loads per slab, a wait and a barrier
+// at each step, then the next slab's loads and the reads of this one.
+template <int BT, int SB>
+void check_ring(int nk, bool loose) {
+    using S = Shape<BT, SB>;
+    std::vector<int> ops;  // the slab of each direct load, in issue order
+    int stage[kStages];
+    for (int& s : stage) s = -1;
+    auto issue = [&](int ks, int step) {
+        int& held = stage[ks % kStages];
+        if (held >= step) fail("a load fills a stage still to be read", ks, held, step);
+        held = ks;
+        for (int j = 0; j < S::kDps; ++j) ops.push_back(ks);
+    };
+    for (int ks = 0; ks < kStages - 1 && ks < nk; ++ks) issue(ks, 0);
+    for (int ks = 0; ks < nk; ++ks) {
+        const int n = younger_slabs(ks, nk) * S::kDps + (loose ? S::kDps : 0);
+        if (n > 63) fail("vmcnt immediate beyond the 6-bit counter", ks, n, 0);
+        long long last = (long long)ops.size() - 1;
+        while (last >= 0 && ops[last] != ks) --last;
+        const long long younger = (long long)ops.size() - 1 - last;
+        if (last < 0) fail("wait for a slab never loaded", ks, nk, n);
+        if (n > younger) fail("wait too loose: slab may be incomplete", ks, n, younger);
+        if (n < younger) fail("wait stricter than needed", ks, n, younger);
+        if (ks + kStages - 1 < nk) issue(ks + kStages - 1, ks);
+        if (stage[ks % kStages] != ks) fail("step reads a stage that holds another slab", ks, stage[ks % kStages], 0);
+    }
+}
+
 template <int BT, int SB>
 void run(long long M, long long N, long long K, int elem, int rpb, long long bt_stride, long long bt_elems,
-         int ncol, bool plant) {
+         int ncol, const char* planted) {
     using S = Shape<BT, SB>;
     const long long row_bytes = K * elem;
     const int nN = (int)(N / BT), nk = (int)(row_bytes / SB);
     if (N % BT || ncol % BT || row_bytes % SB || rpb < BT || M % rpb) fail("shape", M, N, K);
     const int ntiles = (int)(M / rpb) * tiles_per_batch(BT, rpb) * nN;
+    const bool plant = !std::strcmp(planted, "past-end");
+    check_ring<BT, SB>(nk, !std::strcmp(planted, "loose-wait"));
     std::vector<int> seen(ntiles, 0);
     std::vector<char> rows(M, 0);
     const int grid = 8 * ((ntiles + 7) / 8);
@@ -91,7 +126,7 @@ int main(int argc, char** argv) {
     const int tile = std::atoi(argv[1]), slab = std::atoi(argv[2]);
     long long v[8];
     for (int i = 0; i < 8; ++i) v[i] = std::atoll(argv[3 + i]);
-    const bool plant = argc > 11 && !std::strcmp(argv[11], "past-end");
+    const char* plant = argc > 11 ? argv[11] : "";
     if (tile == 128 && slab == 64)
         run<128, 64>(v[0], v[1], v[2], (int)v[3], (int)v[4], v[5], v[6], (int)v[7], plant);
     else if (tile == 64 && slab == 128)

@@ -5,11 +5,12 @@
 workgroup, wave and lane of a launch and checks every direct load, LDS access and
 store against its buffer, and every ``s_waitcnt vmcnt`` against the in-order
 completion of the wave's loads and stores. The launches are the ones the library
-makes (``slime_amd/csrc/api.cpp``): the forward [P|I|V] GEMM, the chained
-projections' per-plane GEMMs, the backward tape's pre-activation GEMM and the
-backward dX GEMM (K = 3C, fp32 output with an addend), on every BASELINE
-configuration whose shape takes the MFMA path, with the MI355X's 256 CUs and
-with CU counts that exercise the other branch of the tile schedule.
+makes (``tests/gemm_launches.py``): the [P|I|V] GEMM of a call's first step over each
+pod's rows and of later steps over each batch entry's, the chained projections'
+per-plane GEMMs and the backward dX GEMM (K = 3C, fp32 output with an addend), on
+every BASELINE configuration whose shape 256 x 256 tiles fit, with the MI355X's 256
+CUs and with CU counts that exercise the other branch of the tile schedule. (The
+backward's tape writes the first step's planes, one of them twice: no other address.)
 """
 import os
 import subprocess
@@ -17,6 +18,7 @@ import subprocess
 import pytest
 
 from slime_amd.synthetic import CONFIGS, CAConfig
+from tests import gemm_launches
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRC = os.path.join(HERE, "gemm_addr_replay.cpp")
@@ -29,30 +31,21 @@ def replay(tmp_path_factory):
     return exe
 
 
-def _uses_mfma(M, N, K, elem, rows_per_batch, ncol):
+def _fits256(M, N, K, elem, rows_per_batch, ncol):
     k_group = 128 if elem == 2 else 64
     return M % 256 == 0 and N % 256 == 0 and ncol % 256 == 0 and K % k_group == 0 \
         and rows_per_batch % 256 == 0
 
 
 def launches(cfg: CAConfig):
-    """(name, M, N, K, elem, rows_per_batch, bt_batch_stride, bt_elems, ncol, nplanes,
-    epilogue) of each GEMM the library launches for this configuration."""
-    C, elem = cfg.C, (2 if cfg.dtype == "bf16" else 4)
-    M, rpb, stride = cfg.B * cfg.G * cfg.G, cfg.G * cfg.G, 3 * C * C
-    wt = cfg.B * 3 * C * C  # per-batch transposed weights [B][3C][C]
-    epi = "bf16" if cfg.dtype == "bf16" else "f32"
-    yield ("forward [P|I|V]", M, 3 * C, C, elem, rpb, stride, wt, C, 3, epi)
-    for p in range(3):  # chained projections: one GEMM per plane, Bt offset by p C^2
-        yield (f"chained plane {p}", M, C, C, elem, rpb, stride, wt - p * C * C, C, 1, epi)
-    yield ("backward tape I~", M, C, C, elem, rpb, stride, wt - C * C, C, 1, epi)
-    rows_pod = (cfg.B // cfg.pods) * cfg.G * cfg.G
-    yield ("backward dX", M, C, 3 * C, elem, rows_pod, stride, cfg.pods * 3 * C * C, C, 1, "f32add")
+    return gemm_launches.launches(cfg.B, cfg.G, cfg.D, cfg.dtype, cfg.pods)
 
 
 CASES = [cfg for cfg in CONFIGS.values()] + [
     CAConfig("persist", B=24, G=32, H=8, D=64, dtype="bf16", steps=1, w_std=0.05, pods=3),
     CAConfig("fp32-32", B=2, G=32, H=8, D=64, dtype="fp32", steps=1, w_std=0.05),
+    # a pod's four batch entries together are whole tiles, one of them is not
+    CAConfig("span-pod", B=4, G=136, H=8, D=64, dtype="bf16", steps=1, w_std=0.05),
 ]
 
 
@@ -67,7 +60,7 @@ def test_every_gemm_address_in_bounds_and_every_wait_exact(replay, cfg):
     ran = 0
     for args in launches(cfg):
         name, M, N, K, elem, rpb = args[:6]
-        if not _uses_mfma(M, N, K, elem, rpb, args[8]):
+        if not _fits256(M, N, K, elem, rpb, args[8]):
             continue
         for n_cu in (256, 80, 7):
             rc, out = _run(replay, args, n_cu)
@@ -75,7 +68,7 @@ def test_every_gemm_address_in_bounds_and_every_wait_exact(replay, cfg):
             assert rc == 0 and out.startswith("OK"), (cfg.name, name, n_cu, out)
             ran += 1
     if cfg.name == "c1":
-        assert ran == 0  # 32x32 grid, D 8: the generic kernel runs
+        assert ran == 0  # 32x32 grid, D 8: 64-wide tiles (test_gemm_small_addr.py)
     else:
         assert ran > 0
 
@@ -83,13 +76,23 @@ def test_every_gemm_address_in_bounds_and_every_wait_exact(replay, cfg):
 def test_replay_reports_planted_mistakes(replay):
     """The checks fire: a weight buffer one 16-row group short of the c3 launch's
     last tile, and waits modelled one slab looser than the kernel's."""
-    args = next(launches(CONFIGS["c3"]))
+    args = launches(CONFIGS["c3"])[0]
     short_bt = list(args)
     short_bt[7] = args[7] - 16 * args[3]
     rc, out = _run(replay, short_bt, 256)
     assert rc == 1 and "direct load from Bt" in out, out
     rc, out = _run(replay, args, 256, ("plant-loose-wait",))
     assert rc == 1 and "too loose" in out, out
+
+
+def test_weights_per_pod_are_not_indexed_by_batch_entry(replay):
+    """The first step's weights hold one copy per pod: taken with the later steps' rows per
+    batch, a launch would read past them."""
+    first, later = launches(CASES[-1])[:2]
+    wrong = first._replace(rows_per_batch=16384, M=65536)  # whole tiles, four "batches", one pod's weights
+    assert first.bt_elems * 4 == later.bt_elems
+    rc, out = _run(replay, wrong, 256)
+    assert rc == 1 and "direct load from Bt" in out, out
 
 
 @pytest.mark.parametrize("plant,message", [
@@ -101,5 +104,5 @@ def test_layout_check_reports_planted_mistakes(tmp_path, plant, message):
     16-byte chunk, or when the staged read-back keeps its rows' halves swapped."""
     exe = str(tmp_path / "replay_planted")
     subprocess.run(["g++", "-O2", "-std=c++17", f"-D{plant}", "-o", exe, SRC], check=True)
-    rc, out = _run(exe, next(launches(CONFIGS["c3"])), 256)
+    rc, out = _run(exe, launches(CONFIGS["c3"])[0], 256)
     assert rc == 1 and message in out, out

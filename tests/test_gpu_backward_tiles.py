@@ -1,6 +1,7 @@
-"""The backward's products at shapes off the large tiles -- ragged grids (576 and 1600 rows per
-pod: row chunks with a remainder, a dX tile moved back to the pod's end), C = 64 in bf16 and
-every fp32 width -- against the oracle's fp64 gradient, with the bounds of
+"""The backward's products at shapes off the 256-wide tiles -- ragged grids (576 and 1600 rows
+per pod: row chunks with a remainder), C = 64 in bf16 and every fp32 width, and the taped
+projections and dX in 128-wide tiles, the last one moved back to the pod's end
+(test_gemm_rule.py holds which tiles these are) -- against the oracle's fp64 gradient, with the bounds of
 test_gpu_backward (normalised maximum 1e-5 for an fp32 state, 2e-2 for bf16)."""
 import pytest
 
@@ -21,6 +22,10 @@ from slime_amd import Pseudopod  # noqa: E402
     ("fp32", 8, 1, 1, 40),
     ("fp32", 32, 2, 2, 24),
     ("fp32", 64, 1, 2, 24),
+    # 128-wide tiles: 3136 and 7744 rows per pod (the last tile moved back by half), 8192 rows
+    ("bf16", 64, 2, 2, 56),
+    ("fp32", 64, 1, 1, 88),
+    ("fp32", 64, 1, 2, 64),
 ])
 def test_backward_products_match_oracle(oracle, dtype, D, pods, B, G):
     if not torch.cuda.is_available():

@@ -43,13 +43,16 @@ def _check(got, x, w, act, bf16, name):
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 @pytest.mark.parametrize("B,G,D,pods,chain", [
+    # The rows of a pod are one batch of the product; test_gemm_rule.py holds the tiles.
     (1, 8, 8, 1, 0),      # one 64-row tile, the narrowest heads
-    (3, 8, 64, 3, 0),     # a batch per tile of rows
-    (2, 24, 16, 1, 0),    # 576 rows: the last tile of 128 moved back
+    (3, 8, 64, 3, 0),     # a pod per tile of rows
+    (2, 24, 16, 1, 0),    # 1152 rows over two batch entries in 64-wide tiles
     (4, 40, 32, 2, 1),
-    (2, 56, 64, 2, 0),
+    (2, 56, 64, 2, 0),    # 3136 rows per pod: bf16 in 128-wide tiles, the last one moved back by half
     (1, 72, 8, 1, 2),
-    (6, 136, 64, 2, 0),   # 73 tiles of 256 per batch, the last one a quarter full
+    (1, 88, 64, 1, 0),    # 7744 rows in 128-wide tiles, the last one moved back by half
+    (6, 136, 64, 2, 0),   # 55,488 rows per pod, likewise
+    (4, 136, 64, 1, 0),   # 73,984 rows: 256-wide tiles, which one batch entry's 18,496 do not fill
 ])
 def test_projections_match_fp64(dtype, B, G, D, pods, chain):
     print(f"[case] {dtype} B={B} G={G} D={D} pods={pods} chain={chain}", flush=True)
