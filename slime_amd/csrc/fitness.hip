@@ -474,7 +474,7 @@ __global__ __launch_bounds__(kFinThreads) void fitness_finalize_kernel(FitnessAr
         double app_now = app;
         if (any1) {
             double cr, sr;
-            jacobi_rotation<true>(app, aqq, rotate ? apq : 1.0, cr, sr);
+            jacobi_rotation(app, aqq, rotate ? apq : 1.0, cr, sr);
             const double app_new = cr * cr * app + sr * sr * aqq - 2.0 * cr * sr * apq;
             const double aqq_new = sr * sr * app + cr * cr * aqq + 2.0 * cr * sr * apq;
             c = rotate ? cr : 1.0;

@@ -11,15 +11,16 @@
 //     reciprocal, then q = a r corrected once by the exact residual a - b q
 //     (Markstein's correctly rounded quotient). Needs b and a / b normal and far
 //     from overflow, which holds for |b| in [2^-900, 2^900] and |a| < 2^900.
-//   * sqrt_ge1(x): Goldschmidt's coupled iteration g -> sqrt(x), h -> 1/(2 sqrt x)
-//     from y = rsq(x), then two residual corrections g += (x - g^2) h. Needs x in
-//     [2^-40, 2^900), where no pre-scale applies.
-//   * sqrt_and_rcp(x, g, r): both sqrt(x) and 1 / sqrt(x), from the same iteration.
-// slime_probe_fp64_core (probe.hip) checks them against `/` and `sqrt` bit for
-// bit over the rotation's operand ranges on the device.
+//   * sqrt_and_rcp(x, g, r): both sqrt(x) and 1 / sqrt(x), from one iteration.
+// slime_probe_fp64_core (probe.hip) checks them against `/` and `sqrt` bit for bit on the
+// device, over exponents from 2^-40 up (x) and in [-60, 60] (a, b), and the whole
+// rotation against its IEEE form; that form's own error is checked on the host
+// (tests/jacobi_wave_check.cpp).
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include "jacobi_wave.hpp"
 
 namespace slime {
 
@@ -31,66 +32,37 @@ __device__ __forceinline__ double div_rn(double a, double b) {
     return __builtin_fma(__builtin_fma(-b, q, a), r, q);
 }
 
-// Goldschmidt's iteration: returns g = sqrt(x) rounded, h ~ 1 / (2 sqrt x) to ~2^-44.
-__device__ __forceinline__ double sqrt_core(double x, double& h) {
+// g = sqrt(x) and r = 1 / sqrt(x) with both IEEE roundings (the bits of `sqrt(x)` and
+// `1.0 / sqrt(x)`), for x in [2^-40, 2^900), where no pre-scale applies: Goldschmidt's coupled
+// iteration g -> sqrt(x), h -> 1 / (2 sqrt x) from y = rsq(x), two residual corrections
+// g += (x - g^2) h, then the reciprocal of g from 2 h (good to ~2^-44) by one Newton-Raphson
+// step and the same correction as div_rn with a = 1. This replaces the v_rcp_f64 and one
+// of the two refinement steps that a division takes.
+__device__ __forceinline__ void sqrt_and_rcp(double x, double& g, double& r) {
     const double y = __builtin_amdgcn_rsq(x);
-    double g = x * y;
-    h = 0.5 * y;
+    g = x * y;
+    double h = 0.5 * y;
     const double e = __builtin_fma(-h, g, 0.5);
     g = __builtin_fma(g, e, g);
     h = __builtin_fma(h, e, h);
     g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
-}
-__device__ __forceinline__ double sqrt_ge1(double x) {
-    double h;
-    return sqrt_core(x, h);
-}
-
-// g = sqrt(x) and r = 1 / sqrt(x) with both IEEE roundings (the bits of `sqrt(x)` and
-// `1.0 / sqrt(x)`), for x in [2^-40, 2^900): sqrt_core, then the reciprocal of g from 2 h by
-// one Newton-Raphson step and the same correction as div_rn with a = 1. This replaces
-// the v_rcp_f64 and one of the two refinement steps that div_rn(1, sqrt_ge1(x)) takes.
-__device__ __forceinline__ void sqrt_and_rcp(double x, double& g, double& r) {
-    double h;
-    g = sqrt_core(x, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
     r = 2.0 * h;
     r = __builtin_fma(r, __builtin_fma(-g, r, 1.0), r);
     r = __builtin_fma(__builtin_fma(-g, r, 1.0), r, r);
 }
-__device__ __forceinline__ double rcp_sqrt_ge1(double x) {
-    double g, r;
-    sqrt_and_rcp(x, g, r);
-    return r;
-}
 
-// The rotation of the cyclic Jacobi solve for the 2x2 block [[app, apq], [apq, aqq]],
-// |apq| > 0, the one with |angle| <= pi / 4: with d = aqq - app and b = 2 apq,
-// |cos 2 theta| = |d| / sqrt(d^2 + b^2), c = sqrt((1 + |cos 2 theta|) / 2) and
-// s = sin 2 theta / (2 c) with the sign of d b (+ at d = 0). The same angle as
-// t = sign(tau) / (|tau| + sqrt(1 + tau^2)), tau = d / b, c = 1 / sqrt(1 + t^2), s = t c, with
-// two hardware estimates in a row instead of four; no difference of close numbers
-// appears in either, so both give c and s to a few units of 2^-53.
-// With the fast helpers (kFast) every precondition holds when d^2 + b^2 is in
-// [2^-40, 2^900): for a Gram of fp32 values summed over at most 2^40 cells, |a_ij| < 2^297,
-// and the solve rotates only for |apq| > 1e-6.
-template <bool kFast>
+// jacobi_wave::rotation with the short forms, the same bits: every precondition holds when
+// d^2 + b^2 is in [2^-40, 2^900). For a Gram of fp32 values summed over at most 2^40 cells,
+// |a_ij| < 2^297, and the solve rotates only for |apq| > 1e-6.
 __device__ __forceinline__ void jacobi_rotation(double app, double aqq, double apq, double& c, double& s) {
     const double d = aqq - app, b = 2.0 * apq;
-    const double h2 = __builtin_fma(d, d, b * b);
-    double r, ic;  // 1 / sqrt(d^2 + b^2), 1 / c
-    if constexpr (kFast) {
-        double h;
-        sqrt_and_rcp(h2, h, r);
-        sqrt_and_rcp(__builtin_fma(0.5 * fabs(d), r, 0.5), c, ic);
-        // The correction step rounds wrongly for a divisor whose significand is all ones, and
-        // a small angle makes c = 1 - 2^-53 common.
-        if (c == 0x1.fffffffffffffp-1) ic = 0x1.0000000000001p0;
-    } else {
-        r = 1.0 / sqrt(h2);
-        c = sqrt(__builtin_fma(0.5 * fabs(d), r, 0.5));
-        ic = 1.0 / c;
-    }
+    double h, r, ic;  // r = 1 / sqrt(d^2 + b^2), ic = 1 / c
+    sqrt_and_rcp(__builtin_fma(d, d, b * b), h, r);
+    sqrt_and_rcp(__builtin_fma(0.5 * fabs(d), r, 0.5), c, ic);
+    // The correction step rounds wrongly for a divisor whose significand is all ones, and
+    // a small angle makes c = 1 - 2^-53 common.
+    if (c == 0x1.fffffffffffffp-1) ic = 0x1.0000000000001p0;
     const double sb = d < 0.0 ? -apq : (d > 0.0 ? apq : fabs(apq));
     s = sb * r * ic;
 }

@@ -106,9 +106,10 @@ __device__ double draw(uint64_t r, int lo, int hi, bool sign) {
     return __builtin_bit_cast(double, bits);
 }
 
-// Per index i: div_rn against / on (a, b) with exponents in [-60, 60], sqrt_ge1 and
-// rcp_sqrt_ge1 against sqrt and 1 / sqrt on x in [1, 2^120), and the whole rotation (c, s) against its IEEE
-// form on (app, aqq, apq) drawn like Gram entries, every eighth with app = aqq.
+// Per index i: div_rn against / on (a, b) with exponents in [-60, 60], sqrt_and_rcp against
+// sqrt and 1 / sqrt on x in [2^-40, 2^120) and, every other index, in [1/2, 1] as under c's
+// root, and the whole rotation (c, s) against its IEEE form on (app, aqq, apq) drawn like
+// Gram entries, every eighth with app = aqq.
 __global__ void fp64_core_check(long long n, uint64_t seed, unsigned long long* bad) {
     unsigned long long miss = 0;
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
@@ -116,15 +117,18 @@ __global__ void fp64_core_check(long long n, uint64_t seed, unsigned long long* 
         const uint64_t r2 = mix64(seed ^ (uint64_t)(4 * i + 2)), r3 = mix64(seed ^ (uint64_t)(4 * i + 3));
         const double a = draw(r0, -60, 60, true), b = draw(r1, -60, 60, true);
         if (__builtin_bit_cast(uint64_t, slime::div_rn(a, b)) != __builtin_bit_cast(uint64_t, a / b)) ++miss;
-        const double x = draw(r2, 0, 119, false);
-        if (__builtin_bit_cast(uint64_t, slime::sqrt_ge1(x)) != __builtin_bit_cast(uint64_t, sqrt(x))) ++miss;
-        if (__builtin_bit_cast(uint64_t, slime::rcp_sqrt_ge1(x)) != __builtin_bit_cast(uint64_t, 1.0 / sqrt(x))) ++miss;
+        const double x = i % 2 ? draw(r2, -1, -1, false) : draw(r2, -40, 119, false);
+        double g, r;
+        slime::sqrt_and_rcp(x, g, r);
+        if (__builtin_bit_cast(uint64_t, g) != __builtin_bit_cast(uint64_t, sqrt(x))) ++miss;
+        // a root whose significand is all ones: the one divisor that the rotation sets apart
+        if (g != 0x1.fffffffffffffp-1 && __builtin_bit_cast(uint64_t, r) != __builtin_bit_cast(uint64_t, 1.0 / sqrt(x))) ++miss;
         const double app = draw(r0 ^ r3, -24, 8, false);
         const double aqq = (i % 8 == 0) ? app : draw(r1 ^ r3, -24, 8, false);
         const double apq = draw(r2 ^ (r3 << 7), -19, 8, true);  // |apq| > 1e-6 as in the solve
         double c0, s0, c1, s1;
-        slime::jacobi_rotation<true>(app, aqq, apq, c0, s0);
-        slime::jacobi_rotation<false>(app, aqq, apq, c1, s1);
+        slime::jacobi_rotation(app, aqq, apq, c0, s0);
+        slime::jacobi_wave::rotation(app, aqq, apq, c1, s1);
         if (__builtin_bit_cast(uint64_t, c0) != __builtin_bit_cast(uint64_t, c1) ||
             __builtin_bit_cast(uint64_t, s0) != __builtin_bit_cast(uint64_t, s1))
             ++miss;
@@ -317,8 +321,9 @@ double slime_probe_hbm_gbs(int kind) {
     return best;
 }
 
-// Mismatches, out of 3 n comparisons, between the short fp64 division, square root
-// and rotation of fp64.hpp and their IEEE forms, over n seeded draws. -1 on error.
+// Mismatches, out of 4 n comparisons, between the short fp64 division, square root and its
+// reciprocal and the rotation of fp64.hpp and their IEEE forms, over n seeded draws. -1 on
+// error.
 long long slime_probe_fp64_core(long long n, unsigned long long seed) {
     unsigned long long* bad = nullptr;
     long long r = -1;

@@ -3,7 +3,14 @@
 // cyclic row order done one rotation at a time. Test infrastructure: built with g++ by
 // tests/test_jacobi_wave.py.
 //
+// The rotations of both are the kernel's own (jacobi_wave::rotation). `rotation` compares
+// that form with the exact angle: t = sign(tau) / (|tau| + sqrt(1 + tau^2)), tau = d / 2 apq,
+// c = 1 / sqrt(1 + t^2), s = t c in 64-bit-significand long double, over blocks of every kind
+// (both signs of d and apq, d = 0, |d| far above and far below |apq|, |apq| just over 1e-6).
+//
 // Usage: jacobi_wave_check D seed kind [plant]   kind: dense | lowrank | diag | rank1
+//        jacobi_wave_check rotation n seed [plant]   plant "sign": the reference's sine negated
+//          for d < 0; "half": its angle taken with tau = d / apq
 //   plant "swap-order": the emulation visits each row's pairs one step late against the
 //   other rows (a planted mistake).
 // Prints "OK sweeps rotations err" or "FAIL ..." and exits 1.
@@ -24,14 +31,6 @@ using namespace slime::jacobi_wave;
 namespace {
 
 constexpr double kTol = 1e-6;
-
-void rotation(double app, double aqq, double apq, double& c, double& s) {
-    const double tau = (aqq - app) / (2.0 * apq);
-    const double u = 1.0 / (std::fabs(tau) + std::sqrt(1.0 + tau * tau));
-    const double t = tau < 0.0 ? -u : u;
-    c = 1.0 / std::sqrt(1.0 + t * t);
-    s = t * c;
-}
 
 // One rotation at a time, in cyclic row order.
 int serial(std::vector<double> A, int D, std::vector<double>& diag, long* nrot) {
@@ -184,10 +183,50 @@ int wave(const std::vector<double>& A0, int D, std::vector<double>& diag, bool p
     }
 }
 
+// The roundings of jacobi_wave::rotation in turn (stated there) bound c by 2.3 u and s by 8.3 u
+// relative, u = 2^-53, and so c^2 + s^2 - 1 by 2 (2.3 c^2 + 8.3 s^2) u, at most 10.6 u.
+int rotation_check(long n, int seed, const std::string& plant) {
+    std::mt19937_64 rng(seed);
+    std::uniform_real_distribution<double> u01(0.0, 1.0);
+    auto mag = [&](double lo, double hi) { return std::exp2(lo + (hi - lo) * u01(rng)); };
+    const long double u = 0x1p-53L;
+    long double ec = 0, es = 0, en = 0;
+    for (long i = 0; i < n; ++i) {
+        double app = mag(-24, 8), aqq = mag(-24, 8), apq = mag(-19, 8);
+        switch (i % 6) {
+            case 1: aqq = app; break;
+            case 2: apq = 1e-6 * (1.0 + 1e-3 * u01(rng)); break;
+            case 3: app = mag(40, 290), apq = mag(-19, 0); break;      // |d| >> |b|
+            case 4: aqq = app * (1.0 + 0x1p-50 * (double)(i % 13)); apq = mag(0, 290); break;  // |b| >> |d|
+            case 5: std::swap(app, aqq); aqq = mag(40, 290), apq = mag(-19, 290); break;
+            default: break;
+        }
+        if (i & 8) apq = -apq;
+        if (i & 16) std::swap(app, aqq);
+        double c, s;
+        rotation(app, aqq, apq, c, s);
+        const double d = aqq - app;  // rounded, as in every form
+        const long double tau = (long double)d / ((plant == "half" ? 1.0L : 2.0L) * apq);
+        long double t = 1.0L / (std::fabs(tau) + std::sqrt(1.0L + tau * tau));
+        if (tau < 0.0L) t = -t;
+        const long double rc = 1.0L / std::sqrt(1.0L + t * t);
+        long double rs = t * rc;
+        if (plant == "sign" && d < 0.0) rs = -rs;
+        ec = std::fmax(ec, std::fabs(c - rc) / rc / u);
+        es = std::fmax(es, std::fabs(s - rs) / std::fabs(rs) / u);
+        en = std::fmax(en, std::fabs((long double)c * c + (long double)s * s - 1.0L) / u);
+    }
+    const bool ok = ec <= 2.3L && es <= 8.3L && en <= 10.6L;
+    std::printf("%s rotation c %.2Lf u, s %.2Lf u, norm %.2Lf u\n", ok ? "OK" : "FAIL", ec, es, en);
+    return ok ? 0 : 1;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     if (argc < 4) return 2;
+    if (!std::strcmp(argv[1], "rotation"))
+        return rotation_check(std::atol(argv[2]), std::atoi(argv[3]), argc > 4 ? argv[4] : "");
     const int D = std::atoi(argv[1]);
     const std::string kind = argv[3];
     std::mt19937_64 rng(std::atoi(argv[2]));

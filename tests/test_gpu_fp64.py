@@ -1,8 +1,9 @@
 """The short fp64 division, square root and Jacobi rotation of
 slime_amd/csrc/fp64.hpp against the IEEE `/` and `sqrt` of the same device, bit for
 bit (slime_probe_fp64_core in libslime_probe.so). The fitness solve uses the short
-forms on its serial rotation chain; equal bits keep its rotations those of the
-IEEE formulas that the oracle (oracle/ca_oracle.cpp, oracle_jacobi_eigs) states.
+forms on its serial rotation chain; equal bits make its rotations those of
+jacobi_wave::rotation, which test_jacobi_wave.py holds to a few units of 2^-53 of the
+angle that the oracle (oracle/ca_oracle.cpp, oracle_jacobi_eigs) states.
 """
 import ctypes
 import os

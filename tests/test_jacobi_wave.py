@@ -29,3 +29,17 @@ def test_wave_front_is_the_cyclic_order(check, D, kind):
 def test_a_stale_element_is_reported(check):
     r = subprocess.run([check, "64", "1", "dense", "swap-order"], capture_output=True, text=True, timeout=60)
     assert r.returncode == 1 and "FAIL" in r.stdout
+
+
+def test_rotation_is_the_exact_one_to_a_few_roundings(check):
+    """Bounds derived from the form's roundings (jacobi_wave.hpp): c 2.3, s 8.3 units of 2^-53."""
+    for seed in ("1", "2"):
+        r = subprocess.run([check, "rotation", "600000", seed], capture_output=True, text=True, timeout=60)
+        print(r.stdout.strip())
+        assert r.returncode == 0, r.stdout
+
+
+@pytest.mark.parametrize("plant", ["sign", "half"])
+def test_a_wrong_rotation_is_reported(check, plant):
+    r = subprocess.run([check, "rotation", "1000", "1", plant], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 1 and "FAIL rotation" in r.stdout
