@@ -401,8 +401,8 @@ __global__ __launch_bounds__(kFinThreads) void fitness_finalize_kernel(FitnessAr
         // element of slot d1's pair.
         static_assert(S * S / 2 <= kFinUpdate, "one work item per thread");
         const int u = tid - 64;
-        const int d1 = u & (S - 1), o = u / S + 1, d2 = (d1 + o) & (S - 1);  // jacobi_wave::item
-        const bool act = o <= S / 2 && (o < S / 2 || d1 < S / 2), pairs = u < S;
+        SLIME_JACOBI_ITEM(u, S, d1, d2, act);
+        const bool pairs = u < S;
         for (int T = 0;; ++T) {
             const int sig = T & (D - 1);
             const double* M = A[cur];

@@ -31,6 +31,7 @@ using namespace slime::jacobi_wave;
 namespace {
 
 constexpr double kTol = 1e-6;
+constexpr int kUpdateThreads = 512;  // kFinUpdate of fitness.hip
 
 // One rotation at a time, in cyclic row order.
 int serial(std::vector<double> A, int D, std::vector<double>& diag, long* nrot) {
@@ -106,9 +107,10 @@ int wave(const std::vector<double>& A0, int D, std::vector<double>& diag, bool p
                 if (!written.insert(upper(i, j, D)).second) std::printf("FAIL element written twice\n"), std::exit(1);
                 A[1 - cur][upper(i, j, D)] = v;
             };
-            for (int n = 0; n < S * S / 2; ++n) {
-                int d1, d2, i1, j1, i2, j2;
-                if (!item(n, S, &d1, &d2)) continue;
+            for (int n = 0; n < kUpdateThreads; ++n) {  // one item per thread of the kernel
+                int i1, j1, i2, j2;
+                SLIME_JACOBI_ITEM(n, S, d1, d2, valid);
+                if (!valid) continue;
                 slot(sig, d1, D, &i1, &j1);
                 slot(sig, d2, D, &i2, &j2);
                 const std::vector<double>& M = A[cur];
