@@ -308,8 +308,8 @@ int run_project(slime_ca* h, const void* x, const float* x_scale, void* P, void*
 }
 
 // S2-S6 plus the mass partials and S7 finalize: y_raw gets the unscaled output,
-// out_scale the per-(b, head) conservation factor. With y_out (a call's last step) the
-// factor is also applied, y_out = out_scale * y_raw in the storage type.
+// out_scale the per-(b, head) conservation factor. With y_out (a call's last step, whose
+// y_raw is fp32) the factor is also applied, y_out = out_scale * y_raw in the storage type.
 // loss_T, loss_part: the backward's tape step on the MFMA stencil (bf16, D = 64), which
 // also sums Y^2, Y T and T^2 per (b, head, tile) into loss_part (StencilArgs).
 int run_stencil(slime_ca* h, const void* x, const float* x_scale, const void* P, const void* I,
@@ -348,7 +348,7 @@ int run_stencil(slime_ca* h, const void* x, const float* x_scale, const void* P,
     if (conserve_pass) HIP_TRY(launch_cell_conserve(x, x_scale, y_raw, y_f32, h->part_out, c.B, c.G, s));
     if (y_out)
         HIP_TRY(launch_mass_rescale(c.dtype, h->part_in, h->part_out, h->tiles, h->mass_in, h->mass_out,
-                                    out_scale, y_raw, y_f32, y_out, c.B, c.G, h->C, c.D, s));
+                                    out_scale, static_cast<const float*>(y_raw), y_out, c.B, c.G, h->C, c.D, s));
     else
         HIP_TRY(launch_mass_finalize(h->part_in, h->part_out, c.B * c.H, h->tiles, h->mass_in,
                                      h->mass_out, out_scale, out_scale64, s));
@@ -887,7 +887,9 @@ int slime_ca_backward(slime_ca* h, const void* x_in, const void* target, float* 
     const int lchunks = loss_fused ? h->tiles : backward_loss_chunks(c.G);
     const int nW = 1024;  // cell-pass workgroups per pod
     const long long rows_pod = (long long)(c.B / c.pods) * c.G * c.G;
-    const DwPlan dw = backward_dw_plan(c.dtype, (int)C, c.pods, rows_pod);
+    int n_cu = 0;
+    HIP_TRY(device_cu_count(&n_cu));
+    const DwPlan dw = backward_dw_plan(c.dtype, (int)C, c.pods, rows_pod, n_cu);
     const bool want_w = grads && (grads->WP || grads->WI || grads->WV);
     // work buffers, allocated on first use
     if (!h->Wcat) {

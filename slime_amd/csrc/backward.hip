@@ -1370,13 +1370,13 @@ int backward_loss_chunks(int G) { return (G * G + kLossCells - 1) / kLossCells; 
 int backward_part_floats() { return kPartF; }
 
 // Tiles of 256 or 128 (bf16, bw_dw_mfma2_kernel and bw_dw_mfma_kernel) or 64 (bw_dw64_kernel),
-// and the rows a chunk sums, by the least time of: rounds of workgroups over 256 CUs at the
+// and the rows a chunk sums, by the least time of: rounds of workgroups over the CUs at the
 // rate one tile reaches (3.9, 2.7 and 0.5 TFLOP/s per CU), plus the chunks' partials written
 // and read once at 4.8 TB/s. One chunk keeps at most 16,384 rows (4096 in 64-wide tiles), so
-// that its fp32 sums stay short, and at least 128. A large product keeps its few long
-// chunks (1,048,576 rows, C = 512: 64 chunks of 768 tiles); one grid of 16,384 rows had 12
-// workgroups.
-DwPlan backward_dw_plan(int dtype, int C, int pods, long long rows_per_pod) {
+// that its fp32 sums stay short, and is halved no further once it has at most 128. A large
+// product keeps its few long chunks (1,048,576 rows, C = 512: 64 chunks of 768 tiles); one
+// grid of 16,384 rows had 12 workgroups.
+DwPlan backward_dw_plan(int dtype, int C, int pods, long long rows_per_pod, int n_cu) {
     DwPlan best{0, 0, 0};
     double best_t = 0.0;
     for (int tile : {256, 128, 64}) {
@@ -1387,7 +1387,7 @@ DwPlan backward_dw_plan(int dtype, int C, int pods, long long rows_per_pod) {
         for (long long n = (rows_per_pod + most - 1) / most;; n *= 2) {
             const long long rows = ((rows_per_pod + n - 1) / n + 31) / 32 * 32;
             const long long chunks = (rows_per_pod + rows - 1) / rows;
-            const double rounds = std::ceil(tiles * chunks / 256.0);
+            const double rounds = std::ceil(tiles * chunks / n_cu);
             const double t = rounds * rows * tile * tile * 2.0 / rate + (double)chunks * pods * C * 3 * C * 8.0 / 4.8e12;
             if (!best.tile || t < best_t) best = DwPlan{tile, rows, (int)chunks}, best_t = t;
             if (rows <= 128) break;

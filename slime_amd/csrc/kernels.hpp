@@ -127,15 +127,11 @@ hipError_t launch_cell_conserve(const void* x, const float* scale, void* y, int 
                                 hipStream_t s);
 // y[i] = x[i] for n elements of 2 or 4 bytes, either side at any element's address.
 hipError_t launch_copy(size_t elem, const void* x, void* y, long long n, hipStream_t s);
-// y[i] = cvt((scale[0][b][h] + scale[1][b][h]) * x[i]) over the whole state; x is
-// fp32 when x_f32 is set, else in the storage type.
-hipError_t launch_rescale(int dtype, const void* x, int x_f32, const float* scale, void* y, int B,
-                          int G, int C, int D, hipStream_t s);
-
-// launch_mass_finalize and launch_rescale together, in one launch for small grids.
+// launch_mass_finalize, then y[i] = cvt((scale[0][b][h] + scale[1][b][h]) * x[i]) over the whole
+// state (x: the stencil's fp32 output), in one launch for small grids.
 hipError_t launch_mass_rescale(int dtype, const double* part_in, const double* part_out, int tiles, double* mass_in,
-                               double* mass_out, float* scale, const void* x, int x_f32, void* y, int B, int G, int C,
-                               int D, hipStream_t s);
+                               double* mass_out, float* scale, const float* x, void* y, int B, int G, int C, int D,
+                               hipStream_t s);
 
 // ---- E1-E5 fitness --------------------------------------------------------------------
 struct FitnessArgs {
@@ -241,7 +237,7 @@ struct DwPlan {
     long long rows_per_chunk;
     int chunks_per_pod;
 };
-DwPlan backward_dw_plan(int dtype, int C, int pods, long long rows_per_pod);
+DwPlan backward_dw_plan(int dtype, int C, int pods, long long rows_per_pod, int n_cu);
 hipError_t launch_backward_stencil(int dtype, const BackwardArgs& a, hipStream_t s);
 hipError_t launch_backward_dw(int dtype, const BackwardArgs& a, const DwArgs& d, hipStream_t s);
 

@@ -94,17 +94,12 @@ __global__ __launch_bounds__(256) void mass_finalize_kernel(const double* part_i
         write_factor(m, bh, gridDim.x, s[0][0] + s[0][1] + s[0][2] + s[0][3], s[1][0] + s[1][1] + s[1][2] + s[1][3]);
 }
 
-// Four consecutive elements times the factor; they never straddle two heads (D >= 8).
-template <typename TI, typename T>
-__device__ __forceinline__ void rescale_quad(const TI* x, T* y, long long q, float s, float s_lo) {
-    float v[4];
-    if constexpr (sizeof(TI) == 2) {
-        const uint2 w = reinterpret_cast<const uint2*>(x)[q];
-        v[0] = bf16lo(w.x); v[1] = bf16hi(w.x); v[2] = bf16lo(w.y); v[3] = bf16hi(w.y);
-    } else {
-        const float4 f = reinterpret_cast<const float4*>(x)[q];
-        v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
-    }
+// Four consecutive fp32 elements times the factor, in the state's type; they never straddle two
+// heads (D >= 8).
+template <typename T>
+__device__ __forceinline__ void rescale_quad(const float* x, T* y, long long q, float s, float s_lo) {
+    const float4 f = reinterpret_cast<const float4*>(x)[q];
+    float v[4] = {f.x, f.y, f.z, f.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = __builtin_fmaf(v[i], s, v[i] * s_lo);
     if constexpr (sizeof(T) == 2) {
@@ -127,8 +122,8 @@ __global__ __launch_bounds__(256) void copy_kernel(const T* x, T* y, long long n
     }
 }
 
-template <typename TI, typename T>
-__global__ __launch_bounds__(256) void rescale_kernel(const TI* x, const float* scale, T* y,
+template <typename T>
+__global__ __launch_bounds__(256) void rescale_kernel(const float* x, const float* scale, T* y,
                                                       long long nquads, int C, int D,
                                                       long long cells_per_batch, int bh_total) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -146,9 +141,9 @@ __global__ __launch_bounds__(256) void rescale_kernel(const TI* x, const float* 
 // forms the entry's eight factors from the partials itself, two heads per wave, and the
 // entry's first workgroup writes them. One wave's tree over the tiles, so the factors have
 // the bits of mass_finalize_kernel.
-template <typename TI, typename T>
+template <typename T>
 __global__ __launch_bounds__(256) void mass_rescale_kernel(const double* part_in, const double* part_out, int tiles,
-                                                           MassOut m, const TI* x, T* y, int C, int D,
+                                                           MassOut m, const float* x, T* y, int C, int D,
                                                            int wgs_per_batch, int BH) {
     __shared__ Factor f[kHeads];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -286,55 +281,36 @@ hipError_t launch_copy(size_t elem, const void* x, void* y, long long n, hipStre
     return hipGetLastError();
 }
 
-hipError_t launch_rescale(int dtype, const void* x, int x_f32, const float* scale, void* y, int B,
-                          int G, int C, int D, hipStream_t s) {
-    const long long cells = (long long)G * G;
-    const long long nquads = (long long)B * cells * C / 4;
-    const dim3 grid((unsigned)((nquads + 255) / 256));
-    const int bh = B * (C / D);
-    if (dtype == 1 && x_f32)
-        hipLaunchKernelGGL((rescale_kernel<float, bf16_t>), grid, dim3(256), 0, s,
-                           static_cast<const float*>(x), scale, static_cast<bf16_t*>(y), nquads, C,
-                           D, cells, bh);
-    else if (dtype == 1)
-        hipLaunchKernelGGL((rescale_kernel<bf16_t, bf16_t>), grid, dim3(256), 0, s,
-                           static_cast<const bf16_t*>(x), scale, static_cast<bf16_t*>(y), nquads, C,
-                           D, cells, bh);
-    else
-        hipLaunchKernelGGL((rescale_kernel<float, float>), grid, dim3(256), 0, s,
-                           static_cast<const float*>(x), scale, static_cast<float*>(y), nquads, C,
-                           D, cells, bh);
-    return hipGetLastError();
-}
-
-namespace {
-template <typename TI, typename T>
-hipError_t launch_fused_t(const double* part_in, const double* part_out, int tiles, const MassOut& m, const void* x,
-                          void* y, int B, int C, int D, int wgs, hipStream_t s) {
-    hipLaunchKernelGGL((mass_rescale_kernel<TI, T>), dim3((unsigned)(B * wgs)), dim3(256), 0, s, part_in, part_out,
-                       tiles, m, static_cast<const TI*>(x), static_cast<T*>(y), C, D, wgs, B * kHeads);
-    return hipGetLastError();
-}
-}  // namespace
-
 // One launch while the partials that every workgroup reads again stay small beside the
 // data: at most 64 tiles, and 16 MiB of partial reads in all. Small grids are bound by
 // their launches (a step of 32^2 x 64 fp32: 20.9 -> 17.1 us); a batch of 64 grids of 32^2 x
 // 512 would read 134 MB of partials beside 201 MB of data.
-hipError_t launch_mass_rescale(int dtype, const double* part_in, const double* part_out, int tiles, double* mass_in,
-                               double* mass_out, float* scale, const void* x, int x_f32, void* y, int B, int G, int C,
-                               int D, hipStream_t s) {
-    const long long wgs = (long long)G * G * C / 1024;
-    const MassOut m{mass_in, mass_out, scale, nullptr};
+namespace {
+template <typename T>
+hipError_t launch_mass_rescale_t(const double* part_in, const double* part_out, int tiles, const MassOut& m,
+                                 const float* x, T* y, int B, int G, int C, int D, hipStream_t s) {
+    const long long cells = (long long)G * G, wgs = cells * C / 1024;
     if (tiles <= 64 && B * wgs * tiles * 2 * kHeads * 8 <= (16 << 20)) {
-        if (dtype == 1 && x_f32)
-            return launch_fused_t<float, bf16_t>(part_in, part_out, tiles, m, x, y, B, C, D, (int)wgs, s);
-        if (dtype == 1) return launch_fused_t<bf16_t, bf16_t>(part_in, part_out, tiles, m, x, y, B, C, D, (int)wgs, s);
-        return launch_fused_t<float, float>(part_in, part_out, tiles, m, x, y, B, C, D, (int)wgs, s);
+        hipLaunchKernelGGL((mass_rescale_kernel<T>), dim3((unsigned)(B * wgs)), dim3(256), 0, s, part_in, part_out,
+                           tiles, m, x, y, C, D, (int)wgs, B * kHeads);
+        return hipGetLastError();
     }
     const hipError_t e =
-        launch_mass_finalize(part_in, part_out, B * kHeads, tiles, mass_in, mass_out, scale, nullptr, s);
-    return e != hipSuccess ? e : launch_rescale(dtype, x, x_f32, scale, y, B, G, C, D, s);
+        launch_mass_finalize(part_in, part_out, B * kHeads, tiles, m.mass_in, m.mass_out, m.scale, m.scale64, s);
+    if (e != hipSuccess) return e;
+    const long long nquads = B * cells * C / 4;
+    hipLaunchKernelGGL((rescale_kernel<T>), dim3((unsigned)((nquads + 255) / 256)), dim3(256), 0, s, x, m.scale, y,
+                       nquads, C, D, cells, B * (C / D));
+    return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_mass_rescale(int dtype, const double* part_in, const double* part_out, int tiles, double* mass_in,
+                               double* mass_out, float* scale, const float* x, void* y, int B, int G, int C, int D,
+                               hipStream_t s) {
+    const MassOut m{mass_in, mass_out, scale, nullptr};
+    return dtype == 1 ? launch_mass_rescale_t(part_in, part_out, tiles, m, x, static_cast<bf16_t*>(y), B, G, C, D, s)
+                      : launch_mass_rescale_t(part_in, part_out, tiles, m, x, static_cast<float*>(y), B, G, C, D, s);
 }
 
 }  // namespace slime

@@ -41,7 +41,8 @@ def test_parallel_heads_match_serial_heads(dtype, D, G, copies, per_cell, cons):
     assert torch.isfinite(outs[0].float()).all()
     assert torch.equal(outs[1], outs[0].expand_as(outs[1]))
     for one, many in zip(masses[0], masses[1]):
-        # fp64 sums of the same lane sums, trees of another shape: 2^-48 of the sums' size
+        # the same lanes' sums added in fp64 in another order: about ten roundings of 2^-53 of
+        # the sum of magnitudes, which is below 2^9 of the sum itself
         np.testing.assert_allclose(many, np.broadcast_to(one, many.shape), rtol=2.0 ** -40)
 
 
