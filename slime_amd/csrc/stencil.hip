@@ -1320,12 +1320,15 @@ __global__ __launch_bounds__(mf::kThreads, 2) void stencil_mfma_kernel(StencilAr
 }
 
 // One workgroup per tile. Heads in parallel (D < 64) while the tiles leave the card room for
-// it: up to kParTiles tiles per CU. Measured, full / parallel in us:
-//   D = 8   fp32 32 tiles 11.7 / 5.5, 1024 tiles 16.2 / 15.7, 1600 tiles 21.3 / 23.4
-//   D = 16  bf16 162 tiles 13.5 / 7.2, 576 tiles 16.1 / 14.7, 1600 tiles 26.5 / 30.1
-//           fp32 162 tiles 14.4 / 8.2, 576 tiles 18.3 / 23.5
-//   D = 32  fp32 162 tiles 16.2 / 11.8, 288 tiles 19.1 / 23.0
+// it: up to kParTiles tiles per CU. Measured, full / parallel in us (kernel trace, flow_lenia):
+//   D = 8   bf16 32 tiles 13.6 / 5.9, 1024 tiles 19.8 / 16.8, 1600 tiles 24.7 / 21.8
+//           fp32 32 tiles 12.5 / 6.1, 1024 tiles 18.6 / 17.9, 1600 tiles 23.6 / 25.2
+//   D = 16  bf16 162 tiles 14.8 / 8.3, 576 tiles 22.1 / 19.2, 1024 tiles 24.5 / 22.3, 1600 tiles 29.9 / 33.2
+//           fp32 162 tiles 15.5 / 10.3, 288 tiles 17.6 / 16.4, 576 tiles 21.1 / 25.2
+//   D = 32  bf16 162 tiles 17.1 / 13.7, 242 tiles 18.2 / 14.4, 288 tiles 22.9 / 24.4
+//           fp32 162 tiles 17.4 / 13.6, 242 tiles 18.0 / 16.0, 288 tiles 20.5 / 24.3
 //   D = 64  fp32 32 tiles 18.5 / 18.2, 162 tiles 19.4 / 20.6: never
+// (Past the line the parallel form still wins by a tenth for D = 8 bf16 up to 1600 tiles.)
 template <typename T, int D, typename TY, bool kCons>
 hipError_t launch_tdy(const StencilArgs& a, hipStream_t s) {
     using L = Layout<T, D>;
