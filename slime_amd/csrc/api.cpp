@@ -32,7 +32,7 @@ struct slime_ca {
 
     float* Wtm = nullptr;      // [pods][3C][C] fp32 masters, transposed (n-major)
     void* Wt = nullptr;        // [B][3C][C] per-batch scaled, transposed
-    void* W1 = nullptr;        // [pods][3C][C] as Wtm, unscaled, in the handle's dtype
+    void* W1 = nullptr;        // [pods][3C][C] as Wtm in bf16; an fp32 handle reads Wtm itself
     float* K = nullptr;        // [pods][H][9]
     float* mu = nullptr;       // [pods][H] or [pods][G][G][H]
     float* sigma = nullptr;
@@ -243,9 +243,9 @@ int give_back(slime_ca* h, const void* from, void* y, size_t elem, hipStream_t s
 }
 
 // S1 for one step, then the projection GEMM(s). Weights that the deferred mass scale of x
-// does not touch come from W1, one copy per pod: all of them when x_scale is NULL (a state
-// as its caller holds it), and the second and third plane of the chained forms. Scaled
-// ones are written per batch entry first.
+// does not touch come from W1 (fp32: Wtm), one copy per pod: all of them when x_scale is
+// NULL (a state as its caller holds it), and the second and third plane of the chained
+// forms. Scaled ones are written per batch entry first.
 // With `pre` (parallel projections only), I before its GELU is also written there.
 int run_project(slime_ca* h, const void* x, const float* x_scale, void* P, void* I, void* V,
                 hipStream_t s, void* pre = nullptr) {
@@ -269,7 +269,8 @@ int run_project(slime_ca* h, const void* x, const float* x_scale, void* P, void*
     g.ncol = C;
     g.bt_batch_stride = 3LL * C * C;
     auto weights = [&](bool scaled, int plane) {
-        g.Bt = static_cast<const char*>(scaled ? h->Wt : h->W1) + (size_t)plane * C * C * h->elem;
+        const void* once = h->W1 ? h->W1 : h->Wtm;
+        g.Bt = static_cast<const char*>(scaled ? h->Wt : once) + (size_t)plane * C * C * h->elem;
         g.rows_per_batch = scaled ? cells : per_pod * cells;
     };
     if (!c.pvi_chain) {
@@ -431,7 +432,7 @@ int slime_ca_create(const slime_ca_config* config, slime_ca** out) {
     rc = 0;
     rc = rc ? rc : dalloc_t(&h->Wtm, (size_t)c.pods * 3 * C * C * 4);
     rc = rc ? rc : dalloc(&h->Wt, (size_t)c.B * 3 * C * C * h->elem);
-    rc = rc ? rc : dalloc(&h->W1, (size_t)c.pods * 3 * C * C * h->elem);
+    if (c.dtype == SLIME_BF16) rc = rc ? rc : dalloc(&h->W1, (size_t)c.pods * 3 * C * C * h->elem);
     rc = rc ? rc : dalloc_t(&h->K, (size_t)c.pods * c.H * 9 * 4);
     rc = rc ? rc : dalloc_t(&h->mu, n_param_growth(c) * 4);
     rc = rc ? rc : dalloc_t(&h->sigma, n_param_growth(c) * 4);
@@ -536,9 +537,9 @@ int slime_ca_set_params(slime_ca* h, const slime_ca_params* p) {
                               hipMemcpyHostToDevice));
         }
     }
-    // The unscaled copy that the GEMMs read: laid out once here, on the stream of the uploads
+    // bf16: the unscaled copy that the GEMMs read, laid out once here, on the stream of the uploads
     // (waited for below, since a step may come on a stream that does not wait for that one).
-    {
+    if (h->W1) {
         WeightPrepArgs w{};
         w.Wtm = h->Wtm;
         w.Wt = h->W1;
@@ -571,7 +572,7 @@ int slime_ca_set_params(slime_ca* h, const slime_ca_params* p) {
     HIP_TRY(hipMemcpy(h->mu, p->mu, ng * 4, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(h->sigma, p->sigma, ng * 4, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(h->M, p->M, (size_t)c.pods * c.H * c.H * 4, hipMemcpyHostToDevice));
-    HIP_TRY(hipStreamSynchronize(nullptr));
+    if (h->W1) HIP_TRY(hipStreamSynchronize(nullptr));
     h->params_set = true;
     return SLIME_OK;
 }

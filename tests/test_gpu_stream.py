@@ -18,9 +18,12 @@ def test_stream_handle_is_the_current_streams():
     assert (_stream().value or 0) == torch.cuda.current_stream().cuda_stream
 
 
-def test_new_parameters_reach_a_step_on_a_side_stream():
-    """set_params lays the weights out on the device; a projection that follows at once on a
-    stream of its own reads the new ones."""
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+def test_new_parameters_reach_a_step_on_a_side_stream(dtype):
+    """set_params uploads the weights (and, in bf16, lays them out on the device); a projection
+    that follows at once on a stream of its own reads the new ones. It holds the result, not
+    the wait that ends set_params: the blocking copies after the layout kernel, on the same
+    stream, would be likely to cover for it."""
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     import numpy as np
@@ -29,8 +32,8 @@ def test_new_parameters_reach_a_step_on_a_side_stream():
     C = 8 * D
     rng = np.random.default_rng(5)
     z = np.zeros
-    ca = Pseudopod(1, G, 8, D, "fp32", 0.1)
-    x = torch.from_numpy(rng.random((1, G, G, C), dtype=np.float32)).cuda()
+    ca = Pseudopod(1, G, 8, D, dtype, 0.1)
+    x = torch.from_numpy(rng.random((1, G, G, C), dtype=np.float32)).to("cuda", ca.torch_dtype)
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     for s in (1.0, 2.0, 0.5, 4.0):  # W = s I: V = s X exactly, for powers of two
