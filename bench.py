@@ -130,7 +130,7 @@ def _trace_work(workload: str) -> dict:
             "gemm_mfma_kernel<unsigned short>": ("[P\\|I\\|V] projection GEMM", "F", 2 * C * 3 * C),
             "stencil_mfma_kernel<unsigned short>": ("S2-S6 + mass partials, bf16 out", "B", 5 * C * 2),
             "stencil_mfma_kernel<float>": ("last step of a call, fp32 out", "B", 4 * C * 2 + C * 4),
-            "rescale_kernel<float, unsigned short>": ("final rescale, fp32 -> bf16", "B", C * 4 + C * 2),
+            "rescale_kernel<unsigned short>": ("final rescale, fp32 -> bf16", "B", C * 4 + C * 2),
             "weight_prep_kernel<unsigned short>": ("per-batch scaled weights", None, None),
             "mass_finalize_kernel": ("S7 factors", None, None),
         }
@@ -156,10 +156,10 @@ def _trace_work(workload: str) -> dict:
             "fitness_finalize_kernel<64>": ("Jacobi eigenvalues, effective rank, fitness", None, None),
             "gemm_mfma_kernel<unsigned short>": ("[P\\|I\\|V] projection GEMM", "F", 2 * C * 3 * C),
             "stencil_mfma_kernel<float>": ("single-step calls: fp32 out", "B", 4 * C * 2 + C * 4),
-            "fitness_partial_kernel<unsigned short, 64>": (
+            "fitness_partial_kernel<unsigned short, 64, 8>": (
                 "8-state history read once, fp64 Gram of the last", "B", 8 * C * 2),
             "stencil_mfma_kernel<unsigned short>": ("rollout: bf16 states", "B", 5 * C * 2),
-            "rescale_kernel<float, unsigned short>": ("single-step calls only", "B", C * 4 + C * 2),
+            "rescale_kernel<unsigned short>": ("single-step calls only", "B", C * 4 + C * 2),
             "weight_prep_kernel<unsigned short>": ("per-pod scaled weights", None, None),
             "mass_finalize_kernel": ("S7 factors", None, None),
             "fill_f64_kernel": ("the rollout's unit factors of state 0", None, None),
